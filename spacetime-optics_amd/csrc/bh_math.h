@@ -23,12 +23,18 @@
      m^{-1/3} from a cubic least-squares seed (5e-4), cbrt(m) = m w^2, then one Newton polish.
    - sincos: Cody-Waite reduction by pi/2 with a three-part constant (33+33+53 bits);
      sin r = r + r z S(z) (S of degree 5), cos r = 1 + z C(z) (C of degree 6) on |r| <= pi/4.
-   - atan2/acos: reciprocal and pi/6 (Hart) reductions to |t| <= tan(pi/12),
+   - atan2/acos: the ratio of the smaller to the larger, a pi/6 (Hart) reduction to |t| <= tan(pi/12),
      atan t = t + t z A(z) with A of degree 8; acos(x) = atan2(sqrt((1-x)(1+x)), x),
      asin(x) = atan2(x, sqrt((1-x)(1+x))).
    - x^-0.2 (the step controller): exp(-0.2 log x) refined by one Newton step on x y^5 = 1 with an
      FMA double-double residual; correctly rounded on [1e-300, 1e300].
-   Subnormal results of exp are flushed to zero (deterministically on both sides). */
+   Subnormal results of exp are flushed to zero (deterministically on both sides).
+
+   exp, expm1, log, cbrt and sincos have a device form beside the host's: the same rounded operations
+   in the same order, with the argument classes (overflow, zero, quadrants) as selects instead of
+   early returns and the exponents through v_frexp / v_ldexp. Every early return was an exec-mask
+   save, a branch and a restore on the device; a flow sample calls these fourteen times. A quotient
+   whose operands stay far from the ends of the exponent range is quot_ (below). */
 #pragma once
 #include <stdint.h>
 
@@ -81,6 +87,46 @@ BHM_HD double horner_(double p, double x, double c) {
 #endif
 }
 
+#if defined(__HIPCC__)
+// a / b, correctly rounded, for b > 0 and |a|, b, |a / b| well inside the exponent range (2^+-900):
+// the reciprocal refined by two Newton steps, the quotient by its exact residual. It is what the
+// division operator computes for such operands, without its range scaling and fix-up (8 operations
+// for 11), and a reciprocal can serve several quotients (3 operations each).
+struct Recip {
+    double b, y;
+};
+__device__ __forceinline__ Recip recip_(double b) {
+    double y = __builtin_amdgcn_rcp(b);
+    y = __builtin_fma(__builtin_fma(-b, y, 1.0), y, y);
+    y = __builtin_fma(__builtin_fma(-b, y, 1.0), y, y);
+    return Recip{b, y};
+}
+__device__ __forceinline__ double quot_(double a, const Recip& r) {
+    const double q = a * r.y;
+    return __builtin_fma(__builtin_fma(-r.b, q, a), r.y, q);
+}
+__device__ __forceinline__ double quot_(double a, double b) { return quot_(a, recip_(b)); }
+
+// sqrt(x), correctly rounded, for x > 0 well inside the exponent range: the reciprocal square root
+// refined by Goldschmidt steps and the exact residual (the operator's sequence without its scaling
+// and its classes: 10 operations for 17)
+__device__ __forceinline__ double sqrt_pos_(double x) {
+    const double y = __builtin_amdgcn_rsq(x);
+    double h = 0.5 * y, g = x * y;
+    const double r = __builtin_fma(-h, g, 0.5);
+    h = __builtin_fma(h, r, h);
+    g = __builtin_fma(g, r, g);
+    g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+    return __builtin_fma(__builtin_fma(-g, g, x), h, g);
+}
+// the same for x >= 0
+__device__ __forceinline__ double sqrt_nn_(double x) { return x == 0.0 ? x : sqrt_pos_(x); }
+// a / b with the IEEE results for a zero, infinite or NaN operand (one more operation)
+__device__ __forceinline__ double quot_ieee_(double a, double b) {
+    return __builtin_amdgcn_div_fixup(quot_(a, b), b, a);
+}
+#endif
+
 // (e^r - 1 - r) / r^2 for |r| <= ln2/2, degree 10 (fit error 2.6e-18)
 BHM_HD double expm1_core_q(double r) {
     double p = 0x1.1f8b3e103c1fep-29;
@@ -98,6 +144,12 @@ BHM_HD double expm1_core_q(double r) {
 }
 
 BHM_HD double exp(double x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    const double kd = floor_(fma_(x, INV_LN2, 0.5));
+    const double r = fma_(-kd, LN2_LO, fma_(-kd, LN2_HI, x));
+    const double e = __builtin_ldexp(1.0 + fma_(r * r, expm1_core_q(r), r), (int)kd);
+    return x > 709.782712893384 ? __builtin_inf() : (x < -708.3964185322641 ? 0.0 : e);   // NaN stays NaN
+#else
     if (isnan_(x)) return x;
     if (x > 709.782712893384) return __builtin_inf();
     if (x < -708.3964185322641) return 0.0;   // result would be subnormal: flushed
@@ -108,9 +160,20 @@ BHM_HD double exp(double x) {
     if (k > 1023) return e * 2.0 * pow2i(k - 1);
     if (k < -1021) return (e * pow2i(k + 54)) * 0x1p-54;
     return e * pow2i(k);
+#endif
 }
 
 BHM_HD double expm1(double x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    // k = 0 is the unreduced range: 2^0 em + (2^0 - 1) = em
+    const double kd = fabs_(x) <= 0.34657359027997264 ? 0.0 : floor_(fma_(x, INV_LN2, 0.5));
+    const int k = (int)kd;
+    const double r = fma_(-kd, LN2_LO, fma_(-kd, LN2_HI, x));
+    const double em = fma_(r * r, expm1_core_q(r), r);
+    const double t = __builtin_ldexp(1.0, k);
+    const double v = k > 56 ? __builtin_ldexp(em + 1.0, k) : fma_(t, em, t - 1.0);
+    return x > 709.782712893384 ? __builtin_inf() : (x < -38.0 ? -1.0 : v);
+#else
     if (isnan_(x)) return x;
     if (x > 709.782712893384) return __builtin_inf();
     if (x < -38.0) return -1.0;   // e^x < 2^-54
@@ -126,9 +189,19 @@ BHM_HD double expm1(double x) {
     }
     double t = pow2i(k);
     return fma_(t, em, t - 1.0);
+#endif
 }
 
 BHM_HD double log(double x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    double m = __builtin_amdgcn_frexp_mant(x);   // [1/2, 1); the host's m is in [1, 2)
+    const bool hi = m + m > SQRT2;
+    const double ed = (double)(__builtin_amdgcn_frexp_exp(x) - (hi ? 0 : 1));
+    m = hi ? m : m + m;
+    const double f = m - 1.0;
+    const double s = quot_(f, 2.0 + f);
+    const double z = s * s;
+#else
     if (isnan_(x)) return x;
     if (x < 0.0) return __builtin_nan("");
     if (x == 0.0) return -__builtin_inf();
@@ -147,6 +220,7 @@ BHM_HD double log(double x) {
     double f = m - 1.0;
     double s = f / (2.0 + f);
     double z = s * s;
+#endif
     // R = 2 atanh(s) / s - 2 = z P(z), P of degree 6 (fit error of R 3.6e-18)
     double P = 0x1.2f056aef6994ap-3;
     P = horner_(P, z, 0x1.39a1b9ea2f5d1p-3);
@@ -157,8 +231,14 @@ BHM_HD double log(double x) {
     P = horner_(P, z, 0x1.5555555555592p-1);
     double R = z * P;
     double lm = fma_(-s, f - R, f);
+#if defined(__HIP_DEVICE_COMPILE__)
+    const double v = fma_(ed, LN2_HI, fma_(ed, LN2_LO, lm));
+    if (x > 0.0 && x < __builtin_inf()) return v;
+    return x == 0.0 ? -__builtin_inf() : (x > 0.0 ? x : __builtin_nan(""));
+#else
     double ed = (double)e;
     return fma_(ed, LN2_HI, fma_(ed, LN2_LO, lm));
+#endif
 }
 
 // x^-0.2 for x > 0 (the step-size controller's factor, with -0.2 the double nearest -1/5), correctly
@@ -185,6 +265,11 @@ BHM_HD double pow_m02(double x) {
 
 BHM_HD double cbrt(double x) {
     if (x == 0.0 || isnan_(x) || isinf_(x)) return x;
+#if defined(__HIP_DEVICE_COMPILE__)
+    const int e = __builtin_amdgcn_frexp_exp(x) - 1;
+    const double m = 2.0 * fabs_(__builtin_amdgcn_frexp_mant(x));   // [1, 2)
+    const int q = (int)(((unsigned)(e + 3072) * 43691u) >> 17) - 1024, rr = e - 3 * q;   // floor(e / 3); 0, 1, 2
+#else
     double sgn = x < 0.0 ? -1.0 : 1.0;
     double ax = fabs_(x);
     int adj = 0;
@@ -197,6 +282,7 @@ BHM_HD double cbrt(double x) {
     double m = dfrom((b & 0x000fffffffffffffull) | 0x3ff0000000000000ull);   // [1, 2)
     int q = e >= 0 ? e / 3 : -((-e + 2) / 3);
     int rr = e - 3 * q;   // 0, 1, 2
+#endif
     double w = -0x1.8b825efdf6842p-5;
     w = w * m + 0x1.3cab785e5a648p-2;
     w = w * m + -0x1.977b7db5d7b17p-1;
@@ -204,6 +290,12 @@ BHM_HD double cbrt(double x) {
     for (int i = 0; i < 2; ++i) w = w * fma_(-m, w * w * w, 4.0) * (1.0 / 3.0);   // 5e-4 -> 6e-13
     double y = m * (w * w);
     double t = m;
+#if defined(__HIP_DEVICE_COMPILE__)
+    y = y * (rr == 0 ? 1.0 : (rr == 1 ? CBRT2 : CBRT4));
+    t = __builtin_ldexp(m, rr);
+    y = fma_(quot_(t, y * y) - y, 1.0 / 3.0, y);
+    return __builtin_copysign(__builtin_ldexp(y, q), x);
+#else
     if (rr == 1) {
         y = y * CBRT2;
         t = m * 2.0;
@@ -214,15 +306,18 @@ BHM_HD double cbrt(double x) {
     y = fma_(t / (y * y) - y, 1.0 / 3.0, y);   // one Newton polish of y^3 = t
     int k = q + adj;
     return sgn * (y * pow2i(k));
+#endif
 }
 
 // sin and cos of x (finite |x| < ~1e6 keeps full accuracy; larger |x| stays deterministic)
 BHM_HD void sincos(double x, double* sp, double* cp) {
+#if !defined(__HIP_DEVICE_COMPILE__)   // the reduction below gives NaN for both by itself
     if (isnan_(x) || isinf_(x)) {
         *sp = __builtin_nan("");
         *cp = __builtin_nan("");
         return;
     }
+#endif
     double kd = floor_(fma_(x, TWO_OVER_PI, 0.5));
     double r = fma_(-kd, PIO2_3, fma_(-kd, PIO2_2, fma_(-kd, PIO2_1, x)));
     int q = (int)(kd - 4.0 * floor_(kd * 0.25));
@@ -244,6 +339,13 @@ BHM_HD void sincos(double x, double* sp, double* cp) {
     pc = horner_(pc, z, 0x1.555555555553cp-5);
     pc = fma_(pc, z, -0.5);
     double c = fma_(z, pc, 1.0);
+#if defined(__HIP_DEVICE_COMPILE__)
+    // odd quadrants swap the two; sin is negative in 2 and 3, cos in 1 and 2
+    const double a = (q & 1) ? c : s, b = (q & 1) ? s : c;
+    *sp = (q & 2) ? -a : a;
+    *cp = ((q + 1) & 2) ? -b : b;
+    return;
+#endif
     switch (q) {
         case 0: *sp = s; *cp = c; break;
         case 1: *sp = c; *cp = -s; break;
@@ -252,12 +354,14 @@ BHM_HD void sincos(double x, double* sp, double* cp) {
     }
 }
 
-// atan(t) for t >= 0 (t may be +inf)
-BHM_HD double atan_pos(double t) {
-    bool inv = t > 1.0;
-    if (inv) t = 1.0 / t;
+// atan(t) for 0 <= t <= 1
+BHM_HD double atan_unit(double t) {
     bool red = t > TAN_PI_12;
+#if defined(__HIP_DEVICE_COMPILE__)
+    if (red) t = quot_(t * SQRT3 - 1.0, t + SQRT3);
+#else
     if (red) t = (t * SQRT3 - 1.0) / (t + SQRT3);
+#endif
     double z = t * t;
     // atan t = t + t z A(z), A of degree 8 (fit error 1.6e-18 relative to t)
     double p = -0x1.3ae4ad1dc9d8ap-5;
@@ -270,9 +374,7 @@ BHM_HD double atan_pos(double t) {
     p = horner_(p, z, 0x1.9999999997695p-3);
     p = horner_(p, z, -0x1.555555555554dp-2);
     double a = fma_(t * z, p, t);
-    if (red) a = PI_6 + a;
-    if (inv) a = PI_2 - a;
-    return a;
+    return red ? PI_6 + a : a;
 }
 
 BHM_HD double atan2(double y, double x) {
@@ -280,8 +382,8 @@ BHM_HD double atan2(double y, double x) {
     double ax = fabs_(x), ay = fabs_(y);
     double a;
     if (ay == 0.0 && ax == 0.0) a = 0.0;
-    else if (ay <= ax) a = atan_pos(ay / ax);
-    else a = PI_2 - atan_pos(ax / ay);
+    else if (ay <= ax) a = atan_unit(ay / ax);
+    else a = PI_2 - atan_unit(ax / ay);
     if ((dbits(x) >> 63) != 0) a = PI_ - a;
     return (dbits(y) >> 63) != 0 ? -a : a;
 }

@@ -54,7 +54,7 @@ __device__ __forceinline__ unsigned long long wave_sum(unsigned long long v) {
 
 // Two waves per SIMD at least: with 256-lane workgroups alone the compiler may take VGPRs and AGPRs
 // beyond 256 together (one wave per SIMD); the bound makes it spill to scratch instead.
-template <int PREC, int RADIO, bool RAYS>
+template <int PREC, int RADIO, bool TIME, bool RAYS>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(2))) void k_trace(
     const TraceParams P, const bhm32::MixedParams M, float4* __restrict__ px_out, bh_ray_out* __restrict__ rays_out,
     BlockOut* __restrict__ blk, int per_xcd) {
@@ -75,10 +75,10 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(2))) void
                 bhd::sample_offsets(P, px, py, s, &ox, &oy);
                 int fp64_attempts;
                 if (PREC == BH_PREC_FP64) {
-                    bhd::trace_ray_fp64<RADIO>(P, ox, oy, r);
+                    bhd::trace_ray_fp64<RADIO, TIME>(P, ox, oy, r);
                     fp64_attempts = r.steps;
                 } else {
-                    fp64_attempts = bhm32::trace_ray_mixed<RADIO>(P, M, ox, oy, r);
+                    fp64_attempts = bhm32::trace_ray_mixed<RADIO, TIME>(P, M, ox, oy, r);
                 }
                 a0 += r.I[0];
                 a1 += r.I[1];
@@ -163,13 +163,13 @@ namespace {
 // spills); 1 leaves the register budget to the compiler.
 static_assert(BLOCK == bhp::MAX_BLOCK && NCNT == bhp::NSTAT, "persistent kernel slots");
 
-template <int PREC, int RADIO, int WAVES, class Work>
+template <int PREC, int RADIO, bool TIME, int WAVES, class Work>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WAVES))) void k_persist(
     const Work wk, unsigned int* __restrict__ queue, int interval, int refill_min, int prio_age,
     BlockOut* __restrict__ blk) {
     double flux;
     unsigned long long c[NCNT];
-    bhp::persist_body<PREC, RADIO>(wk, queue, interval, refill_min, prio_age, &flux, c);
+    bhp::persist_body<PREC, RADIO, TIME>(wk, queue, interval, refill_min, prio_age, &flux, c);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
     __shared__ double s_flux[BLOCK / 64];
     __shared__ unsigned long long s_cnt[BLOCK / 64][NCNT];
@@ -534,7 +534,11 @@ TraceParams make_params_scene(const bh_ctx* c, const bh_scene& S, const bh_frame
     P.rh = S.rh;
     P.r_isco = S.r_isco;
     P.tol = S.tol;
-    P.tol4 = S.tol * 4.0;
+    P.inv_tol = 1.0 / S.tol;
+    // numerators of the scaled error above which a step is rejected unscaled: far above any scale, and
+    // low enough that the quotients below it stay finite. A tolerance of zero rejects every error, one
+    // below zero none.
+    P.err_big = S.tol >= 1e-280 ? 1e200 * std::min(1.0, S.tol) : (S.tol >= 0.0 ? 0.0 : HUGE_VAL);
     P.r_escape = S.r_escape;
     P.r_stop = S.r_stop;
     P.step_frac = S.step_frac;
@@ -556,6 +560,7 @@ TraceParams make_params_scene(const bh_ctx* c, const bh_scene& S, const bh_frame
     P.k2_n = c->k2_n;
     P.k2_l0 = c->k2_l0;
     P.k2_dl = c->k2_dl;
+    P.k2_inv_dl = 1.f / c->k2_dl;
     P.turb = c->d_turb;
     P.turb_n = c->turb_n;
     P.turb_nt = c->turb_nt;
@@ -648,6 +653,9 @@ int prepare_turbulence(bh_ctx* c, const bh_scene& S, const bh_frame* f, bool may
     V.zmax = B.zmax;
     V.d0 = B.d0;
     V.dd = B.dd;
+    V.inv_dd = 1.f / B.dd;
+    V.inv_lr = 1.0 / (double)(B.lr1 - B.lr0);
+    V.inv_zmax = 1.0 / (double)B.zmax;
     V.cam_t = B.cam_t;
     V.cam_r = B.cam_r;
     HIPCK(c, hipMemcpyAsync(c->d_tsv, &V, sizeof V, hipMemcpyHostToDevice, c->st));
@@ -666,24 +674,60 @@ int check_frame(bh_ctx* c, const bh_frame* f) {
 
 using KernelFn = void (*)(const TraceParams, const bhm32::MixedParams, float4*, bh_ray_out*, BlockOut*, int);
 
-// The tracers' RADIO argument for a scene mode and the context's turbulence model
-int radio_kind(const bh_ctx* c, int mode) {
-    if (mode != BH_MODE_RADIO) return bhd::RADIO_OFF;
-    return c->turb_model == BH_TURB_SHEARED ? bhd::RADIO_SHEARED : bhd::RADIO_GRID;
+// The tracers' RADIO and TIME arguments for a scene, the context's turbulence model and the call.
+struct Variant {
+    int radio;
+    bool time;
+};
+
+// coordinate-time bound of a mixed-tracer call: the caller's, or the default where the emission
+// depends on the time a sample is emitted at
+double time_bound(const bh_ctx* c, const bh_scene& S, const bh_trace_opts& o);
+
+// The emission reads the coordinate time: time slices, or the sheared model
+bool flow_reads_time(const bh_ctx* c, const bh_scene& S) {
+    return S.mode == BH_MODE_RADIO && S.flow_on &&
+           ((c->turb_model == BH_TURB_GRID && c->d_turb && c->turb_nt > 1) || c->turb_model == BH_TURB_SHEARED);
 }
 
-template <int PREC, bool RAYS>
-KernelFn pick_kernel_p(int radio) {
-    switch (radio) {
-        case bhd::RADIO_SHEARED: return k_trace<PREC, bhd::RADIO_SHEARED, RAYS>;
-        case bhd::RADIO_GRID: return k_trace<PREC, bhd::RADIO_GRID, RAYS>;
-        default: return k_trace<PREC, bhd::RADIO_OFF, RAYS>;
+Variant variant_of(const bh_ctx* c, const bh_scene& S, const bh_trace_opts& o) {
+    Variant v{bhd::RADIO_OFF, flow_reads_time(c, S)};
+    if (S.mode == BH_MODE_RADIO) v.radio = c->turb_model == BH_TURB_SHEARED ? bhd::RADIO_SHEARED : bhd::RADIO_GRID;
+    if (o.precision == BH_PREC_MIXED && time_bound(c, S, o) > 0.0) v.time = true;
+    return v;
+}
+
+// The kernel `at<RADIO, TIME>()` of a variant. ALWAYS: the kernel reads the coordinate time whatever
+// the frame (ray records). The sheared model always reads it, and the FP64 tracer of a vacuum frame
+// never does.
+template <int PREC, bool ALWAYS, class At>
+auto pick_variant(const Variant& v, const At& at) {
+    switch (v.radio) {
+        case bhd::RADIO_SHEARED: return at.template operator()<bhd::RADIO_SHEARED, true>();
+        case bhd::RADIO_GRID:
+            return v.time ? at.template operator()<bhd::RADIO_GRID, true>() : at.template operator()<bhd::RADIO_GRID, ALWAYS>();
+        default:
+            return v.time ? at.template operator()<bhd::RADIO_OFF, ALWAYS || PREC == BH_PREC_MIXED>()
+                          : at.template operator()<bhd::RADIO_OFF, ALWAYS>();
     }
 }
 
-KernelFn pick_kernel(int prec, int radio, bool rays) {
-    if (prec == BH_PREC_FP64) return rays ? pick_kernel_p<BH_PREC_FP64, true>(radio) : pick_kernel_p<BH_PREC_FP64, false>(radio);
-    return rays ? pick_kernel_p<BH_PREC_MIXED, true>(radio) : pick_kernel_p<BH_PREC_MIXED, false>(radio);
+template <int PREC, bool RAYS>
+struct TraceAt {
+    template <int RADIO, bool TIME>
+    KernelFn operator()() const {
+        return k_trace<PREC, RADIO, TIME, RAYS>;
+    }
+};
+
+template <bool RAYS>
+KernelFn pick_kernel_r(int prec, const Variant& v) {
+    return prec == BH_PREC_FP64 ? pick_variant<BH_PREC_FP64, RAYS>(v, TraceAt<BH_PREC_FP64, RAYS>{})
+                                : pick_variant<BH_PREC_MIXED, RAYS>(v, TraceAt<BH_PREC_MIXED, RAYS>{});
+}
+
+KernelFn pick_kernel(int prec, const Variant& v, bool rays) {
+    return rays ? pick_kernel_r<true>(prec, v) : pick_kernel_r<false>(prec, v);
 }
 
 constexpr double C_C = 2.99792458e10, C_H = 6.62607015e-27, C_ME = 9.1093837e-28, C_MP = 1.67262192e-24,
@@ -741,6 +785,10 @@ double emission_radius(const bh_scene& S, const std::vector<float>& k2, float k2
 
 // Default bound on a mixed-tracer step's coordinate-time error (M) for time-dependent turbulence
 constexpr double DEFAULT_TOL_T = 1e-3;
+double time_bound(const bh_ctx* c, const bh_scene& S, const bh_trace_opts& o) {
+    if (o.tol_t > 0) return o.tol_t;
+    return o.tol_t == 0 && flow_reads_time(c, S) && S.flow_turb_amp > 0.f ? DEFAULT_TOL_T : 0.0;
+}
 // Default long-ray relaxation: off until measured
 constexpr int DEFAULT_RELAX_AFTER = 0;
 constexpr double DEFAULT_TOL_RELAX = 1e-9;
@@ -795,17 +843,8 @@ bhm32::MixedParams make_mixed(bh_ctx* c, const bh_scene& S, const bh_frame* f, c
         if (!o.full_flow) M.tol_mid = std::max(M.tol_mid, M.tol_far * 0.1);
     }
     M.r_f32 = o.far_fp32 ? M.r_far : 1e300;
-    // coordinate-time bound: only where the emission depends on the time a sample is emitted at
-    const bool time_dependent = S.mode == BH_MODE_RADIO && S.flow_on && S.flow_turb_amp > 0.f &&
-                                ((c->turb_model == BH_TURB_GRID && c->d_turb && c->turb_nt > 1) ||
-                                 c->turb_model == BH_TURB_SHEARED);
-    const double tol_t = o.tol_t > 0 ? o.tol_t : (o.tol_t == 0 && time_dependent ? DEFAULT_TOL_T : 0.0);
+    const double tol_t = time_bound(c, S, o);
     M.inv_tol_t = tol_t > 0 ? 1.0 / tol_t : 0.0;
-    // the FP64 stages integrate t only where the emission reads it (time slices, the sheared model,
-    // a t bound); launch_trace_into sets it for ray records as well
-    M.need_t = (S.mode == BH_MODE_RADIO && S.flow_on &&
-                ((c->turb_model == BH_TURB_GRID && c->d_turb && c->turb_nt > 1) ||
-                 c->turb_model == BH_TURB_SHEARED)) || tol_t > 0;
     // long-ray relaxation of the emission-region tolerance
     M.relax_after = o.relax_after > 0 ? o.relax_after : (o.relax_after == 0 ? DEFAULT_RELAX_AFTER : 0x7fffffff);
     M.tol_relax = o.tol_relax > 0 ? o.tol_relax : std::max(S.tol, DEFAULT_TOL_RELAX);
@@ -869,7 +908,6 @@ int launch_trace_into(bh_ctx* c, const bh_frame* f, const bh_trace_opts& o, int 
                       float4* px, bh_ray_out* rays_out, BlockOut* blk, BlockOut* tot_dev, bool may_alloc,
                       bh_stats* st) {
     bhm32::MixedParams M = make_mixed(c, c->S, f, o);
-    if (rays) M.need_t = 1;   // the records carry t
     if (o.emissivity == BH_EMIS_MLP) {
         M.use_surrogate = 1;
         M.S = c->stab;
@@ -886,7 +924,7 @@ int launch_trace_into(bh_ctx* c, const bh_frame* f, const bh_trace_opts& o, int 
     P.jitter = o.jitter;
     int per_xcd;
     const int nb = trace_blocks(w, h, &per_xcd);
-    KernelFn k = pick_kernel(o.precision, radio_kind(c, c->S.mode), rays);
+    KernelFn k = pick_kernel(o.precision, variant_of(c, c->S, o), rays);
     HIPCK(c, hipEventRecord(c->ev0, c->st));
     hipLaunchKernelGGL(k, dim3(nb), dim3(BLOCK), 0, c->st, P, M, px, rays_out, blk, per_xcd);
     HIPCK(c, hipGetLastError());
@@ -938,36 +976,31 @@ template <class Work>
 using WorkFn = void (*)(const Work, unsigned int*, int, int, int, BlockOut*);
 
 template <int PREC, int W, class Work>
-WorkFn<Work> pick_persist_p(int radio) {
-    switch (radio) {
-        case bhd::RADIO_SHEARED: return k_persist<PREC, bhd::RADIO_SHEARED, W, Work>;
-        case bhd::RADIO_GRID: return k_persist<PREC, bhd::RADIO_GRID, W, Work>;
-        default: return k_persist<PREC, bhd::RADIO_OFF, W, Work>;
+struct PersistAt {
+    template <int RADIO, bool TIME>
+    WorkFn<Work> operator()() const {
+        return k_persist<PREC, RADIO, TIME, W, Work>;
     }
-}
+};
 
 template <int W, class Work>
-WorkFn<Work> pick_persist_pw(int prec, int radio) {
-    return prec == BH_PREC_FP64 ? pick_persist_p<BH_PREC_FP64, W, Work>(radio) : pick_persist_p<BH_PREC_MIXED, W, Work>(radio);
+WorkFn<Work> pick_persist_w(int prec, const Variant& v) {
+    return prec == BH_PREC_FP64 ? pick_variant<BH_PREC_FP64, Work::RECORDS>(v, PersistAt<BH_PREC_FP64, W, Work>{})
+                                : pick_variant<BH_PREC_MIXED, Work::RECORDS>(v, PersistAt<BH_PREC_MIXED, W, Work>{});
 }
 
-template <int W>
-PersistFn pick_persist_w(int prec, int radio) {
-    return pick_persist_pw<W, bhp::BatchWork>(prec, radio);
-}
-
-// adaptive passes: the kernel compiled for at least 3 waves per SIMD (waves 3 or 4) or for the
-// compiler's register budget (waves 0)
+// adaptive passes and ray records: the kernel compiled for at least 3 waves per SIMD (waves 3 or 4) or
+// for the compiler's register budget (waves 0)
 template <class Work>
-WorkFn<Work> pick_adaptive(int prec, int radio, int waves) {
-    return waves >= 3 ? pick_persist_pw<3, Work>(prec, radio) : pick_persist_pw<1, Work>(prec, radio);
+WorkFn<Work> pick_adaptive(int prec, const Variant& v, int waves) {
+    return waves >= 3 ? pick_persist_w<3, Work>(prec, v) : pick_persist_w<1, Work>(prec, v);
 }
 
-PersistFn pick_persist(int prec, int radio, int waves) {
+PersistFn pick_persist(int prec, const Variant& v, int waves) {
     switch (waves) {
-        case 3: return pick_persist_w<3>(prec, radio);
-        case 4: return pick_persist_w<4>(prec, radio);
-        default: return pick_persist_w<1>(prec, radio);
+        case 3: return pick_persist_w<3, bhp::BatchWork>(prec, v);
+        case 4: return pick_persist_w<4, bhp::BatchWork>(prec, v);
+        default: return pick_persist_w<1, bhp::BatchWork>(prec, v);
     }
 }
 
@@ -1120,7 +1153,10 @@ int launch_batch(bh_ctx* c, const bh_batch_frame* frames, int n, const bh_trace_
         }
     }
     const int prio = cfg.prio_age > 0 ? cfg.prio_age : 0;
-    PersistFn k = pick_persist(o.precision, radio_kind(c, mode), cfg.waves);
+    // one kernel for all frames: it integrates the coordinate time if any of them reads it
+    Variant v = variant_of(c, frames[0].scene, o);
+    for (int i = 1; i < n; ++i) v.time = v.time || variant_of(c, frames[i].scene, o).time;
+    PersistFn k = pick_persist(o.precision, v, cfg.waves);
     const int grid = persist_grid(c, (const void*)k, cfg.block, cfg.grid_per_cu);
     rc = ensure(c, &c->d_bframes, &c->bframes_cap, sizeof(bhp::BatchFrame) * (size_t)n);
     if (rc) return rc;
@@ -1212,7 +1248,7 @@ int launch_records(bh_ctx* c, const bh_frame* f, const bh_trace_opts* opts, int 
     if (rc) return rc;
     rc = prepare_turbulence(c, c->S, f);
     if (rc) return rc;
-    const auto k = pick_adaptive<bhp::RecordWork>(o.precision, radio_kind(c, c->S.mode), cfg.waves);
+    const auto k = pick_adaptive<bhp::RecordWork>(o.precision, variant_of(c, c->S, o), cfg.waves);
     const int grid = persist_grid(c, (const void*)k, cfg.block, cfg.grid_per_cu);
     const int tiles_x = (w + 7) / 8, tiles = tiles_x * ((h + 7) / 8);
     bhp::BatchFrame B;
@@ -1225,7 +1261,6 @@ int launch_records(bh_ctx* c, const bh_frame* f, const bh_trace_opts* opts, int 
     B.P.spp = 1;
     B.P.jitter = o.jitter;
     B.M = make_mixed(c, c->S, f, o);
-    B.M.need_t = 1;   // the records carry t
     if (o.emissivity == BH_EMIS_MLP) {
         B.M.use_surrogate = 1;
         B.M.S = c->stab;
@@ -1279,7 +1314,7 @@ int launch_adaptive(bh_ctx* c, const bh_frame* f, const bh_trace_opts* opts, lon
     if (rc) return rc;
     rc = prepare_turbulence(c, c->S, f);
     if (rc) return rc;
-    const int rk = radio_kind(c, c->S.mode);
+    const Variant rk = variant_of(c, c->S, o);
     const auto k1 = pick_adaptive<bhp::SampleWork>(o.precision, rk, cfg.waves);
     const auto k2 = pick_adaptive<bhp::ChunkWork>(o.precision, rk, cfg.waves);
     const int grid = std::min(persist_grid(c, (const void*)k1, cfg.block, cfg.grid_per_cu),

@@ -46,11 +46,13 @@ __device__ __forceinline__ void tile_pixel(int tiles_x, unsigned int tile, unsig
     *py = (int)(tile / (unsigned)tiles_x) * 8 + (int)(within >> 3);
 }
 
-/* Work mappings: entry e of frame f -> (pixel, sample index) and where a finished ray goes.
+/* Work mappings: entry e of frame f -> (pixel, sample index) and where a finished ray goes. RECORDS: the
+   finished ray's coordinate time is part of the output.
    Entries of 64 consecutive indices are 8 x 8 pixel tiles, so a wave's rays are image neighbours. */
 
 // Frame batches: one pixel-centre (or jittered sample 0) ray per pixel, written as a float4 pixel.
 struct BatchWork {
+    static constexpr bool RECORDS = false;
     const BatchFrame* frames;
     int n;
     __device__ __forceinline__ bool begin(int f, unsigned int e, int* px, int* py, int* s) const {
@@ -88,6 +90,7 @@ __device__ __forceinline__ void write_record(bh_ray_out* __restrict__ q, const R
 // region's size and P.x0 / P.y0 its origin; one ray per pixel (centre, or jittered sample 0), its
 // record at out[(py - y0) * w + (px - x0)].
 struct RecordWork {
+    static constexpr bool RECORDS = true;
     const BatchFrame* frames;   // one frame
     int n;
     bh_ray_out* out;
@@ -110,6 +113,7 @@ struct RecordWork {
 // First pass of adaptive sampling: samples 0..spp-1 of every pixel (entry = tile, sample, pixel in
 // tile), each kept in FP64 at out[pixel * spp + sample].
 struct SampleWork {
+    static constexpr bool RECORDS = false;
     const BatchFrame* frames;   // one frame
     int n;
     int spp;
@@ -132,6 +136,7 @@ struct SampleWork {
 // the last pixel p with offsets[p] <= g; its 8 samples continue p's sequence at
 // spp + 8 * (g - offsets[p]). Each sample is kept in FP64 at out[entry].
 struct ChunkWork {
+    static constexpr bool RECORDS = false;
     const BatchFrame* frames;   // one frame
     int n;
     int spp;
@@ -158,18 +163,18 @@ struct ChunkWork {
     }
 };
 
-template <int PREC, int RADIO>
+template <int PREC, int RADIO, bool TIME>
 struct Tracer;
 
-template <int RADIO>
-struct Tracer<BH_PREC_FP64, RADIO> {
+template <int RADIO, bool TIME>
+struct Tracer<BH_PREC_FP64, RADIO, TIME> {
     using State = bhd::RayState;
     static __device__ __forceinline__ void init(const TraceParams& P, const bhm32::MixedParams&, double x, double y,
                                                 State& R) {
         bhd::ray_init<RADIO>(P, x, y, R);
     }
     static __device__ __forceinline__ void step(const TraceParams& P, const bhm32::MixedParams&, State& R) {
-        bhd::ray_step<RADIO>(P, R);
+        bhd::ray_step<RADIO, TIME>(P, R);
     }
     static __device__ __forceinline__ int result(const TraceParams& P, const State& R, RayResult& out) {
         bhd::ray_result(P, R, out);
@@ -177,26 +182,26 @@ struct Tracer<BH_PREC_FP64, RADIO> {
     }
 };
 
-template <int RADIO>
-struct Tracer<BH_PREC_MIXED, RADIO> {
+template <int RADIO, bool TIME>
+struct Tracer<BH_PREC_MIXED, RADIO, TIME> {
     using State = bhm32::RayStateM;
     static __device__ __forceinline__ void init(const TraceParams& P, const bhm32::MixedParams& M, double x, double y,
                                                 State& R) {
         bhm32::ray_init_m<RADIO>(P, M, x, y, R);
     }
     static __device__ __forceinline__ void step(const TraceParams& P, const bhm32::MixedParams& M, State& R) {
-        bhm32::ray_step_m<RADIO>(P, M, R);
+        bhm32::ray_step_m<RADIO, TIME>(P, M, R);
     }
     static __device__ __forceinline__ int result(const TraceParams& P, const State& R, RayResult& out) {
         return bhm32::ray_result_m(P, R, out);
     }
 };
 
-template <int PREC, int RADIO, class Work>
+template <int PREC, int RADIO, bool TIME, class Work>
 __device__ __forceinline__ void persist_body(const Work& Wk, unsigned int* __restrict__ queue, int interval,
                                              int refill_min, int prio_age, double* flux_out,
                                              unsigned long long* cnt_out) {
-    using T = Tracer<PREC, RADIO>;
+    using T = Tracer<PREC, RADIO, TIME>;
     const BatchFrame* __restrict__ frames = Wk.frames;
     const int nframes = Wk.n;
     const int lane = threadIdx.x & 63;

@@ -14,7 +14,18 @@
    - The phi and t components never enter the right-hand side (kerr.hpp:103-116), so their stage
      states are never formed; only their 5th-order sums (and phi's error term) are kept.
    - d[0] = y[1] and d[2] = y[3]: the r and u components of each stage derivative are the stage
-     state's r' and u' and are not stored separately. */
+     state's r' and u' and are not stored separately.
+   - The coordinate time enters neither the right-hand side nor the error norm, so a frame that reads
+     it nowhere (static turbulence, no ray records) does not integrate it.
+   - The kernels are bound by VALU issue, so the correctly rounded quotients and roots take their
+     shortest form (bh_math.h quot_, sqrt_pos_): the operators' range scaling and fix-up are half of
+     their instructions and the operands here stay far from the ends of the exponent range. Where one
+     can leave it (a stage inside the horizon or past the pole, a step that diverged), the code below
+     says what catches it. With the time left out where nothing reads it, one power per attempt and the
+     sine, cosine and root of the swept angle handed on to the flow, the bound per attempt fell by a
+     third at the same bits: 1024^2 230 GHz frame 27.8 -> 20.3 ms, 160^2 normalising flux 15.5 -> 9.7
+     ms, 256^2 vacuum records 5.2 -> 4.1 ms (static VALU instructions of the frame's persistent kernel
+     3997 -> 2885, 164 -> 140 VGPRs). */
 #pragma once
 #include "bh_math.h"
 
@@ -29,6 +40,9 @@ constexpr double PI = 3.14159265358979323846;
 // turbulence or with the sheared turbulence. The turbulence model is a compile-time choice so a
 // kernel carries the lookup code of one model only (registers and instruction cache).
 constexpr int RADIO_OFF = 0, RADIO_GRID = 1, RADIO_SHEARED = 2;
+// The TIME template argument: whether something reads the coordinate time (time-dependent turbulence,
+// ray records, a bound on its error); without it t is not integrated. A compile-time choice too: both
+// steps in one kernel cost 26 registers (166 and 140 alone, 168 and spills together).
 constexpr int MODE_VISIBLE = 0;   // bh_scene.mode: vacuum geodesics and the celestial sphere
 
 // Dormand-Prince 1980 tableau (kerr.hpp:124-129): the same constant expressions, folded by the compiler.
@@ -45,18 +59,22 @@ struct ShearedView {
     const float* data;
     int nphi, nlr, nz, nt;
     float lr0, lr1, zmax, d0, dd;
+    float inv_dd;               // 1 / dd
+    double inv_lr, inv_zmax;    // 1 / (lr1 - lr0), 1 / zmax
     double cam_t, cam_r;
 };
 
 // Uniform scene and frame parameters: passed by value as the kernel argument, so they sit in SGPRs.
 struct TraceParams {
     // scene (bh_scene)
-    double a, a2, rh, r_isco, tol, tol4, r_escape, r_stop, step_frac;
+    double a, a2, rh, r_isco, tol, r_escape, r_stop, step_frac;
+    double inv_tol;   // 1 / tol
+    double err_big;   // scaled errors whose numerators exceed this are rejected unscaled (dp54_step)
     int max_steps, mode, flow_on, turb_on;
     double n0, n_index, theta_index, theta0, h_r, beta_p, r_flow_max, nu_obs, rg_cm, flow_kep;
     const float* __restrict__ k2;
     int k2_n;
-    float k2_l0, k2_dl;
+    float k2_l0, k2_dl, k2_inv_dl;
     const float* __restrict__ turb;
     int turb_n, turb_nt;
     double turb_half, turb_inv_dx, turb_t0, turb_inv_dt;
@@ -122,6 +140,10 @@ __device__ __forceinline__ void sample_offsets(const TraceParams& P, int px, int
 struct Rhs {
     double d1, d3, d4, d5;
 };
+// The quotients by Delta share its reciprocal; Delta may vanish or overflow at a wild stage, which
+// the fix-up instruction turns into the IEEE result. s2 is at least 1e-300, so lam / s2 needs none
+// (past the pole it is finite for |lam| < 1e8). Without TIME d5 is not formed.
+template <bool TIME>
 __device__ __forceinline__ Rhs rhs(const TraceParams& P, const RayConst& c, double r, double u) {
     double r2 = r * r;
     double Delta = r2 - 2.0 * r + P.a2;
@@ -130,8 +152,15 @@ __device__ __forceinline__ Rhs rhs(const TraceParams& P, const RayConst& c, doub
     Rhs o;
     o.d1 = 2.0 * r * Pp - (r - 1.0) * c.K;
     o.d3 = u * (P.a2 * (1.0 - 2.0 * u * u) - c.eta - c.lam2);
-    o.d4 = -(P.a * Pp / Delta + c.lam / s2 - P.a);
-    o.d5 = -((r2 + P.a2) * Pp / Delta + P.a * (c.lam - P.a * s2));
+    const bhm::Recip iD = bhm::recip_(Delta);
+    const double n4 = P.a * Pp;
+    o.d4 = -(__builtin_amdgcn_div_fixup(bhm::quot_(n4, iD), Delta, n4) + bhm::quot_(c.lam, s2) - P.a);
+    if (TIME) {
+        const double n5 = (r2 + P.a2) * Pp;
+        o.d5 = -(__builtin_amdgcn_div_fixup(bhm::quot_(n5, iD), Delta, n5) + P.a * (c.lam - P.a * s2));
+    } else {
+        o.d5 = 0.0;
+    }
     return o;
 }
 
@@ -142,6 +171,7 @@ struct State {
 };
 
 // blackholes/src/kerr.hpp:122-157. Returns the scaled error; on return `o` holds (yout, k7).
+template <bool TIME>
 __device__ __forceinline__ double dp54_step(const TraceParams& P, const RayConst& c, const State& s, double h,
                                             State& o) {
     // partial sums of stages 3..6, of the 5th-order increment (O) and of the error (E), per component
@@ -152,11 +182,11 @@ __device__ __forceinline__ double dp54_step(const TraceParams& P, const RayConst
     double S4_0 = a41 * q0, S4_1 = a41 * q1, S4_2 = a41 * q2, S4_3 = a41 * q3;
     double S5_0 = a51 * q0, S5_1 = a51 * q1, S5_2 = a51 * q2, S5_3 = a51 * q3;
     double S6_0 = a61 * q0, S6_1 = a61 * q1, S6_2 = a61 * q2, S6_3 = a61 * q3;
-    double O0 = b1 * q0, O1 = b1 * q1, O2 = b1 * q2, O3 = b1 * q3, O4 = b1 * s.k4, O5 = b1 * s.k5;
+    double O0 = b1 * q0, O1 = b1 * q1, O2 = b1 * q2, O3 = b1 * q3, O4 = b1 * s.k4, O5 = TIME ? b1 * s.k5 : 0.0;
     double E0 = e1 * q0, E1 = e1 * q1, E2 = e1 * q2, E3 = e1 * q3, E4 = e1 * s.k4;
     // stage 2
     double t0 = s.y0 + ha21 * q0, t1 = s.y1 + ha21 * q1, t2 = s.y2 + ha21 * q2, t3 = s.y3 + ha21 * q3;
-    Rhs k = rhs(P, c, t0, t2);
+    Rhs k = rhs<TIME>(P, c, t0, t2);
     q0 = t1; q1 = k.d1; q2 = t3; q3 = k.d3;
     S3_0 = S3_0 + a32 * q0; S3_1 = S3_1 + a32 * q1; S3_2 = S3_2 + a32 * q2; S3_3 = S3_3 + a32 * q3;
     S4_0 = S4_0 + a42 * q0; S4_1 = S4_1 + a42 * q1; S4_2 = S4_2 + a42 * q2; S4_3 = S4_3 + a42 * q3;
@@ -164,64 +194,92 @@ __device__ __forceinline__ double dp54_step(const TraceParams& P, const RayConst
     S6_0 = S6_0 + a62 * q0; S6_1 = S6_1 + a62 * q1; S6_2 = S6_2 + a62 * q2; S6_3 = S6_3 + a62 * q3;
     // stage 3
     t0 = s.y0 + h * S3_0; t1 = s.y1 + h * S3_1; t2 = s.y2 + h * S3_2; t3 = s.y3 + h * S3_3;
-    k = rhs(P, c, t0, t2);
+    k = rhs<TIME>(P, c, t0, t2);
     q0 = t1; q1 = k.d1; q2 = t3; q3 = k.d3;
     S4_0 = S4_0 + a43 * q0; S4_1 = S4_1 + a43 * q1; S4_2 = S4_2 + a43 * q2; S4_3 = S4_3 + a43 * q3;
     S5_0 = S5_0 + a53 * q0; S5_1 = S5_1 + a53 * q1; S5_2 = S5_2 + a53 * q2; S5_3 = S5_3 + a53 * q3;
     S6_0 = S6_0 + a63 * q0; S6_1 = S6_1 + a63 * q1; S6_2 = S6_2 + a63 * q2; S6_3 = S6_3 + a63 * q3;
     O0 = O0 + b3 * q0; O1 = O1 + b3 * q1; O2 = O2 + b3 * q2; O3 = O3 + b3 * q3; O4 = O4 + b3 * k.d4;
-    O5 = O5 + b3 * k.d5;
+    if (TIME) O5 = O5 + b3 * k.d5;
     E0 = E0 + e3 * q0; E1 = E1 + e3 * q1; E2 = E2 + e3 * q2; E3 = E3 + e3 * q3; E4 = E4 + e3 * k.d4;
     // stage 4
     t0 = s.y0 + h * S4_0; t1 = s.y1 + h * S4_1; t2 = s.y2 + h * S4_2; t3 = s.y3 + h * S4_3;
-    k = rhs(P, c, t0, t2);
+    k = rhs<TIME>(P, c, t0, t2);
     q0 = t1; q1 = k.d1; q2 = t3; q3 = k.d3;
     S5_0 = S5_0 + a54 * q0; S5_1 = S5_1 + a54 * q1; S5_2 = S5_2 + a54 * q2; S5_3 = S5_3 + a54 * q3;
     S6_0 = S6_0 + a64 * q0; S6_1 = S6_1 + a64 * q1; S6_2 = S6_2 + a64 * q2; S6_3 = S6_3 + a64 * q3;
     O0 = O0 + b4 * q0; O1 = O1 + b4 * q1; O2 = O2 + b4 * q2; O3 = O3 + b4 * q3; O4 = O4 + b4 * k.d4;
-    O5 = O5 + b4 * k.d5;
+    if (TIME) O5 = O5 + b4 * k.d5;
     E0 = E0 + e4 * q0; E1 = E1 + e4 * q1; E2 = E2 + e4 * q2; E3 = E3 + e4 * q3; E4 = E4 + e4 * k.d4;
     // stage 5
     t0 = s.y0 + h * S5_0; t1 = s.y1 + h * S5_1; t2 = s.y2 + h * S5_2; t3 = s.y3 + h * S5_3;
-    k = rhs(P, c, t0, t2);
+    k = rhs<TIME>(P, c, t0, t2);
     q0 = t1; q1 = k.d1; q2 = t3; q3 = k.d3;
     S6_0 = S6_0 + a65 * q0; S6_1 = S6_1 + a65 * q1; S6_2 = S6_2 + a65 * q2; S6_3 = S6_3 + a65 * q3;
     O0 = O0 + b5 * q0; O1 = O1 + b5 * q1; O2 = O2 + b5 * q2; O3 = O3 + b5 * q3; O4 = O4 + b5 * k.d4;
-    O5 = O5 + b5 * k.d5;
+    if (TIME) O5 = O5 + b5 * k.d5;
     E0 = E0 + e5 * q0; E1 = E1 + e5 * q1; E2 = E2 + e5 * q2; E3 = E3 + e5 * q3; E4 = E4 + e5 * k.d4;
     // stage 6
     t0 = s.y0 + h * S6_0; t1 = s.y1 + h * S6_1; t2 = s.y2 + h * S6_2; t3 = s.y3 + h * S6_3;
-    k = rhs(P, c, t0, t2);
+    k = rhs<TIME>(P, c, t0, t2);
     q0 = t1; q1 = k.d1; q2 = t3; q3 = k.d3;
     O0 = O0 + b6 * q0; O1 = O1 + b6 * q1; O2 = O2 + b6 * q2; O3 = O3 + b6 * q3; O4 = O4 + b6 * k.d4;
-    O5 = O5 + b6 * k.d5;
+    if (TIME) O5 = O5 + b6 * k.d5;
     E0 = E0 + e6 * q0; E1 = E1 + e6 * q1; E2 = E2 + e6 * q2; E3 = E3 + e6 * q3; E4 = E4 + e6 * k.d4;
     // 5th-order solution and its derivative (FSAL)
     o.y0 = s.y0 + h * O0; o.y1 = s.y1 + h * O1; o.y2 = s.y2 + h * O2; o.y3 = s.y3 + h * O3;
-    o.y4 = s.y4 + h * O4; o.y5 = s.y5 + h * O5;
-    k = rhs(P, c, o.y0, o.y2);
-    o.k1 = k.d1; o.k3 = k.d3; o.k4 = k.d4; o.k5 = k.d5;
+    o.y4 = s.y4 + h * O4; o.y5 = TIME ? s.y5 + h * O5 : s.y5;
+    k = rhs<TIME>(P, c, o.y0, o.y2);
+    o.k1 = k.d1; o.k3 = k.d3; o.k4 = k.d4; o.k5 = TIME ? k.d5 : s.k5;
     E0 = E0 + e7 * o.y1; E1 = E1 + e7 * k.d1; E2 = E2 + e7 * o.y3; E3 = E3 + e7 * k.d3; E4 = E4 + e7 * k.d4;
-    // scaled max-norm over r, r', u, u', phi (kerr.hpp:145-155)
-    double sc0 = P.tol * (1e-6 + fmax(fabs(s.y0), fabs(o.y0)));
-    double sc1 = P.tol * (1e-6 + fmax(fmax(fabs(s.y1), fabs(o.y1)), s.y0 * s.y0));
-    double sc3 = P.tol * fmax(1.0, fmax(fabs(s.y3), fabs(o.y3)));
-    double m = 0.0;
-    m = fmax(m, fabs(h * E0) / sc0);
-    m = fmax(m, fabs(h * E1) / sc1);
-    m = fmax(m, fabs(h * E2) / P.tol);
-    m = fmax(m, fabs(h * E3) / sc3);
-    m = fmax(m, fabs(h * E4) / P.tol4);
-    return m;
+    // scaled max-norm over r, r', u, u', phi (kerr.hpp:145-155): max_i |h E_i| / sc_i with sc = tol
+    // for u and 4 tol for phi. Rounding is monotone and the factor 4 exact, so those two quotients are
+    // the one of their larger numerator.
+    const double x0 = fabs(h * E0), x1 = fabs(h * E1), x3 = fabs(h * E3);
+    const double x2 = fmax(fabs(h * E2), 0.25 * fabs(h * E4));
+    const double sc0 = P.tol * (1e-6 + fmax(fabs(s.y0), fabs(o.y0)));
+    const double sc1 = P.tol * (1e-6 + fmax(fmax(fabs(s.y1), fabs(o.y1)), s.y0 * s.y0));
+    const double sc3 = P.tol * fmax(1.0, fmax(fabs(s.y3), fabs(o.y3)));
+    double m = fmax(0.0, bhm::quot_(x0, sc0));
+    m = fmax(m, bhm::quot_(x1, sc1));
+    m = fmax(m, bhm::quot_(x2, bhm::Recip{P.tol, P.inv_tol}));
+    m = fmax(m, bhm::quot_(x3, sc3));
+    // A diverged step (an error beyond 1e200 tol, an infinity) is rejected without its quotients, which
+    // could overflow: the controller's factor is 0.2 for every error above 2e3. A NaN is no error, as
+    // in the maximum above and in the reference's.
+    return fmax(fmax(x0, x1), fmax(x2, x3)) > P.err_big ? 1e300 : m;
 }
 
+// The controller's factor min(5, max(0.2, 0.9 err^-0.2)) (trace.cuh:88,146) with the correctly rounded
+// power of bhm::pow_m02. Errors outside [1e-6, 1e6] give the limits, so the argument is clamped there
+// and the seed comes from the hardware's FP32 base-2 units (3e-7 relative) instead of the FP64 log and
+// exp: two plain Newton steps on x y^5 = 1 (3e-13, then rounding), then pow_m02's last step, whose
+// residual is formed in double-double. One evaluation serves both outcomes of a step (a rejected
+// step's factor is below 0.9): 46 operations for 100, and lanes that disagree share them.
+__device__ __forceinline__ double step_factor(double err) {
+    const double x = fmin(fmax(err, 1e-6), 1e6);
+    const float l2 = __builtin_amdgcn_logf((float)x);
+    double y = (double)__builtin_amdgcn_exp2f(-0.2f * l2);
+    for (int i = 0; i < 2; ++i) {
+        const double y2 = y * y;
+        y = fma(y * 0.2, fma(-x, y2 * y2 * y, 1.0), y);
+    }
+    const double p2 = y * y, e2 = fma(y, y, -p2);
+    const double p4 = p2 * p2, e4 = fma(2.0 * p2, e2, fma(p2, p2, -p4));
+    const double p5 = p4 * y, e5 = fma(e4, y, fma(p4, y, -p5));
+    const double p6 = p5 * x, e6 = fma(e5, x, fma(p5, x, -p6));
+    const double r = (1.0 - p6) - e6;
+    // the double nearest 0.2 is 2^-56 * 4/5 above it: x^-0.2 = x^(-1/5) (1 - that * ln x)
+    const double off = (double)(l2 * (0x1.999999999999ap-57f * 0.6931471805599453f));
+    return fmin(5.0, fmax(0.2, 0.9 * fma(y, fma(r, 0.2, -off), y)));
+}
 // blackholes/src/kerr.hpp:166-173
 __device__ __forceinline__ void project_radial(const TraceParams& P, const RayConst& c, State& s) {
     double r = s.y0;
     double Pp = r * r + P.a2 - c.alam, D = r * r - 2.0 * r + P.a2;
     double R = Pp * Pp - D * c.K;
     if (R > 0.25 * r * r * r * r) {
-        double v = sqrt(R);
+        double v = bhm::sqrt_pos_(R);
         s.y1 = s.y1 < 0.0 ? -v : v;
     }
 }
@@ -229,6 +287,18 @@ __device__ __forceinline__ void project_radial(const TraceParams& P, const RayCo
 // blackholes/src/device_util.cuh:74-80
 __device__ __forceinline__ float table_lerp(const float* __restrict__ t, int n, float x0, float dx, float x) {
     float f = (x - x0) / dx;
+    f = fminf(fmaxf(f, 0.f), (float)(n - 2) + 0.9999f);
+    int i = (int)f;
+    f -= i;
+    float t0 = t[i], t1 = t[i + 1];
+    return t0 + (t1 - t0) * f;
+}
+
+// The same with 1 / dx (correctly rounded) at hand: the quotient by its residual, as bhm::quot_.
+__device__ __forceinline__ float table_lerp(const float* __restrict__ t, int n, float x0, float dx, float inv_dx,
+                                            float x) {
+    const float a = x - x0, q = a * inv_dx;
+    float f = fmaf(fmaf(-dx, q, a), inv_dx, q);
     f = fminf(fmaxf(f, 0.f), (float)(n - 2) + 0.9999f);
     int i = (int)f;
     f -= i;
@@ -265,10 +335,8 @@ __device__ __forceinline__ double grid_trilinear(const TraceParams& P, const flo
     return c0 + (c1 - c0) * fz;
 }
 
-__device__ __forceinline__ double turb_factor(const TraceParams& P, double r, double u, double phi, double t) {
-    double s = sqrt(fmax(1.0 - u * u, 1e-12));
-    double R = r * s, sp, cp;
-    bhm::sincos(phi, &sp, &cp);
+__device__ __forceinline__ double turb_factor(const TraceParams& P, double r, double R, double u, double sp,
+                                              double cp, double t) {
     double px = R * cp, py = R * sp, pz = r * u;
     if (P.turb_nt <= 1) return grid_trilinear(P, P.turb, px, py, pz);
     // time slices: linear in coordinate time, clamped to the first/last slice
@@ -283,64 +351,88 @@ __device__ __forceinline__ double turb_factor(const TraceParams& P, double r, do
     return A + (B - A) * f;
 }
 
-// blackholes/src/emission.cuh:99-175 (exact thermal-synchrotron coefficients)
+// a / b for a constant b of the physics
+__device__ __forceinline__ double quot_const(double a, double b, double inv_b) {
+    return bhm::quot_(a, bhm::Recip{b, inv_b});
+}
+
+// blackholes/src/emission.cuh:99-175 (exact thermal-synchrotron coefficients). w = 1 - u^2, sn =
+// sqrt(max(w, 0)) and the azimuth's sine and cosine are those of the swept angle: the flow and the
+// turbulence lookup read the same values. Quotients whose operands a scene or a sample can make zero
+// or infinite keep the IEEE fix-up; j / B_nu keeps the operator (j falls to the denormals).
 template <int RADIO>
-__device__ __forceinline__ void flow_step(const TraceParams& P, double r, double u, double phi, double t, double lam,
-                                          double Ecam, double h, double* dI, double* dtau) {
+__device__ __forceinline__ void flow_step(const TraceParams& P, double r, double u, double w, double sn, double phi,
+                                          double sv, double cv, double t, double lam, double Ecam, double h, double* dI,
+                                          double* dtau) {
+    using bhm::quot_;
+    using bhm::quot_ieee_;
+    using bhm::sqrt_pos_;
     *dI = 0.0;
     *dtau = 0.0;
     const double a = P.a;
-    double s2 = fmax(1.0 - u * u, 1e-12), s = sqrt(s2);
+    const double s2 = fmax(w, 1e-12), s = w >= 1e-12 ? sn : __builtin_sqrt(1e-12);
     double R = r * s, z = r * u;
     if (r > P.r_flow_max || R < 1e-3) return;
-    double zh = z / (P.h_r * R);
+    double zh = quot_ieee_(z, P.h_r * R);
     double vert = bhm::exp(-0.5 * zh * zh);
     if (vert < 1e-7) return;
     double lr = bhm::log(r);
     double ne = P.n0 * bhm::exp(-P.n_index * lr) * vert;
     if (P.turb_on) {
         if constexpr (RADIO == RADIO_SHEARED) ne *= (double)sheared_factor(P, r, R, z, phi, t);
-        else ne *= turb_factor(P, r, u, phi, t);
+        else ne *= turb_factor(P, r, R, u, sv, cv, t);
     }
     ne *= 1.0 - bhm::exp(-(r - P.rh) * (r - P.rh) / 0.25);
     if (ne < 1e-30) return;
     double Th = P.theta0 * bhm::exp(-P.theta_index * lr);
-    double B = sqrt(8.0 * PI * ne * C_MP * C_C * C_C / (6.0 * r * P.beta_p));
+    double B = sqrt_pos_(quot_ieee_(8.0 * PI * ne * C_MP * C_C * C_C, 6.0 * r * P.beta_p));
     double r2 = r * r, a2 = P.a2;
     double Sigma = r2 + a2 * u * u, Delta = r2 - 2.0 * r + a2;
     double A = (r2 + a2) * (r2 + a2) - a2 * Delta * s2;
-    double g_tt = -(1.0 - 2.0 * r / Sigma), g_tph = -2.0 * a * r * s2 / Sigma, g_phph = A * s2 / Sigma;
-    double omz = 2.0 * a * r / A;
+    const bhm::Recip iS = bhm::recip_(Sigma), iA = bhm::recip_(A);
+    double g_tt = -(1.0 - quot_(2.0 * r, iS)), g_tph = quot_(-2.0 * a * r * s2, iS), g_phph = quot_(A * s2, iS);
+    double omz = quot_(2.0 * a * r, iA);
     double Rk = fmax(R, P.r_isco);
-    double Om = P.flow_kep * (1.0 / (Rk * sqrt(Rk) + a));
-    double vmax = sqrt(Sigma * Delta / A) / sqrt(g_phph) * 0.999;
+    double Om = P.flow_kep * quot_(1.0, Rk * sqrt_pos_(Rk) + a);
+    double vmax = quot_(bhm::sqrt_nn_(quot_(Sigma * Delta, iA)), sqrt_pos_(g_phph)) * 0.999;
     Om = omz + fmax(-vmax, fmin(vmax, Om - omz));
     double norm = -(g_tt + 2.0 * g_tph * Om + g_phph * Om * Om);
     if (norm <= 0.0) return;
-    double ut = 1.0 / sqrt(norm);
+    double ut = quot_(1.0, sqrt_pos_(norm));
     double kdotu = ut * (1.0 - Om * lam);
     double nu_f = P.nu_obs * Ecam * kdotu;
-    double g = P.nu_obs / nu_f;
+    double g = quot_ieee_(P.nu_obs, nu_f);
     double u_ph = ut * (g_tph + g_phph * Om);
     double kb = lam - kdotu * u_ph;
     double bb = g_phph + u_ph * u_ph;
-    double cosb = kb / (kdotu * sqrt(bb));
-    double sinb = sqrt(fmax(1.0 - cosb * cosb, 1e-6));
-    double nuc = C_QE * B / (2.0 * PI * C_ME * C_C);
+    double cosb = quot_ieee_(kb, kdotu * sqrt_pos_(bb));
+    double sinb = sqrt_pos_(fmax(1.0 - cosb * cosb, 1e-6));
+    constexpr double NUC = 2.0 * PI * C_ME * C_C, CC2 = C_C * C_C;
+    double nuc = quot_const(C_QE * B, NUC, 1.0 / NUC);
     double nus = 2.0 / 9.0 * nuc * Th * Th * sinb;
-    double X = nu_f / nus;
+    double X = quot_ieee_(nu_f, nus);
     double x3 = bhm::cbrt(X);
-    double k2 = bhm::exp((double)table_lerp(P.k2, P.k2_n, P.k2_l0, P.k2_dl, (float)bhm::log(Th)));
-    double brk = sqrt(X) + 1.887748625363387 * sqrt(x3);
-    double j = ne * 1.4142135623730951 * PI * C_QE * C_QE * nus / (3.0 * k2 * C_C) * brk * brk * bhm::exp(-x3);
-    double Te = Th * C_ME * C_C * C_C / C_KB;
-    double hnu = C_H * nu_f / (C_KB * Te);
-    double Bnu = 2.0 * C_H * nu_f * nu_f * nu_f / (C_C * C_C) / bhm::expm1(hnu);
+    double k2 = bhm::exp((double)table_lerp(P.k2, P.k2_n, P.k2_l0, P.k2_dl, P.k2_inv_dl, (float)bhm::log(Th)));
+    double brk = bhm::sqrt_nn_(X) + 1.887748625363387 * bhm::sqrt_nn_(x3);
+    double j = quot_ieee_(ne * 1.4142135623730951 * PI * C_QE * C_QE * nus, 3.0 * k2 * C_C) * brk * brk * bhm::exp(-x3);
+    double Te = quot_const(Th * C_ME * C_C * C_C, C_KB, 1.0 / C_KB);
+    double hnu = quot_ieee_(C_H * nu_f, C_KB * Te);
+    double Bnu = quot_ieee_(quot_const(2.0 * C_H * nu_f * nu_f * nu_f, CC2, 1.0 / CC2), bhm::expm1(hnu));
     double alpha = j / Bnu;
     double dl = kdotu * Sigma * h * P.rg_cm;
     double tau = alpha * dl;
     *dtau = tau;
     *dI = g * g * g * Bnu * (-bhm::expm1(-tau));
+}
+
+// atan2(y, x) for y >= 0 and a vector of length about 1 (the angle between two directions): the
+// operations of bhm::atan2 with one quotient for both octant orders
+__device__ __forceinline__ double angle_pos(double y, double x) {
+    const double ax = fabs(x);
+    const bool steep = !(y <= ax);
+    double a = bhm::atan_unit(bhm::quot_(steep ? ax : y, steep ? y : ax));
+    a = steep ? bhm::PI_2 - a : a;
+    return x < 0.0 ? bhm::PI_ - a : a;
 }
 
 // blackholes/src/kerr.hpp:63-92 (+ trace.cuh:64 direction): initial state and constants
@@ -395,7 +487,8 @@ __device__ __forceinline__ double initial_step(const State& s) {
 struct RayState {
     RayConst c;
     State s;
-    double h, acc0, acc1, acc2, acc3, trans, psi, ppx, ppy, ppz;
+    double h, acc0, acc1, acc2, acc3, trans, psi;
+    double sn, ppx, ppy;   // radio: sin theta of the state and its direction's x and y (z is u = s.y2)
     int ncross, accepted, flow_steps, it, fate;
     bool done;
 };
@@ -405,7 +498,7 @@ template <int RADIO>
 __device__ __forceinline__ void ray_init(const TraceParams& P, double x, double yv, RayState& R) {
     camera_photon(P, x, yv, R.c, R.s);
     {
-        Rhs k = rhs(P, R.c, R.s.y0, R.s.y2);
+        Rhs k = rhs<true>(P, R.c, R.s.y0, R.s.y2);
         R.s.k1 = k.d1; R.s.k3 = k.d3; R.s.k4 = k.d4; R.s.k5 = k.d5;
     }
     R.h = initial_step(R.s);
@@ -413,54 +506,55 @@ __device__ __forceinline__ void ray_init(const TraceParams& P, double x, double 
     R.trans = 1.0;
     R.psi = 0.0;
     R.ncross = R.accepted = R.flow_steps = R.it = R.fate = 0;
-    R.ppx = R.ppy = R.ppz = 0.0;
+    R.sn = R.ppx = R.ppy = 0.0;
     if (RADIO) {
-        double sp = sqrt(fmax(1.0 - R.s.y2 * R.s.y2, 0.0)), sv, cv;
+        double sv, cv;
+        R.sn = bhm::sqrt_nn_(fmax(1.0 - R.s.y2 * R.s.y2, 0.0));
         bhm::sincos(R.s.y4, &sv, &cv);
-        R.ppx = sp * cv;
-        R.ppy = sp * sv;
-        R.ppz = R.s.y2;
+        R.ppx = R.sn * cv;
+        R.ppy = R.sn * sv;
     }
     R.done = P.max_steps <= 0;
 }
 
 // One iteration of trace.cuh:81-163 (one DP54 attempt); sets R.done when the ray stops.
-template <int RADIO>
+template <int RADIO, bool TIME>
 __device__ __forceinline__ void ray_step(const TraceParams& P, RayState& R) {
     const bool flow = RADIO && P.flow_on;
     State n;
     double hc = R.h;
     if (flow && R.s.y0 < P.r_flow_max) {
-        double sn = sqrt(fmax(1.0 - R.s.y2 * R.s.y2, 0.0));
-        double cap = P.step_frac * fmin(R.s.y0 / (fabs(R.s.y1) + 1e-30), fmax(sn, 0.05) / (fabs(R.s.y3) + 1e-30));
+        double cap = P.step_frac * fmin(bhm::quot_(R.s.y0, fabs(R.s.y1) + 1e-30),
+                                        bhm::quot_(fmax(R.sn, 0.05), fabs(R.s.y3) + 1e-30));
         hc = fmin(hc, cap);
     }
-    double err = dp54_step(P, R.c, R.s, hc, n);
+    const double err = dp54_step<TIME>(P, R.c, R.s, hc, n);
     ++R.it;
+    R.h = hc * step_factor(err);
     if (!(err <= 1.0)) {
-        R.h = hc * fmax(0.2, 0.9 * bhm::pow_m02(fmax(err, 1e-30)));
-        if (!(err == err)) R.h = hc * 0.1;
         if (R.it >= P.max_steps) R.done = true;
         return;
     }
     ++R.accepted;
+    double w = 0.0, sv = 0.0, cv = 1.0;
     if (RADIO) {
-        double sn = sqrt(fmax(1.0 - n.y2 * n.y2, 0.0)), sv, cv;
+        w = 1.0 - n.y2 * n.y2;
+        const double sn = bhm::sqrt_nn_(fmax(w, 0.0));
         bhm::sincos(n.y4, &sv, &cv);
-        double pnx = sn * cv, pny = sn * sv, pnz = n.y2;
-        double cx = R.ppy * pnz - R.ppz * pny, cy = R.ppz * pnx - R.ppx * pnz, cz = R.ppx * pny - R.ppy * pnx;
-        double cl = sqrt(cx * cx + cy * cy + cz * cz);
-        double dt = R.ppx * pnx + R.ppy * pny + R.ppz * pnz;
-        R.psi += bhm::atan2(cl, dt);
+        const double pnx = sn * cv, pny = sn * sv, pnz = n.y2, ppz = R.s.y2;
+        double cx = R.ppy * pnz - ppz * pny, cy = ppz * pnx - R.ppx * pnz, cz = R.ppx * pny - R.ppy * pnx;
+        double cl = bhm::sqrt_nn_(cx * cx + cy * cy + cz * cz);
+        double dt = R.ppx * pnx + R.ppy * pny + ppz * pnz;
+        R.psi += angle_pos(cl, dt);
         R.ppx = pnx;
         R.ppy = pny;
-        R.ppz = pnz;
+        R.sn = sn;
     }
     if ((R.s.y2 > 0.0) != (n.y2 > 0.0)) ++R.ncross;
     if (flow && n.y0 < P.r_flow_max) {
         double dI, dtau;
         ++R.flow_steps;
-        flow_step<RADIO>(P, n.y0, n.y2, n.y4, n.y5, R.c.lam, R.c.E, hc, &dI, &dtau);
+        flow_step<RADIO>(P, n.y0, n.y2, w, R.sn, n.y4, sv, cv, n.y5, R.c.lam, R.c.E, hc, &dI, &dtau);
         double cI = R.trans * dI;
         int ord = (int)(R.psi * (1.0 / PI));
         R.acc0 += cI;
@@ -477,7 +571,6 @@ __device__ __forceinline__ void ray_step(const TraceParams& P, RayState& R) {
     }
     R.s = n;
     project_radial(P, R.c, R.s);
-    R.h = hc * fmin(5.0, fmax(0.2, 0.9 * bhm::pow_m02(fmax(err, 1e-30))));
     if (R.s.y0 < P.r_stop) {
         R.fate = -1;
         R.done = true;
@@ -557,11 +650,11 @@ __device__ __forceinline__ void ray_result(const TraceParams& P, const RayState&
 }
 
 // blackholes/src/trace.cuh:62-165 (disk branch out of scope, procedural sky), FP64 intensity.
-template <int RADIO>
+template <int RADIO, bool TIME>
 __device__ __forceinline__ void trace_ray_fp64(const TraceParams& P, double x, double yv, RayResult& out) {
     RayState R;
     ray_init<RADIO>(P, x, yv, R);
-    while (!R.done) ray_step<RADIO>(P, R);
+    while (!R.done) ray_step<RADIO, TIME>(P, R);
     ray_result(P, R, out);
 }
 
@@ -577,19 +670,16 @@ __device__ __forceinline__ int vacuum_fate(const TraceParams& P, const double* p
     c.alam = P.a * c.lam;
     State s, n;
     s.y0 = ph[3]; s.y1 = ph[4]; s.y2 = ph[5]; s.y3 = ph[6]; s.y4 = ph[7]; s.y5 = ph[8];
-    Rhs k = rhs(P, c, s.y0, s.y2);
+    Rhs k = rhs<false>(P, c, s.y0, s.y2);   // the fate reads no coordinate time
     s.k1 = k.d1; s.k3 = k.d3; s.k4 = k.d4; s.k5 = k.d5;
     double h = initial_step(s);
     const double rcap = P.rh * 1.0001 + 1e-3;
     for (int it = 0; it < max_steps; ++it) {
-        double err = dp54_step(P, c, s, h, n);
-        if (err > 1.0) {
-            h *= fmax(0.2, 0.9 * bhm::pow_m02(err));
-            continue;
-        }
+        const double err = dp54_step<false>(P, c, s, h, n);
+        h *= step_factor(err);
+        if (err > 1.0) continue;
         s = n;
         project_radial(P, c, s);
-        h *= fmin(5.0, fmax(0.2, 0.9 * bhm::pow_m02(fmax(err, 1e-30))));
         if (s.y0 < rcap) return -1;
         if (s.y0 > r_escape && s.y1 > 0.0) return 1;
     }

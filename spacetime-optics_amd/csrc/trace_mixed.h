@@ -549,7 +549,6 @@ struct MixedParams {
     double tol_mid;   // tolerance between r_tol and r_far
     double tol_far;   // tolerance of the far-field steps
     double inv_tol_t; // 1 / (absolute bound on a step's coordinate-time error); 0: no bound
-    int need_t;       // integrate the coordinate time t (emission read at its time, or ray records)
     double tol_relax; // emission-region tolerance of a ray after relax_after attempts
     double relax_cap; // and the factor on its transfer step cap
     int relax_after;
@@ -600,7 +599,7 @@ __device__ __forceinline__ void ray_init_m(const TraceParams& P, const MixedPara
 // One attempt of trace.cuh:81-163 under the mixed policy. TCACHE keeps the ray's turbulence cell
 // in its state across attempts (the persistent engine); without it every flow sample loads its
 // corners (the frame kernel, already at the register limit, would spill the cache in its loop).
-template <int RADIO, bool TCACHE = true>
+template <int RADIO, bool TIME, bool TCACHE = true>
 __device__ __forceinline__ void ray_step_m(const TraceParams& P, const MixedParams& M, RayStateM& R) {
     const bool flow = RADIO && P.flow_on;
     State n;
@@ -626,9 +625,7 @@ __device__ __forceinline__ void ray_step_m(const TraceParams& P, const MixedPara
         // relax_after attempts (an orbit near the photon sphere)
         const double inv_tol = R.s.y0 < M.r_tol ? (R.it >= M.relax_after ? M.inv_tol_relax : M.inv_tol)
                                                 : (R.s.y0 < M.r_far ? M.inv_tol_mid : M.inv_tol_far);
-        // coordinate time only where something reads it (wave-uniform: the frame's policy)
-        err = M.need_t ? dp54<double, true>(cd, R.s, hc, inv_tol, M.inv_tol_t, n)
-                       : dp54<double, false>(cd, R.s, hc, inv_tol, M.inv_tol_t, n);
+        err = dp54<double, TIME>(cd, R.s, hc, inv_tol, M.inv_tol_t, n);
         ++R.fp64_attempts;
     }
     R.k1_f32 = R.s.y0 >= M.r_f32;
@@ -754,12 +751,12 @@ __device__ __forceinline__ int ray_result_m(const TraceParams& P, const RayState
 
 /* blackholes/src/trace.cuh:62-165 under the mixed policy. Returns the number of FP64 step attempts
    (near field and flow); out.steps counts all attempts. */
-template <int RADIO>
+template <int RADIO, bool TIME>
 __device__ __forceinline__ int trace_ray_mixed(const TraceParams& P, const MixedParams& M, double x, double yv,
                                                RayResult& out) {
     RayStateM R;
     ray_init_m<RADIO>(P, M, x, yv, R);
-    while (!R.done) ray_step_m<RADIO, false>(P, M, R);
+    while (!R.done) ray_step_m<RADIO, TIME, false>(P, M, R);
     return ray_result_m(P, R, out);
 }
 

@@ -140,11 +140,13 @@ __device__ __forceinline__ float sh_tex(const float* __restrict__ T, int nx, int
     const int x1 = x0 + 1 == nx ? 0 : x0 + 1;
     const int y0 = min(max(iy, 0), ny - 1), y1 = min(max(iy + 1, 0), ny - 1);
     const int z0 = min(max(iz, 0), nz - 1), z1 = min(max(iz + 1, 0), nz - 1);
-    const size_t sy = (size_t)nx, sz = (size_t)nx * ny;
-    const float v000 = T[z0 * sz + y0 * sy + x0], v100 = T[z0 * sz + y0 * sy + x1];
-    const float v010 = T[z0 * sz + y1 * sy + x0], v110 = T[z0 * sz + y1 * sy + x1];
-    const float v001 = T[z1 * sz + y0 * sy + x0], v101 = T[z1 * sz + y0 * sy + x1];
-    const float v011 = T[z1 * sz + y1 * sy + x0], v111 = T[z1 * sz + y1 * sy + x1];
+    // 32-bit offsets inside a slice: bh_create keeps all slices together at most 2^31 cells
+    const unsigned int sy = (unsigned int)nx, sz = sy * (unsigned int)ny;
+    const unsigned int r00 = z0 * sz + y0 * sy, r10 = z0 * sz + y1 * sy, r01 = z1 * sz + y0 * sy, r11 = z1 * sz + y1 * sy;
+    const float v000 = T[r00 + x0], v100 = T[r00 + x1];
+    const float v010 = T[r10 + x0], v110 = T[r10 + x1];
+    const float v001 = T[r01 + x0], v101 = T[r01 + x1];
+    const float v011 = T[r11 + x0], v111 = T[r11 + x1];
     const float bx = 1.f - ax, by = 1.f - ay, bz = 1.f - az;
     return bz * (by * (bx * v000 + ax * v100) + ay * (bx * v010 + ax * v110)) +
            az * (by * (bx * v001 + ax * v101) + ay * (bx * v011 + ax * v111));
@@ -155,11 +157,13 @@ __device__ __forceinline__ float sh_tex(const float* __restrict__ T, int nx, int
 __device__ __forceinline__ float sheared_factor(const TraceParams& P, double r, double R, double z, double phi,
                                                 double t) {
     const ShearedView& T = *P.ts;
-    const float u = (float)((bhm::log(R) - T.lr0) / (T.lr1 - T.lr0));
+    // quotients by the slices' constants from their reciprocals (bhm::quot_)
+    const float u = (float)bhm::quot_(bhm::log(R) - T.lr0, bhm::Recip{T.lr1 - T.lr0, T.inv_lr});
     const float v = (float)(phi * (0.5 / PI));
-    const float w = (float)(0.5 + 0.5 * (z / R) / T.zmax);
-    const double tref = T.cam_t - (T.cam_r - r + 2.0 * bhm::log(T.cam_r / r));
-    float s = (float)((t - tref) - T.d0) / T.dd;
+    const float w = (float)(0.5 + bhm::quot_(0.5 * bhm::quot_(z, R), bhm::Recip{T.zmax, T.inv_zmax}));
+    const double tref = T.cam_t - (T.cam_r - r + 2.0 * bhm::log(bhm::quot_(T.cam_r, r)));
+    const float sn = (float)((t - tref) - T.d0), sq = sn * T.inv_dd;
+    float s = fmaf(fmaf(-T.dd, sq, sn), T.inv_dd, sq);
     s = fminf(fmaxf(s, 0.f), (float)(T.nt - 1) - 1e-4f);
     const int k = (int)s;
     const float f = s - (float)k;
