@@ -18,7 +18,7 @@
      r_tol; the rest of the flow is traced as vacuum with tol_mid = tol_far / 10 (or, with
      full_flow, the whole flow as the FP64 tracer with tol_mid = 1e-6).
    - Stage precision: FP64 stages evaluated with fused multiply-adds and Newton-refined FP64
-     reciprocals; optionally (r >= r_f32) DP5(4) stages in FP32 with hardware reciprocals, the
+     reciprocals (in vacuum by dp54_n, a form of the method with fewer operations); optionally (r >= r_f32) DP5(4) stages in FP32 with hardware reciprocals, the
      state accumulated in FP64, the error norm, step controller and radial-constraint projection
      in FP64. The coordinate time is integrated only where something reads it (time-dependent
      turbulence, a t bound, ray records). The projection r' = +-sqrt(R(r)) after every accepted
@@ -246,6 +246,156 @@ __device__ __forceinline__ RConst<R> make_const(const TraceParams& P, const RayC
     k.lam2 = (R)c.lam2;
     k.alam = (R)c.alam;
     k.s2min = sizeof(R) == 4 ? (R)1e-30 : (R)1e-300;
+    return k;
+}
+
+// Constants of a ray's motion in the form the right-hand side uses
+struct NConst {
+    double a, a2, lam;
+    double q, K;     // r'' = 2 r P - (r - 1) K,  P = r^2 + q,  q = a^2 - a lam
+    double a2m1;     // Delta = (r - 1)^2 + a^2 - 1
+    double B, m2a2;  // u'' = u (B - 2 a^2 u^2),  B = a^2 - eta - lam^2
+    double aal, m2a; // numerator of phi' over Delta: a (a lam - 2 r)
+};
+
+// blackholes/src/kerr.hpp:103-116 with the two quotients of phi' over one reciprocal:
+//   phi' = a - a P / Delta - lam / s2 = (a (a lam - 2 r) s2 - lam Delta) / (Delta s2).
+// r'' and Delta are formed from r - 1, which is exact where it matters: near the horizon of a fast
+// spinning hole both are small differences (multiplied out, r'' loses a digit at r = 1.07, where the
+// rays of a = 0.998 orbit).
+// s2 is kept above 1e-30 so a stage past the pole gives a huge finite phi' and its step is rejected.
+// Without TIME the coordinate-time derivative d5 is left at zero.
+template <bool TIME>
+__device__ __forceinline__ Rhs<double> rhs_n(const NConst& c, double r, double u) {
+    const double u2 = u * u, r1 = r - 1.0;
+    const double P = r * r + c.q, Delta = r1 * r1 + c.a2m1;
+    const double s2 = fmax(1.0 - u2, 1e-30);
+    const double inv = rcpd(Delta * s2);
+    Rhs<double> o;
+    o.d1 = (r + r) * P - r1 * c.K;
+    o.d3 = u * (c.m2a2 * u2 + c.B);
+    const double num = (c.m2a * r + c.aal) * s2;
+    o.d4 = (num - c.lam * Delta) * inv;
+    o.d5 = TIME ? -((r * r + c.a2) * P * (inv * s2) + c.a * (c.lam - c.a * s2)) : 0.0;
+    return o;
+}
+
+/* Dormand-Prince 5(4) for the second-order pairs (r, r') and (u, u'): r'' and u'' do not depend on r'
+   and u', so the stage velocities need not be formed. Substituting q_i = v + h sum_j a_ij k_j into the
+   position sums leaves y_i = y + c_i h v + h^2 sum_k (A^2)_ik k_k, and likewise for the solution
+   (b A) and the error estimate (e A, whose weights on v sum to zero, so it no longer cancels there):
+   the same method in 60 multiply-adds per pair instead of 104. Coefficients n_ik = (A^2)_ik, f_k =
+   (b A)_k = b_k (1 - c_k), g_k = (e A)_k. The stage values of u are rounded once: near the spin axis
+   1 - u^2 carries that rounding, and a second one added 40 % to the attempts of rays on the axis. */
+constexpr double c3 = 3.0 / 10, c4 = 4.0 / 5, c5 = 8.0 / 9;
+constexpr double n31 = 9.0 / 200, n41 = -12.0 / 25, n42 = 4.0 / 5;
+constexpr double n51 = -12248.0 / 6561, n52 = 7208.0 / 2187, n53 = -6784.0 / 6561;
+constexpr double n61 = -533.0 / 264, n62 = 91.0 / 22, n63 = -56.0 / 33, n64 = 7.0 / 88;
+constexpr double f1 = 35.0 / 384, f3 = 50.0 / 159, f4 = 25.0 / 192, f5 = -243.0 / 6784;
+constexpr double g1 = 611.0 / 230400, g3 = -514.0 / 83475, g4 = 391.0 / 38400, g5 = -4617.0 / 1356800,
+                 g6 = -11.0 / 3360;
+
+/* One step in this form, FP64 throughout: the vacuum tracer's step. It is bound by VALU issue: 253
+   instructions for 328 and 6 reciprocals for 13 (20 cycles each, against 4); the 640^2 photon-ring zoom
+   at a = 0.94 (the kernel alone) 13.2 -> 10.7 ms, the 768^2 one with its copy 17.2 -> 14.4 ms.
+   The radio tracer keeps dp54: its emission is summed over the step sequence, which on rays past the
+   spin axis follows phi's error estimate down to the rounding of 1 - u^2, so another rounding moves
+   samples of the n = 1 image across an order boundary in a few pixels of every million (1e-3 to 2e-2
+   of the mean pixel). A vacuum ray's escape direction does not depend on where its steps fall. */
+template <bool TIME>
+__device__ __forceinline__ double dp54_n(const NConst& c, const State& s, double h, double inv_tol, double inv_tol_t,
+                                         State& o) {
+    using namespace bhd;
+    const double hh = h * h;
+    const double y0 = s.y0, y2 = s.y2, w0 = h * s.y1, w2 = h * s.y3;
+    double p = s.k1, q = s.k3;   // this stage's r'' and u''
+    double S3_0 = n31 * p, S4_0 = n41 * p, S5_0 = n51 * p, S6_0 = n61 * p;
+    double S3_2 = n31 * q, S4_2 = n41 * q, S5_2 = n51 * q, S6_2 = n61 * q;
+    double F0 = f1 * p, O1 = b1 * p, G0 = g1 * p, E1 = e1 * p;
+    double F2 = f1 * q, O3 = b1 * q, G2 = g1 * q, E3 = e1 * q;
+    double O4 = b1 * s.k4, E4 = e1 * s.k4;
+    double O5 = TIME ? b1 * s.k5 : 0.0, E5 = TIME ? e1 * s.k5 : 0.0;
+    // stage 2 (its phi' and t' carry no weight)
+    Rhs<double> k = rhs_n<false>(c, y0 + a21 * w0, y2 + a21 * w2);
+    p = k.d1; q = k.d3;
+    S4_0 += n42 * p; S5_0 += n52 * p; S6_0 += n62 * p;
+    S4_2 += n42 * q; S5_2 += n52 * q; S6_2 += n62 * q;
+    // stage 3
+    double t0 = y0 + c3 * w0;
+    k = rhs_n<TIME>(c, t0 + hh * S3_0, y2 + (c3 * w2 + hh * S3_2));
+    p = k.d1; q = k.d3;
+    S5_0 += n53 * p; S6_0 += n63 * p; F0 += f3 * p; O1 += b3 * p; G0 += g3 * p; E1 += e3 * p;
+    S5_2 += n53 * q; S6_2 += n63 * q; F2 += f3 * q; O3 += b3 * q; G2 += g3 * q; E3 += e3 * q;
+    O4 += b3 * k.d4; E4 += e3 * k.d4;
+    if (TIME) { O5 += b3 * k.d5; E5 += e3 * k.d5; }
+    // stage 4
+    t0 = y0 + c4 * w0;
+    k = rhs_n<TIME>(c, t0 + hh * S4_0, y2 + (c4 * w2 + hh * S4_2));
+    p = k.d1; q = k.d3;
+    S6_0 += n64 * p; F0 += f4 * p; O1 += b4 * p; G0 += g4 * p; E1 += e4 * p;
+    S6_2 += n64 * q; F2 += f4 * q; O3 += b4 * q; G2 += g4 * q; E3 += e4 * q;
+    O4 += b4 * k.d4; E4 += e4 * k.d4;
+    if (TIME) { O5 += b4 * k.d5; E5 += e4 * k.d5; }
+    // stage 5
+    t0 = y0 + c5 * w0;
+    k = rhs_n<TIME>(c, t0 + hh * S5_0, y2 + (c5 * w2 + hh * S5_2));
+    p = k.d1; q = k.d3;
+    F0 += f5 * p; O1 += b5 * p; G0 += g5 * p; E1 += e5 * p;
+    F2 += f5 * q; O3 += b5 * q; G2 += g5 * q; E3 += e5 * q;
+    O4 += b5 * k.d4; E4 += e5 * k.d4;
+    if (TIME) { O5 += b5 * k.d5; E5 += e5 * k.d5; }
+    // stage 6
+    t0 = y0 + w0;
+    k = rhs_n<TIME>(c, t0 + hh * S6_0, y2 + (w2 + hh * S6_2));
+    p = k.d1; q = k.d3;
+    O1 += b6 * p; G0 += g6 * p; E1 += e6 * p;
+    O3 += b6 * q; G2 += g6 * q; E3 += e6 * q;
+    O4 += b6 * k.d4; E4 += e6 * k.d4;
+    if (TIME) { O5 += b6 * k.d5; E5 += e6 * k.d5; }
+    // 5th-order solution and its derivative (FSAL)
+    o.y0 = s.y0 + (w0 + hh * F0);
+    o.y1 = s.y1 + h * O1;
+    o.y2 = s.y2 + (w2 + hh * F2);
+    o.y3 = s.y3 + h * O3;
+    o.y4 = s.y4 + h * O4;
+    o.y5 = TIME ? s.y5 + h * O5 : s.y5;
+    k = rhs_n<TIME>(c, o.y0, o.y2);
+    o.k1 = k.d1;
+    o.k3 = k.d3;
+    o.k4 = k.d4;
+    o.k5 = TIME ? k.d5 : s.k5;
+    E1 += e7 * k.d1; E3 += e7 * k.d3; E4 += e7 * k.d4;
+    if (TIME) E5 += e7 * k.d5;
+    // scaled max-norm over r, r', u, u', phi (kerr.hpp:145-155) in FP64. Each of its scales is tol
+    // times a factor a_i (a = 1 for u, 4 for phi), so the norm is max_i(|h E_i| / a_i) / tol: one
+    // Newton-refined FP64 reciprocal for the three state-dependent factors, and 1 / tol precomputed
+    const double a0 = 1e-6 + fmax(fabs(s.y0), fabs(o.y0));
+    const double a1 = 1e-6 + fmax(fmax(fabs(s.y1), fabs(o.y1)), s.y0 * s.y0);
+    const double a3 = fmax(1.0, fmax(fabs(s.y3), fabs(o.y3)));
+    const double a01 = a0 * a1;
+    double m = fmax(fabs(h * G0) * (a1 * a3), fabs(E1) * (a0 * a3));
+    m = fmax(m, fabs(E3) * a01) * rcpd(a01 * a3);
+    m = fmax(m, fabs(h * G2));
+    m = fmax(m, fabs(E4) * 0.25);
+    m *= fabs(h) * inv_tol;
+    // coordinate time (not in the reference's norm): an absolute bound per step where the turbulence
+    // depends on the emission time (inv_tol_t = 1 / bound, 0 when it does not)
+    if (TIME) m = fmax(m, fabs(h * E5) * inv_tol_t);
+    return m;
+}
+
+__device__ __forceinline__ NConst make_nconst(const TraceParams& P, const RayConst& c) {
+    NConst k;
+    k.a = P.a;
+    k.a2 = P.a2;
+    k.lam = c.lam;
+    k.q = P.a2 - c.alam;
+    k.K = c.K;
+    k.a2m1 = fma(P.a, P.a, -1.0);
+    k.B = P.a2 - c.eta - c.lam2;
+    k.m2a2 = -2.0 * P.a2;
+    k.aal = P.a * c.alam;
+    k.m2a = -2.0 * P.a;
     return k;
 }
 
@@ -625,7 +775,8 @@ __device__ __forceinline__ void ray_step_m(const TraceParams& P, const MixedPara
         // relax_after attempts (an orbit near the photon sphere)
         const double inv_tol = R.s.y0 < M.r_tol ? (R.it >= M.relax_after ? M.inv_tol_relax : M.inv_tol)
                                                 : (R.s.y0 < M.r_far ? M.inv_tol_mid : M.inv_tol_far);
-        err = dp54<double, TIME>(cd, R.s, hc, inv_tol, M.inv_tol_t, n);
+        if constexpr (RADIO == bhd::RADIO_OFF) err = dp54_n<TIME>(make_nconst(P, R.c), R.s, hc, inv_tol, M.inv_tol_t, n);
+        else err = dp54<double, TIME>(cd, R.s, hc, inv_tol, M.inv_tol_t, n);
         ++R.fp64_attempts;
     }
     R.k1_f32 = R.s.y0 >= M.r_f32;

@@ -5,7 +5,10 @@
   bit for bit.
 - The FP64 step at tolerances where its scaled error leaves the ordinary range (every step accepted at
   the largest growth, every step rejected, errors that overflow) against the oracle, bit for bit.
-- The FP64 tracer at cameras whose steps pass near the pole and the horizon, likewise."""
+- The FP64 tracer at cameras whose steps pass near the pole and the horizon, likewise.
+- The mixed vacuum step (its own form of the method) over spins, on and beside the spin axis, where the
+  stage values of u decide the attempts: the FP64 tracer's fates, fewer attempts, and its escape angles
+  to the far field's tolerance."""
 import numpy as np
 import pytest
 
@@ -59,5 +62,25 @@ def test_pole_and_horizon(oracle_bhm, spin, incl):
         gpu = t.trace_tile(cfg["F"], 20, 21, 23, 22)
         _, ref, _ = oracle_bhm.trace_pixels(cfg["OS"], cfg["OF"], *pixel_grid(23, 22, 20, 21))
         assert_rays_equal(gpu, ref, sets)
+    finally:
+        t.close()
+
+
+@pytest.mark.parametrize("spin", [1e-6, 0.5, 0.9999])
+@pytest.mark.parametrize("cx", [0.0, 1e-3, 3.0])   # M from the axis to the image's centre column
+def test_mixed_vacuum_step(spin, cx):
+    sets = f"bh.spin={spin!r}"
+    S = bh.build_scene(shot("c1_vacuum_256.ini"), sets)[0]
+    F = bh.make_frame(S.a, 1000.0, 0.3, fov=16.0, off_x=cx, W=45, H=61)
+    t = bh.Tracer(S)
+    try:
+        ref = t.trace_tile(F, 0, 0, 45, 61, t.opts())
+        got = t.trace_tile(F, 0, 0, 45, 61, t.opts(precision=bh.PREC_MIXED))
+        same = ref["fate"] == got["fate"]
+        assert same.mean() > 0.998   # a ray on the critical curve may fall either way
+        assert got["steps"].sum() < 0.6 * ref["steps"].sum()
+        esc = same & (ref["fate"] == 1) & (ref["ncross"] <= 1)
+        d = np.abs(np.cos(ref["th_inf"][esc]) - np.cos(got["th_inf"][esc]))
+        assert esc.sum() > 500 and np.median(d) < 2e-5
     finally:
         t.close()
