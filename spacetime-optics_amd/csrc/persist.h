@@ -264,22 +264,23 @@ __device__ __forceinline__ void persist_body(const Work& Wk, unsigned int* __res
         CFrame* cfr = (CFrame*)frames;
         const TraceParams& P = *(const TraceParams*)&cfr[cf].P;
         const bhm32::MixedParams& M = *(const bhm32::MixedParams*)&cfr[cf].M;
-        for (int k = 0; k < interval; ++k) {
-            if (active) {
-                if (!R.done) T::step(P, M, R);
-                if (R.done) {
-                    RayResult r;
-                    const int f64 = T::result(P, R, r);
-                    Wk.finish(cf, ent, r);
-                    s_flux[tid] += r.I[0];
-                    s_stat[0][tid] += (unsigned long long)r.steps;
-                    s_stat[1][tid] += (unsigned long long)r.accepted;
-                    s_stat[2][tid] += (unsigned long long)r.flow_steps;
-                    s_stat[3][tid] += r.fate == 0 ? 1ull : 0ull;
-                    s_stat[4][tid] += (unsigned long long)f64;
-                    active = false;
-                }
-            }
+        for (int k = 0; k < interval; ++k)
+            if (active && !R.done) T::step(P, M, R);
+        // Finished rays are written here, all of the interval's together: inside the loop nearly every
+        // step of a 64-ray wave would end some ray and hold the others up for its output (LDS sums, a
+        // store, the escape direction). Mixed radio, 8 frames of 4.0 M rays: 11.6 -> 11.0 ms; 1024^2 with
+        // the surrogate: 3.02 -> 2.94.
+        if (active && R.done) {
+            RayResult r;
+            const int f64 = T::result(P, R, r);
+            Wk.finish(cf, ent, r);
+            s_flux[tid] += r.I[0];
+            s_stat[0][tid] += (unsigned long long)r.steps;
+            s_stat[1][tid] += (unsigned long long)r.accepted;
+            s_stat[2][tid] += (unsigned long long)r.flow_steps;
+            s_stat[3][tid] += r.fate == 0 ? 1ull : 0ull;
+            s_stat[4][tid] += (unsigned long long)f64;
+            active = false;
         }
     }
     if (prio_age > 0) __builtin_amdgcn_s_setprio(0);

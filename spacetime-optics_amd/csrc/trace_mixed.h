@@ -781,8 +781,10 @@ __device__ __forceinline__ void ray_step_m(const TraceParams& P, const MixedPara
     }
     R.k1_f32 = R.s.y0 >= M.r_f32;
     ++R.it;
+    // one power for both outcomes (a rejected step's factor is below 0.9), so lanes that disagree share it
+    double fac = fmin(5.0, fmax(0.2, 0.9 * pow_m02_d(err)));
     if (!(err <= 1.0)) {
-        R.h = hc * fmax(0.2, 0.9 * pow_m02_d(err));
+        R.h = hc * fac;
         if (!(err == err)) R.h = hc * 0.1;
         if (R.it >= P.max_steps) R.done = true;
         return;
@@ -853,7 +855,6 @@ __device__ __forceinline__ void ray_step_m(const TraceParams& P, const MixedPara
     const double r0 = R.s.y0;
     R.s = n;
     project_radial_m(P, R.c, R.s);
-    double fac = fmin(5.0, fmax(0.2, 0.9 * pow_m02_d(err)));
     // Outside the scene-tolerance region the step follows the radial scale: there the Mino-time
     // step that meets the tolerance goes as 1/r (dr/dlambda ~ r^2), and the error-only controller
     // lags one step behind it - on the way out every other step was rejected.
