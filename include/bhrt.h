@@ -257,9 +257,12 @@ typedef struct bh_batch_cfg {
                            which grows with the number of orbits near the critical curve); 0 -> the
                            default */
     int prio_age;       /* > 0: a wave holding a ray that has taken prio_age steps raises its issue
-                           priority; < 0: off; 0 -> the default. A NULL cfg (and no autotuned one)
-                           means, for the mixed tracer, 128 / 4 / 32 / 32 / graph / 3 / critical order /
-                           256, for the FP64 tracer 256 / 8 / 64 / 48 / graph / 3 / row order / 256. */
+                           priority; < 0: off; 0 -> the default. The defaults (a NULL cfg, no autotuned one)
+                           follow the launch's number of rays: from workgroups of one wave, one wave or fewer
+                           per SIMD, for launches that hold all their rays at once, to 256 threads and three
+                           waves per SIMD; rows order for the largest FP64 launches and those without
+                           generations, else critical; interval 64, refill_min 32 (mixed) / 48 (FP64), graph,
+                           waves 3, prio_age 256. */
 } bh_batch_cfg;
 
 /* Traces every frame of `frames`; px_out (nullable) receives the frames one after the other,

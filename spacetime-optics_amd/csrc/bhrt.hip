@@ -118,6 +118,31 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(2))) void
     }
 }
 
+// The frame kernel's block partials of the flux from samples already traced (samp[pixel * spp + sample]):
+// the same workgroups, lanes and order of additions, so the total has the same bits.
+__global__ __launch_bounds__(BLOCK) void k_flux_blocks(const double4* __restrict__ samp, int w, int h, int spp,
+                                                       BlockOut* __restrict__ blk, int per_xcd) {
+    const int tiles_x = (w + TILE - 1) / TILE, tiles_y = (h + TILE - 1) / TILE;
+    const int tile = xcd_tile(blockIdx.x, tiles_x * tiles_y, per_xcd);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    double flux = 0.0;
+    if (tile >= 0) {
+        const int tx = (tile % tiles_x) * TILE + (wave & 1) * 8 + (lane & 7);
+        const int ty = (tile / tiles_x) * TILE + (wave >> 1) * 8 + (lane >> 3);
+        if (tx < w && ty < h)
+            for (int s = 0; s < spp; ++s) flux += samp[((size_t)ty * w + tx) * spp + s].x;
+    }
+    __shared__ double s_flux[BLOCK / 64];
+    flux = wave_sum(flux);
+    if (lane == 0) s_flux[wave] = flux;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        BlockOut b{};
+        b.flux = ((s_flux[0] + s_flux[1]) + s_flux[2]) + s_flux[3];
+        blk[blockIdx.x] = b;
+    }
+}
+
 // Sums nb block partials in index order (one workgroup; each lane a strided slice, then a fixed tree).
 __global__ __launch_bounds__(256) void k_reduce(const BlockOut* __restrict__ blk, int nb, BlockOut* __restrict__ tot) {
     __shared__ double s_f[256];
@@ -1017,30 +1042,54 @@ int persist_grid(const bh_ctx* c, const void* k, int block, int grid_per_cu) {
 constexpr size_t PLAIN_SPP_SAMPLE_BUDGET = size_t(1) << 30;   // bytes of per-sample storage of bh_render, spp > 1
 constexpr long long BATCH_MAX_PIXELS = 1ll << 30;   // per frame: keeps the 32-bit queue counters from wrapping
 
-// Defaults: the autotuner's choices on the 1024^2 230 GHz frame (MI355X). The mixed tracer's launch is
-// bound by its longest rays (over 10x the mean step count): queueing them first (critical order) and
-// raising the priority of waves that hold rays older than 256 steps cut its frame time by a quarter;
-// four 128-lane workgroups per CU (2 waves per SIMD of the 3 its registers allow) keep each wave's
-// share of the SIMD, and so the latency of the longest rays, high.
-// The FP64 tracer (at most 3x the mean) is throughput-bound: 3 waves per SIMD (all the CU holds at
-// 164 registers), longer retire intervals, row order.
-bh_batch_cfg batch_defaults(int prec) {
+/* Defaults of a persistent launch of `entries` rays (all frames). w = waves of rays per compute unit; a
+   CU holds 12 waves of these kernels (3 per SIMD). Measured on frames of 32^2 to 2048^2 (MI355X, ms of
+   the launch):
+   - A SIMD issues one wave's instructions at half its rate, so 2 waves fill it and a third covers the
+     stalls; but the longest rays set the end of a launch, and each of their instructions waits for the
+     SIMD's other waves. Few rays are therefore spread thinly - and evenly: the waves that find no ray
+     exit, and with 3 resident waves per SIMD which SIMD they leave idle is chance. 256^2 vacuum, FP64:
+     4.2 with 12 waves per CU, 2.8 with 3; 512^2 radio, FP64: 8.7 with 12, 6.0 with 8; 1024^2: 18.3 with
+     12. Mixed radio, 256^2: 2.16 with 8, 2.01 with 4; 1400^2: 4.82 with 8, 4.17 with 12; zoom 768^2:
+     13.5 with 8, 11.9 with 12 (every ray is long: throughput, from 8 waves of rays per CU on).
+   - Longest rays first (critical order) where several generations of rays share the launch, but not so
+     many that its tail no longer counts: FP64 radio 384^2 6.0 -> 4.8, 768^2 11.3 -> 11.1, 1024^2 18.3
+     -> 18.9, 1500^2 37.6 -> 39.9. A launch that holds all its rays at once needs no sort. The mixed
+     tracer's rays differ by over 10x in length: always.
+   - Workgroups of one wave where they are few, so that the dispatcher can place each on its own. */
+bh_batch_cfg batch_defaults(const bh_ctx* c, int prec, const Variant& v, long long entries) {
     bh_batch_cfg d{};
-    const bool mixed = prec == BH_PREC_MIXED;
-    d.block = mixed ? 128 : 256;
-    d.grid_per_cu = mixed ? 4 : 8;
-    d.interval = mixed ? 32 : 64;
-    d.refill_min = mixed ? 32 : 48;
+    const double w = (double)entries / 64.0 / c->n_cu;
     d.use_graph = 1;
     d.waves = 3;
-    d.order = mixed ? BH_ORDER_CRITICAL : BH_ORDER_ROWS;
-    d.prio_age = 256;
+    d.interval = 64;
+    d.prio_age = prec == BH_PREC_MIXED ? 128 : 256;
+    if (prec == BH_PREC_MIXED) {
+        const bool vacuum = v.radio == bhd::RADIO_OFF;
+        const int per_cu = w <= (vacuum ? 8.0 : 20.0) ? 4 : (!vacuum && w <= 48.0 ? 8 : 12);
+        d.block = per_cu == 4 && !vacuum ? 64 : 256;
+        d.grid_per_cu = per_cu * 64 / d.block;
+        d.refill_min = 32;
+        d.order = BH_ORDER_CRITICAL;
+    } else {
+        d.block = w <= 20.0 ? 64 : 256;
+        d.grid_per_cu = w <= 5.0 ? 3 : (w <= 7.0 ? 4 : (w <= 20.0 ? 8 : 3));
+        d.refill_min = 48;
+        d.order = w > 5.0 && w <= 48.0 ? BH_ORDER_CRITICAL : BH_ORDER_ROWS;
+    }
     return d;
 }
 
+// Queue entries of a batch: the pixels of whole 8 x 8 tiles (frame sizes are checked later)
+long long batch_entries(const bh_batch_frame* frames, int n) {
+    long long e = 0;
+    for (int i = 0; i < n; ++i)
+        e += (long long)((std::max(frames[i].frame.W, 0) + 7ll) / 8) * ((std::max(frames[i].frame.H, 0) + 7ll) / 8) * 64;
+    return e;
+}
+
 // Replaces the 0 ("default") fields of a launch configuration and checks the ranges.
-int resolve_cfg(bh_ctx* c, int prec, bh_batch_cfg* g) {
-    const bh_batch_cfg d = batch_defaults(prec);
+int resolve_cfg(bh_ctx* c, const bh_batch_cfg& d, bh_batch_cfg* g) {
     if (g->block == 0) g->block = d.block;
     if (g->grid_per_cu == 0) g->grid_per_cu = d.grid_per_cu;
     if (g->interval == 0) g->interval = d.interval;
@@ -1083,8 +1132,12 @@ int launch_batch(bh_ctx* c, const bh_batch_frame* frames, int n, const bh_trace_
     if (opts) o = *opts;
     int rc = check_opts(c, o);
     if (rc) return rc;
-    bh_batch_cfg cfg = cfg_in ? *cfg_in : (c->tuned_ok[o.precision] ? c->tuned[o.precision] : batch_defaults(o.precision));
-    rc = resolve_cfg(c, o.precision, &cfg);
+    // one kernel for all frames: it integrates the coordinate time if any of them reads it
+    Variant v = variant_of(c, frames[0].scene, o);
+    for (int i = 1; i < n; ++i) v.time = v.time || variant_of(c, frames[i].scene, o).time;
+    const bh_batch_cfg dflt = batch_defaults(c, o.precision, v, batch_entries(frames, n));
+    bh_batch_cfg cfg = cfg_in ? *cfg_in : (c->tuned_ok[o.precision] ? c->tuned[o.precision] : dflt);
+    rc = resolve_cfg(c, dflt, &cfg);
     if (rc) return rc;
     const int mode = frames[0].scene.mode;
     if (c->turb_model == BH_TURB_SHEARED) {
@@ -1153,9 +1206,6 @@ int launch_batch(bh_ctx* c, const bh_batch_frame* frames, int n, const bh_trace_
         }
     }
     const int prio = cfg.prio_age > 0 ? cfg.prio_age : 0;
-    // one kernel for all frames: it integrates the coordinate time if any of them reads it
-    Variant v = variant_of(c, frames[0].scene, o);
-    for (int i = 1; i < n; ++i) v.time = v.time || variant_of(c, frames[i].scene, o).time;
     PersistFn k = pick_persist(o.precision, v, cfg.waves);
     const int grid = persist_grid(c, (const void*)k, cfg.block, cfg.grid_per_cu);
     rc = ensure(c, &c->d_bframes, &c->bframes_cap, sizeof(bhp::BatchFrame) * (size_t)n);
@@ -1243,14 +1293,16 @@ int launch_records(bh_ctx* c, const bh_frame* f, const bh_trace_opts* opts, int 
     if (opts) o = *opts;
     rc = check_opts(c, o);
     if (rc) return rc;
-    bh_batch_cfg cfg = c->tuned_ok[o.precision] ? c->tuned[o.precision] : batch_defaults(o.precision);
-    rc = resolve_cfg(c, o.precision, &cfg);
+    const int tiles_x = (w + 7) / 8, tiles = tiles_x * ((h + 7) / 8);
+    const Variant v = variant_of(c, c->S, o);
+    const bh_batch_cfg dflt = batch_defaults(c, o.precision, v, (long long)tiles * 64);
+    bh_batch_cfg cfg = c->tuned_ok[o.precision] ? c->tuned[o.precision] : dflt;
+    rc = resolve_cfg(c, dflt, &cfg);
     if (rc) return rc;
     rc = prepare_turbulence(c, c->S, f);
     if (rc) return rc;
-    const auto k = pick_adaptive<bhp::RecordWork>(o.precision, variant_of(c, c->S, o), cfg.waves);
+    const auto k = pick_adaptive<bhp::RecordWork>(o.precision, v, cfg.waves);
     const int grid = persist_grid(c, (const void*)k, cfg.block, cfg.grid_per_cu);
-    const int tiles_x = (w + 7) / 8, tiles = tiles_x * ((h + 7) / 8);
     bhp::BatchFrame B;
     std::memset(&B, 0, sizeof B);
     B.P = make_params(c, f);
@@ -1288,6 +1340,63 @@ int launch_records(bh_ctx* c, const bh_frame* f, const bh_trace_opts* opts, int 
     return BH_OK;
 }
 
+// A persistent launch over the samples of a frame: every (tile, sample, pixel) entry's intensities in
+// d_samp1[pixel * spp + sample]. Enqueues the launch and fills B[0] (the frame's descriptor) and B[1]
+// (the same with one entry per pixel). The caller has checked the frame, the options and the sizes.
+int launch_samples(bh_ctx* c, const bh_frame* f, const bh_trace_opts& o, int spp, bhp::BatchFrame B[2],
+                   bh_batch_cfg* cfg_out, int* grid_out) {
+    const int W = f->W, H = f->H;
+    const int tiles_x = (W + 7) / 8, tiles = tiles_x * ((H + 7) / 8);
+    const Variant v = variant_of(c, c->S, o);
+    const bh_batch_cfg dflt = batch_defaults(c, o.precision, v, (long long)tiles * 64 * spp);
+    bh_batch_cfg cfg = c->tuned_ok[o.precision] ? c->tuned[o.precision] : dflt;
+    int rc = resolve_cfg(c, dflt, &cfg);
+    if (rc) return rc;
+    rc = prepare_turbulence(c, c->S, f);
+    if (rc) return rc;
+    const auto k = pick_adaptive<bhp::SampleWork>(o.precision, v, cfg.waves);
+    const int grid = persist_grid(c, (const void*)k, cfg.block, cfg.grid_per_cu);
+    const bool ordered = cfg.order != BH_ORDER_ROWS;
+    std::memset(B, 0, 2 * sizeof B[0]);
+    B[0].P = make_params(c, f);
+    B[0].P.w = W;
+    B[0].P.h = H;
+    B[0].P.spp = spp;
+    B[0].P.jitter = o.jitter;
+    B[0].M = make_mixed(c, c->S, f, o);
+    if (o.emissivity == BH_EMIS_MLP) {
+        B[0].M.use_surrogate = 1;
+        B[0].M.S = c->stab;
+    }
+    B[0].tiles_x = tiles_x;
+    B[0].nentries = (unsigned int)(tiles * 64 * spp);
+    if (ordered) {
+        if ((rc = ensure(c, &c->d_order, &c->order_cap, (size_t)tiles)) ||
+            (rc = ensure(c, &c->d_ohist, &c->ohist_cap, (size_t)ORDER_BUCKETS)))
+            return rc;
+        B[0].order = c->d_order;
+    }
+    // the sort reads nentries / 64 tiles from its descriptor and pass 1 has spp entries per pixel, so the
+    // sort gets slot 1 (pass 2's, written again before pass 2) with one entry per pixel
+    B[1] = B[0];
+    B[1].nentries = (unsigned int)(tiles * 64);
+    if ((rc = ensure(c, &c->d_bframes, &c->bframes_cap, 2 * sizeof B[0])) ||
+        (rc = ensure(c, &c->d_queue, &c->queue_cap, 1)) || (rc = ensure(c, &c->d_blk, &c->blk_cap, (size_t)grid)) ||
+        (rc = ensure(c, &c->d_samp1, &c->samp1_cap, (size_t)W * H * spp)))
+        return rc;
+    const bhp::BatchFrame* dB = (const bhp::BatchFrame*)c->d_bframes;
+    HIPCK(c, hipEventRecord(c->ev0, c->st));
+    HIPCK(c, hipMemcpyAsync(c->d_bframes, B, 2 * sizeof B[0], hipMemcpyHostToDevice, c->st));
+    hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, c->st, c->d_queue, 1);
+    if (ordered) enqueue_tile_order(c->st, dB + 1, 1, (unsigned int)tiles, c->d_ohist, cfg.order);
+    hipLaunchKernelGGL(k, dim3(grid), dim3(cfg.block), 0, c->st, bhp::SampleWork{dB, 1, spp, c->d_samp1}, c->d_queue,
+                       cfg.interval, cfg.refill_min, cfg.prio_age > 0 ? cfg.prio_age : 0, c->d_blk);
+    HIPCK(c, hipGetLastError());
+    *cfg_out = cfg;
+    *grid_out = grid;
+    return BH_OK;
+}
+
 // Adaptive render (render.cu:677-721): persistent pass 1 over (tile, sample, pixel) entries, the
 // statistics and decisions on the device, one host read of the pass-2 size, persistent pass 2 over
 // chunks, resolve. px_out / nsamp_out are device pointers (d_px, d_nsamp).
@@ -1305,67 +1414,24 @@ int launch_adaptive(bh_ctx* c, const bh_frame* f, const bh_trace_opts* opts, lon
     const float target = c->rs.target_err > 0.f ? c->rs.target_err : 0.03f;
     const int W = f->W, H = f->H, npix = W * H;
     const int extra_max = std::max(spp_max - spp, 0);
-    const int tiles_x = (W + 7) / 8, tiles = tiles_x * ((H + 7) / 8);
-    if ((long long)tiles * 64 * spp >= (1ll << 31) ||
+    const long long tiles = (long long)((W + 7) / 8) * ((H + 7) / 8);
+    if (tiles * 64 * spp >= (1ll << 31) ||
         (long long)npix * ((extra_max + ADAPT_CHUNK - 1) / ADAPT_CHUNK) * ADAPT_CHUNK >= (1ll << 31))
         return fail(c, BH_ERR_ARG, "frame too large for adaptive sampling (2^31 samples)");
-    bh_batch_cfg cfg = c->tuned_ok[o.precision] ? c->tuned[o.precision] : batch_defaults(o.precision);
-    rc = resolve_cfg(c, o.precision, &cfg);
-    if (rc) return rc;
-    rc = prepare_turbulence(c, c->S, f);
-    if (rc) return rc;
-    const Variant rk = variant_of(c, c->S, o);
-    const auto k1 = pick_adaptive<bhp::SampleWork>(o.precision, rk, cfg.waves);
-    const auto k2 = pick_adaptive<bhp::ChunkWork>(o.precision, rk, cfg.waves);
-    const int grid = std::min(persist_grid(c, (const void*)k1, cfg.block, cfg.grid_per_cu),
-                              persist_grid(c, (const void*)k2, cfg.block, cfg.grid_per_cu));
-    const int prio = cfg.prio_age > 0 ? cfg.prio_age : 0;
-    const bool ordered = cfg.order != BH_ORDER_ROWS;
-    bhp::BatchFrame B[2];
-    std::memset(B, 0, sizeof B);
-    B[0].P = make_params(c, f);
-    B[0].P.w = W;
-    B[0].P.h = H;
-    B[0].P.spp = spp;
-    B[0].P.jitter = o.jitter;
-    B[0].M = make_mixed(c, c->S, f, o);
-    if (o.emissivity == BH_EMIS_MLP) {
-        B[0].M.use_surrogate = 1;
-        B[0].M.S = c->stab;
-    }
-    B[0].tiles_x = tiles_x;
-    B[0].nentries = (unsigned int)(tiles * 64 * spp);
-    B[1] = B[0];
     const size_t n = (size_t)npix;
-    if (ordered) {
-        if ((rc = ensure(c, &c->d_order, &c->order_cap, (size_t)tiles)) ||
-            (rc = ensure(c, &c->d_ohist, &c->ohist_cap, (size_t)ORDER_BUCKETS)))
-            return rc;
-        B[0].order = c->d_order;
-        // the sort reads nentries / 64 tiles from its descriptor; pass 1 has spp entries per pixel, so
-        // the sort gets slot 1 (pass 2's, written again before pass 2) with one entry per pixel
-        B[1] = B[0];
-        B[1].nentries = (unsigned int)(tiles * 64);
-    }
-    if ((rc = ensure(c, &c->d_bframes, &c->bframes_cap, sizeof B)) || (rc = ensure(c, &c->d_queue, &c->queue_cap, 1)) ||
-        (rc = ensure(c, &c->d_blk, &c->blk_cap, (size_t)grid)) ||
-        (rc = ensure(c, &c->d_samp1, &c->samp1_cap, n * spp)) || (rc = ensure(c, &c->d_acc, &c->acc_cap, n)) ||
+    if ((rc = ensure(c, &c->d_acc, &c->acc_cap, n)) ||
         (rc = ensure(c, &c->d_ystat, &c->ystat_cap, n)) || (rc = ensure(c, &c->d_extra, &c->extra_cap, n)) ||
         (rc = ensure(c, &c->d_chunks, &c->chunks_cap, n)) || (rc = ensure(c, &c->d_offsets, &c->offsets_cap, n)) ||
         (rc = ensure(c, &c->d_bsum, &c->bsum_cap, (n + 1023) / 1024)) ||
         (rc = ensure(c, &c->d_fpart, &c->fpart_cap, (n + FSUM_BLOCK - 1) / FSUM_BLOCK)) ||
         (rc = ensure(c, &c->d_nsamp, &c->nsamp_cap, n)) || (rc = ensure(c, &c->d_px, &c->px_cap, n)))
         return rc;
-    const bhp::BatchFrame* dB = (const bhp::BatchFrame*)c->d_bframes;
     const bool radio = c->S.mode == BH_MODE_RADIO;
-    HIPCK(c, hipEventRecord(c->ev0, c->st));
-    HIPCK(c, hipMemcpyAsync(c->d_bframes, B, sizeof B, hipMemcpyHostToDevice, c->st));
-    // pass 1
-    hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, c->st, c->d_queue, 1);
-    if (ordered) enqueue_tile_order(c->st, dB + 1, 1, (unsigned int)tiles, c->d_ohist, cfg.order);
-    hipLaunchKernelGGL(k1, dim3(grid), dim3(cfg.block), 0, c->st,
-                       bhp::SampleWork{dB, 1, spp, c->d_samp1}, c->d_queue, cfg.interval, cfg.refill_min, prio,
-                       c->d_blk);
+    bhp::BatchFrame B[2];
+    bh_batch_cfg cfg;
+    int grid;
+    rc = launch_samples(c, f, o, spp, B, &cfg, &grid);
+    if (rc) return rc;
     hipLaunchKernelGGL(k_reduce, dim3(1), dim3(256), 0, c->st, c->d_blk, grid, c->d_tot);
     HIPCK(c, hipGetLastError());
     BlockOut tot1, tot2{};
@@ -1392,8 +1458,18 @@ int launch_adaptive(bh_ctx* c, const bh_frame* f, const bh_trace_opts* opts, lon
         HIPCK(c, hipStreamSynchronize(c->st));
         total = last[0] + last[1];
         if (total > 0) {
-            rc = ensure(c, &c->d_samp2, &c->samp2_cap, (size_t)total * ADAPT_CHUNK);
+            // pass 2's launch by its own number of rays
+            const Variant v = variant_of(c, c->S, o);
+            const bh_batch_cfg dflt = batch_defaults(c, o.precision, v, (long long)total * ADAPT_CHUNK);
+            if (!c->tuned_ok[o.precision]) cfg = dflt;
+            rc = resolve_cfg(c, dflt, &cfg);
             if (rc) return rc;
+            const auto k2 = pick_adaptive<bhp::ChunkWork>(o.precision, v, cfg.waves);
+            grid = persist_grid(c, (const void*)k2, cfg.block, cfg.grid_per_cu);
+            if ((rc = ensure(c, &c->d_samp2, &c->samp2_cap, (size_t)total * ADAPT_CHUNK)) ||
+                (rc = ensure(c, &c->d_blk, &c->blk_cap, (size_t)grid)))
+                return rc;
+            const bhp::BatchFrame* dB = (const bhp::BatchFrame*)c->d_bframes;
             B[1].nentries = total * ADAPT_CHUNK;
             B[1].order = nullptr;
             HIPCK(c, hipMemcpyAsync(c->d_bframes + sizeof(bhp::BatchFrame), &B[1], sizeof B[1], hipMemcpyHostToDevice,
@@ -1401,7 +1477,7 @@ int launch_adaptive(bh_ctx* c, const bh_frame* f, const bh_trace_opts* opts, lon
             hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, c->st, c->d_queue, 1);
             hipLaunchKernelGGL(k2, dim3(grid), dim3(cfg.block), 0, c->st,
                                bhp::ChunkWork{dB + 1, 1, spp, npix, c->d_offsets, c->d_samp2}, c->d_queue,
-                               cfg.interval, cfg.refill_min, prio, c->d_blk);
+                               cfg.interval, cfg.refill_min, cfg.prio_age > 0 ? cfg.prio_age : 0, c->d_blk);
             hipLaunchKernelGGL(k_reduce, dim3(1), dim3(256), 0, c->st, c->d_blk, grid, c->d_tot);
             HIPCK(c, hipGetLastError());
             HIPCK(c, hipMemcpyAsync(&tot2, c->d_tot, sizeof tot2, hipMemcpyDeviceToHost, c->st));
@@ -1716,8 +1792,33 @@ int bh_radio_flux(bh_ctx* c, const bh_frame* f, int n, double pix_sr, double* jy
     o.jitter = 1;
     o.spp = 2;
     bh_stats st{};
-    int rc = launch_trace(c, &g, &o, 0, 0, n, n, false, &st);
-    if (rc) return rc;
+    const long long entries = (long long)((n + 7) / 8) * ((n + 7) / 8) * 64 * o.spp;
+    if ((double)entries * sizeof(double4) <= (double)PLAIN_SPP_SAMPLE_BUDGET) {
+        // Each sample a ray of its own on the persistent engine. The frame kernel traces a pixel's two
+        // samples one after the other and n = 160 is 100 workgroups for 256 CUs: it ends with the longest
+        // pair of rays on a lane, this with the longest ray (the 230 GHz flow at 17 degrees, three
+        // cameras in turn: 13.7 ms there, 10.6 here).
+        int rc = check_frame(c, &g);
+        if (rc) return rc;
+        bhp::BatchFrame B[2];
+        bh_batch_cfg cfg;
+        int grid, per_xcd;
+        rc = launch_samples(c, &g, o, o.spp, B, &cfg, &grid);
+        if (rc) return rc;
+        const int nb = trace_blocks(n, n, &per_xcd);
+        rc = ensure(c, &c->d_blk, &c->blk_cap, (size_t)nb);
+        if (rc) return rc;
+        hipLaunchKernelGGL(k_flux_blocks, dim3(nb), dim3(BLOCK), 0, c->st, c->d_samp1, n, n, o.spp, c->d_blk, per_xcd);
+        hipLaunchKernelGGL(k_reduce, dim3(1), dim3(256), 0, c->st, c->d_blk, nb, c->d_tot);
+        HIPCK(c, hipGetLastError());
+        BlockOut tot;
+        HIPCK(c, hipMemcpyAsync(&tot, c->d_tot, sizeof tot, hipMemcpyDeviceToHost, c->st));
+        HIPCK(c, hipStreamSynchronize(c->st));
+        st.flux_sum = tot.flux;
+    } else {
+        int rc = launch_trace(c, &g, &o, 0, 0, n, n, false, &st);
+        if (rc) return rc;
+    }
     // render.cu:803-808: sum of the per-pixel means times the pixel solid angle, in Jy
     *jy = st.flux_sum / 2.0 * pix_sr / 1e-23;
     return BH_OK;
@@ -1747,7 +1848,9 @@ int bh_autotune(bh_ctx* c, const bh_batch_frame* frames, int n, const bh_trace_o
     HIPCK(c, hipSetDevice(c->device));
     // coordinate descent from the defaults: one parameter at a time over its candidate list, two passes
     const int prec = opts ? opts->precision : BH_PREC_FP64;
-    bh_batch_cfg cur = batch_defaults(prec);
+    if (!frames || n <= 0) return fail(c, BH_ERR_ARG, "empty batch");
+    const Variant v = variant_of(c, frames[0].scene, opts ? *opts : bh_trace_opts{});
+    bh_batch_cfg cur = batch_defaults(c, prec, v, batch_entries(frames, n));
     int count = 0;
     double cur_ms = 0.0;
     auto time_cfg = [&](const bh_batch_cfg& g, double* ms) -> int {
