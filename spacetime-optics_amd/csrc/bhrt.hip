@@ -1591,6 +1591,12 @@ int bh_create(int device, const bh_scene* scene, const bh_tables* tables, const 
         c->err = "cannot query the compute-unit count";
         return bail(BH_ERR_HIP);
     }
+    try {
+        c->transfer = Transfer::of_device(device);
+    } catch (...) {
+        c->err = "host allocation failed";
+        return bail(BH_ERR_HIP);
+    }
     c->emit_cache.reserve(64);   // make_mixed then never allocates (bh_render_noalloc)
     if (device < NOALLOC_MAX_DEVICES) {
         // this device's copy of the no-alloc scratch array, resolved once with the device current
@@ -1682,8 +1688,7 @@ int bh_render(bh_ctx* c, const bh_frame* f, const bh_trace_opts* opts, float* px
     int rc = render_frame(c, f, opts, &img, &local);
     if (rc) return rc;
     if (px_out) {
-        HIPCK(c, hipMemcpyAsync(px_out, img, sizeof(float4) * (size_t)f->W * f->H, hipMemcpyDeviceToHost, c->st));
-        HIPCK(c, hipStreamSynchronize(c->st));
+        HIPCK(c, c->transfer->to_host(px_out, img, sizeof(float4) * (size_t)f->W * f->H, c->st));
     }
     local.ms_trace = now_ms() - t0;
     if (st) *st = local;
@@ -1699,9 +1704,8 @@ int bh_render_adaptive(bh_ctx* c, const bh_frame* f, const bh_trace_opts* opts, 
     int rc = launch_adaptive(c, f, opts, nullptr, &local);
     if (rc) return rc;
     const size_t n = (size_t)f->W * f->H;
-    if (px_out) HIPCK(c, hipMemcpyAsync(px_out, c->d_px, sizeof(float4) * n, hipMemcpyDeviceToHost, c->st));
-    if (nsamp_out) HIPCK(c, hipMemcpyAsync(nsamp_out, c->d_nsamp, sizeof(unsigned int) * n, hipMemcpyDeviceToHost, c->st));
-    HIPCK(c, hipStreamSynchronize(c->st));
+    if (px_out) HIPCK(c, c->transfer->to_host(px_out, c->d_px, sizeof(float4) * n, c->st));
+    if (nsamp_out) HIPCK(c, c->transfer->to_host(nsamp_out, c->d_nsamp, sizeof(unsigned int) * n, c->st));
     local.ms_trace = now_ms() - t0;
     if (st) *st = local;
     return BH_OK;
@@ -1758,8 +1762,7 @@ int bh_trace_tile(bh_ctx* c, const bh_frame* f, int x0, int y0, int w, int h, co
     int rc = frame_kernel ? launch_trace(c, f, opts, x0, y0, w, h, true, nullptr)
                           : launch_records(c, f, opts, x0, y0, w, h);
     if (rc) return rc;
-    HIPCK(c, hipMemcpyAsync(out, c->d_rays, sizeof(bh_ray_out) * (size_t)w * h, hipMemcpyDeviceToHost, c->st));
-    HIPCK(c, hipStreamSynchronize(c->st));
+    HIPCK(c, c->transfer->to_host(out, c->d_rays, sizeof(bh_ray_out) * (size_t)w * h, c->st));
     return BH_OK;
 }
 
@@ -1775,8 +1778,7 @@ int bh_sheared_slices(bh_ctx* c, const bh_frame* f, float* out, size_t n) {
     if (!(S.flow_turb_amp > 0.f)) return fail(c, BH_ERR_ARG, "the scene has no turbulence (flow_turb_amp = 0)");
     int rc = prepare_turbulence(c, S, f);
     if (rc) return rc;
-    HIPCK(c, hipMemcpyAsync(out, c->d_ts, sizeof(float) * total, hipMemcpyDeviceToHost, c->st));
-    HIPCK(c, hipStreamSynchronize(c->st));
+    HIPCK(c, c->transfer->to_host(out, c->d_ts, sizeof(float) * total, c->st));
     return BH_OK;
 }
 
@@ -1834,8 +1836,7 @@ int bh_trace_batch(bh_ctx* c, const bh_batch_frame* frames, int n, const bh_trac
     int rc = launch_batch(c, frames, n, opts, cfg, &npix, &local);
     if (rc) return rc;
     if (px_out) {
-        HIPCK(c, hipMemcpyAsync(px_out, c->d_bout, sizeof(float4) * (size_t)npix, hipMemcpyDeviceToHost, c->st));
-        HIPCK(c, hipStreamSynchronize(c->st));
+        HIPCK(c, c->transfer->to_host(px_out, c->d_bout, sizeof(float4) * (size_t)npix, c->st));
     }
     local.ms_trace = now_ms() - t0;
     if (st) *st = local;

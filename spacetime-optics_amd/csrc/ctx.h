@@ -10,6 +10,7 @@
 #include "../../include/bhrt.h"
 #include "mlp.h"
 #include "trace_fp64.h"
+#include "transfer.h"
 
 constexpr int NCNT = 5;   // counters per block: attempts, accepted, flow, limited, fp64 attempts
 
@@ -22,6 +23,7 @@ struct BlockOut {
 struct bh_ctx {
     int device = 0;
     hipStream_t st = nullptr;
+    std::shared_ptr<Transfer> transfer;   // large copies to and from the caller's memory
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     bh_scene S{};
     bh_settings rs{};

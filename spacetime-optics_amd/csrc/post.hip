@@ -315,8 +315,7 @@ int bh_post_radio(bh_ctx* c, float* px, int W, int H, const bh_post_params* para
         if (k > 0) hipLaunchKernelGGL(k_pyr_up, grid1((long long)npix), dim3(POST_BLOCK), 0, c->st, L, lw[k], lh[k],
                                       lev, W, H);
         PCK(c, hipGetLastError());
-        PCK(c, hipMemcpyAsync(px, lev, sizeof(float4) * npix, hipMemcpyDeviceToHost, c->st));
-        PCK(c, hipStreamSynchronize(c->st));
+        PCK(c, c->transfer->to_host(px, lev, sizeof(float4) * npix, c->st));
     }
     // statistics of the displayed intensity (render.cu:771-791)
     if (lum_percentile || lum_max) {
@@ -348,8 +347,7 @@ int bh_post_radio(bh_ctx* c, float* px, int W, int H, const bh_post_params* para
 }
 
 static int copy_rgb(bh_ctx* c, int W, int H, unsigned char* rgb8) {
-    PCK(c, hipMemcpyAsync(rgb8, c->d_post_rgb, 3 * (size_t)W * H, hipMemcpyDeviceToHost, c->st));
-    PCK(c, hipStreamSynchronize(c->st));
+    PCK(c, c->transfer->to_host(rgb8, c->d_post_rgb, 3 * (size_t)W * H, c->st));
     return BH_OK;
 }
 
