@@ -18,6 +18,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstring>
 #include <string>
 #include <vector>
 
@@ -36,6 +37,7 @@ namespace {
     } while (0)
 
 constexpr int POST_BLOCK = 256;
+constexpr int HUD_MAX_GLYPHS = 4096, HUD_MAX_RECTS = 1024;   // the reference's limits
 constexpr int POST_MAX_LEVELS = 9;   // pyramid depth of the reference (render.cu:32)
 
 __device__ __forceinline__ float sat(float x) { return x < 0.f ? 0.f : (x > 1.f ? 1.f : x); }
@@ -181,6 +183,105 @@ __global__ __launch_bounds__(POST_BLOCK) void k_tone_radio(const float4* __restr
     }
 }
 
+/* Display statistics (render.cu:771-791) of a frame in device memory: the maximum of the displayed
+   intensity Y and the `rank`-th smallest of the values above 1e-5 of it, exactly (no sort: three counting
+   passes over the value's bits, 11 + 10 + 10 of them - positive floats order as their bits do). The
+   passes read 4 bytes a pixel at memory rate; what they replace is one host core's pass over the frame,
+   two growing arrays and a selection (1920 x 1080: about 4 ms; the passes take 0.13). */
+constexpr int LUM_BINS = 2048;
+struct LumState {
+    unsigned int max_bits;   // of the largest Y > 0; 0: none
+    unsigned int n;          // values above the threshold
+    unsigned int rank;       // of the value sought among those that share `prefix`
+    unsigned int prefix;     // the leading bits found so far; after the last pass the value's bits
+    unsigned int hist[3][LUM_BINS];
+};
+
+__global__ void k_lum_zero(LumState* __restrict__ S) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < (int)(sizeof(LumState) / sizeof(unsigned int))) ((unsigned int*)S)[i] = 0u;
+}
+
+// Y of every pixel (0 where it is not positive) and the largest
+__global__ __launch_bounds__(POST_BLOCK) void k_lum(const float4* __restrict__ img, int npix, float hide,
+                                                    float* __restrict__ lum, LumState* __restrict__ S) {
+    unsigned int top = 0u;
+    for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < npix; p += gridDim.x * blockDim.x) {
+        const float4 v = img[p];
+        float d = v.x - v.y - v.z - v.w;
+        d = d < 0.f ? 0.f : d;   // std::max: a NaN stays
+        const float Y = v.x - hide * d;
+        const float y = Y > 0.f ? Y : 0.f;
+        lum[p] = y;
+        top = max(top, __float_as_uint(y));
+    }
+    for (int off = 32; off > 0; off >>= 1) top = max(top, (unsigned int)__shfl_down((int)top, off, 64));
+    // one atomic per workgroup: all of them on one word, one per wave took 60 us
+    __shared__ unsigned int s_top[POST_BLOCK / 64];
+    if ((threadIdx.x & 63) == 0) s_top[threadIdx.x >> 6] = top;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < POST_BLOCK / 64; ++w) top = max(top, s_top[w]);
+        if (top) atomicMax(&S->max_bits, top);
+    }
+}
+
+// Counts the values above the threshold by the next bits below those already found. A workgroup counts
+// in LDS first: neighbouring pixels fall into the same few bins.
+template <int PASS>
+__global__ __launch_bounds__(POST_BLOCK) void k_lum_count(const float* __restrict__ lum, int npix,
+                                                          LumState* __restrict__ S) {
+    constexpr int SHIFT = PASS == 0 ? 20 : (PASS == 1 ? 10 : 0), BINS = PASS == 0 ? LUM_BINS : LUM_BINS / 2;
+    __shared__ unsigned int h[BINS];
+    for (int i = threadIdx.x; i < BINS; i += POST_BLOCK) h[i] = 0u;
+    __syncthreads();
+    const double thr = (double)__uint_as_float(S->max_bits) * 1e-5;
+    const unsigned int prefix = S->prefix;
+    for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < npix; p += gridDim.x * blockDim.x) {
+        const float y = lum[p];
+        const unsigned int b = __float_as_uint(y);
+        if ((double)y > thr && (PASS == 0 || b >> (SHIFT + 10) == prefix)) atomicAdd(&h[(b >> SHIFT) & (BINS - 1)], 1u);
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < BINS; i += POST_BLOCK)
+        if (h[i]) atomicAdd(&S->hist[PASS][i], h[i]);
+}
+
+// The bin that holds the rank, from a scan of the counts (one workgroup, 8 or 4 bins per thread)
+template <int PASS>
+__global__ __launch_bounds__(POST_BLOCK) void k_lum_pick(LumState* __restrict__ S, double q) {
+    constexpr int BINS = PASS == 0 ? LUM_BINS : LUM_BINS / 2, PER = BINS / POST_BLOCK;
+    __shared__ unsigned int part[POST_BLOCK];
+    unsigned int v[PER], sum = 0u;
+    for (int i = 0; i < PER; ++i) {
+        v[i] = S->hist[PASS][threadIdx.x * PER + i];
+        sum += v[i];
+    }
+    part[threadIdx.x] = sum;
+    __syncthreads();
+    for (int off = 1; off < POST_BLOCK; off <<= 1) {
+        const unsigned int x = (int)threadIdx.x >= off ? part[threadIdx.x - off] : 0u;
+        __syncthreads();
+        part[threadIdx.x] += x;
+        __syncthreads();
+    }
+    const unsigned int n = part[POST_BLOCK - 1];
+    if (n == 0u) return;   // no value above the threshold
+    // idx = min(n - 1, floor(q (n - 1))) of the sorted values
+    const unsigned int rank = PASS == 0 ? min(n - 1u, (unsigned int)(q * (double)(n - 1u))) : S->rank;
+    __syncthreads();       // every thread has read the rank
+    unsigned int run = part[threadIdx.x] - sum;
+    for (int i = 0; i < PER; ++i) {
+        if (rank >= run && rank < run + v[i]) {
+            S->rank = rank - run;
+            S->prefix = PASS == 0 ? (unsigned int)(threadIdx.x * PER + i)
+                                  : S->prefix << 10 | (unsigned int)(threadIdx.x * PER + i);
+            if (PASS == 0) S->n = n;
+        }
+        run += v[i];
+    }
+}
+
 int grow(bh_ctx* c, void** p, size_t* cap, size_t bytes) {
     if (*cap >= bytes && *p) return BH_OK;
     if (*p) {
@@ -196,23 +297,56 @@ int grow(bh_ctx* c, void** p, size_t* cap, size_t bytes) {
 
 inline dim3 grid1(long long n) { return dim3((unsigned int)((n + POST_BLOCK - 1) / POST_BLOCK)); }
 
+// Appends to the workgroup's list, in order, the elements i < n that `hit` accepts. Every thread calls it.
+template <typename F>
+__device__ __forceinline__ int collect(int n, unsigned short* list, int* s_wave, F hit) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int total = 0;
+    for (int base = 0; base < n; base += POST_BLOCK) {
+        const int i = base + threadIdx.x;
+        const bool in = i < n && hit(i);
+        const unsigned long long m = __ballot(in);
+        if (lane == 0) s_wave[wave] = __popcll(m);
+        __syncthreads();
+        int before = total;
+        for (int w = 0; w < POST_BLOCK / 64; ++w) {
+            if (w < wave) before += s_wave[w];
+            total += s_wave[w];
+        }
+        if (in) list[before + __popcll(m & ((1ull << lane) - 1ull))] = (unsigned short)i;
+        __syncthreads();   // the list is complete, and s_wave may be written again
+    }
+    return total;
+}
+
 // HUD over the tone-mapped bytes, one work-item per pixel: every rectangle (sorted by layer on the
 // host), then every glyph's shadow, then every glyph, in list order - the blends of k_hud_rects and
-// k_hud_glyphs (render.cu:409-446) in the same float operations. The element loops are wave-uniform,
-// so each element's fields arrive through scalar loads; a glyph touches only the pixels of its cell.
+// k_hud_glyphs (render.cu:409-446) in the same float operations. A workgroup's 256 pixels first collect
+// the elements whose boxes touch them (one test per element and workgroup; most touch none), then blend
+// those in order: with every pixel walking every element the full HD overlay took 235 us, now 36.
 __global__ __launch_bounds__(POST_BLOCK) void k_hud(unsigned char* __restrict__ rgb, int W, int H,
                                                     const bh_hud_rect* __restrict__ rects, int nr,
                                                     const bh_hud_glyph* __restrict__ glyphs, int ng,
                                                     const unsigned char* __restrict__ atlas, int cell_w, int cell_h,
                                                     float off) {
-    const long long p = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= (long long)W * H) return;
+    __shared__ unsigned short list[HUD_MAX_GLYPHS];
+    __shared__ int s_wave[POST_BLOCK / 64];
+    const long long p0 = (long long)blockIdx.x * POST_BLOCK, npix = (long long)W * H;
+    const long long p1 = min(p0 + POST_BLOCK, npix) - 1, p = min(p0 + threadIdx.x, npix - 1);
+    const bool mine = p0 + threadIdx.x < npix;
     const int X = (int)(p % W), Y = (int)(p / W);
+    // the pixels' box: part of a row, or whole rows
+    const int ya = (int)(p0 / W), yb = (int)(p1 / W);
+    const int xa = ya == yb ? (int)(p0 % W) : 0, xb = ya == yb ? (int)(p1 % W) : W - 1;
     unsigned char* o = rgb + 3 * p;
     float d0 = (float)o[0], d1 = (float)o[1], d2 = (float)o[2];
     bool touched = false;
-    for (int i = 0; i < nr; ++i) {
+    const int hr = collect(nr, list, s_wave, [&](int i) {
         const bh_hud_rect R = rects[i];
+        return xa < R.x1 && xb >= R.x0 && ya < R.y1 && yb >= R.y0;
+    });
+    for (int k = 0; k < hr; ++k) {
+        const bh_hud_rect R = rects[list[k]];
         if (X < R.x0 || X >= R.x1 || Y < R.y0 || Y >= R.y1) continue;
         const float a = (float)((R.rgba >> 24) & 255u) / 255.f;
         d0 = (float)(unsigned char)fminf(d0 * (1.f - a) + (float)(int)(R.rgba & 255u) * a + 0.5f, 255.f);
@@ -222,8 +356,15 @@ __global__ __launch_bounds__(POST_BLOCK) void k_hud(unsigned char* __restrict__ 
     }
     for (int pass = 0; pass < 2; ++pass) {
         const float dxy = pass == 0 ? off : 0.f;
-        for (int i = 0; i < ng; ++i) {
+        __syncthreads();   // the list is rewritten
+        const int hg = collect(ng, list, s_wave, [&](int i) {
             const bh_hud_glyph G = glyphs[i];
+            const int cw = (int)ceilf((float)cell_w * G.scale) + 1, ch = (int)ceilf((float)cell_h * G.scale) + 1;
+            const int gx = (int)floorf(G.x + dxy), gy = (int)floorf(G.y + dxy);
+            return xb >= gx && yb >= gy && xa - gx < cw && ya - gy < ch;
+        });
+        for (int k = 0; k < hg; ++k) {
+            const bh_hud_glyph G = glyphs[list[k]];
             const int cw = (int)ceilf((float)cell_w * G.scale) + 1, ch = (int)ceilf((float)cell_h * G.scale) + 1;
             const int ix = X - (int)floorf(G.x + dxy), iy = Y - (int)floorf(G.y + dxy);
             if (ix < 0 || iy < 0 || ix >= cw || iy >= ch) continue;
@@ -249,7 +390,7 @@ __global__ __launch_bounds__(POST_BLOCK) void k_hud(unsigned char* __restrict__ 
             touched = true;
         }
     }
-    if (touched) {
+    if (touched && mine) {
         o[0] = (unsigned char)d0;
         o[1] = (unsigned char)d1;
         o[2] = (unsigned char)d2;
@@ -270,7 +411,8 @@ int bh_post_radio(bh_ctx* c, float* px, int W, int H, const bh_post_params* para
     PCK(c, hipSetDevice(c->device));
     const bh_post_params pp = params ? *params : bh_post_params{0.0, 0.f};
     const size_t npix = (size_t)W * H;
-    if (pp.blur_sigma_px > 0.5) {
+    const bool blurred = pp.blur_sigma_px > 0.5;   // then the frame stays in d_post_lev
+    if (blurred) {
         // pyramid of the reference: halve (rounding up) while both sides are >= 2, at most 9 levels
         int lw[POST_MAX_LEVELS], lh[POST_MAX_LEVELS], nlev = 0;
         size_t loff[POST_MAX_LEVELS], total = 0;
@@ -319,6 +461,41 @@ int bh_post_radio(bh_ctx* c, float* px, int W, int H, const bh_post_params* para
     }
     // statistics of the displayed intensity (render.cu:771-791)
     if (lum_percentile || lum_max) {
+        const double q = std::min(std::max(percentile, 0.0), 1.0);
+        // On the device for all but small frames: its launches take about as long as the host's pass over
+        // 16384 pixels, with the frame's copy to the device as long as that over 65536.
+        if (npix >= (blurred ? (size_t)1 << 14 : (size_t)1 << 16) && q == q) {
+            int rc;
+            if (!blurred) {
+                if ((rc = grow(c, (void**)&c->d_post_lev, &c->post_lev_cap, sizeof(float4) * npix))) return rc;
+                PCK(c, hipMemcpyAsync(c->d_post_lev, px, sizeof(float4) * npix, hipMemcpyHostToDevice, c->st));
+            }
+            if ((rc = grow(c, (void**)&c->d_post_tmp, &c->post_tmp_cap, sizeof(float) * npix)) ||
+                (rc = grow(c, (void**)&c->d_post_wt, &c->post_wt_cap, sizeof(LumState))))
+                return rc;
+            float* lum = (float*)c->d_post_tmp;
+            LumState* S = (LumState*)c->d_post_wt;
+            const dim3 one(1), blk(POST_BLOCK), g((unsigned)std::min<size_t>((npix + POST_BLOCK - 1) / POST_BLOCK, 1024));
+            const int n = (int)npix;
+            hipLaunchKernelGGL(k_lum_zero, grid1(sizeof(LumState) / 4), blk, 0, c->st, S);
+            hipLaunchKernelGGL(k_lum, g, blk, 0, c->st, (const float4*)c->d_post_lev, n, pp.hide_direct, lum, S);
+            hipLaunchKernelGGL(k_lum_count<0>, g, blk, 0, c->st, lum, n, S);
+            hipLaunchKernelGGL(k_lum_pick<0>, one, blk, 0, c->st, S, q);
+            hipLaunchKernelGGL(k_lum_count<1>, g, blk, 0, c->st, lum, n, S);
+            hipLaunchKernelGGL(k_lum_pick<1>, one, blk, 0, c->st, S, q);
+            hipLaunchKernelGGL(k_lum_count<2>, g, blk, 0, c->st, lum, n, S);
+            hipLaunchKernelGGL(k_lum_pick<2>, one, blk, 0, c->st, S, q);
+            PCK(c, hipGetLastError());
+            unsigned int out[4];   // max_bits, n, rank, prefix
+            PCK(c, hipMemcpyAsync(out, S, sizeof out, hipMemcpyDeviceToHost, c->st));
+            PCK(c, hipStreamSynchronize(c->st));
+            float top, value;
+            std::memcpy(&top, &out[0], 4);
+            std::memcpy(&value, &out[3], 4);
+            if (lum_percentile) *lum_percentile = out[1] ? (double)value : 0.0;
+            if (lum_max) *lum_max = (double)top;
+            return BH_OK;
+        }
         std::vector<float> lum;
         lum.reserve(npix);
         double mx = 0.0;
@@ -335,7 +512,6 @@ int bh_post_radio(bh_ctx* c, float* px, int W, int H, const bh_post_params* para
             if (v > mx * 1e-5) sig.push_back(v);
         double pv = 0.0;
         if (!sig.empty()) {
-            const double q = std::min(std::max(percentile, 0.0), 1.0);
             const size_t idx = std::min(sig.size() - 1, (size_t)(q * (double)(sig.size() - 1)));
             std::nth_element(sig.begin(), sig.begin() + (long)idx, sig.end());
             pv = sig[idx];
@@ -384,7 +560,7 @@ int bh_tonemap_hud(bh_ctx* c, const float* px, int W, int H, const bh_tone_param
                    int n_glyphs, const bh_hud_rect* rects, int n_rects, const bh_font* font, unsigned char* rgb8) {
     if (!c || !px || !rgb8 || !params || W <= 0 || H <= 0 || n_glyphs < 0 || n_rects < 0) return BH_ERR_ARG;
     if ((n_glyphs > 0 && !glyphs) || (n_rects > 0 && !rects)) return BH_ERR_ARG;
-    const int ng = std::min(n_glyphs, 4096), nr = std::min(n_rects, 1024);   // the reference's limits
+    const int ng = std::min(n_glyphs, HUD_MAX_GLYPHS), nr = std::min(n_rects, HUD_MAX_RECTS);
     if (ng > 0) {
         if (!font || !font->atlas || font->cell_w < 1 || font->cell_h < 1 || font->glyphs < 1 ||
             font->cell_w > 256 || font->cell_h > 256) {
