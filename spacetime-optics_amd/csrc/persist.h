@@ -173,8 +173,9 @@ struct Tracer<BH_PREC_FP64, RADIO, TIME> {
                                                 State& R) {
         bhd::ray_init<RADIO>(P, x, y, R);
     }
-    static __device__ __forceinline__ void step(const TraceParams& P, const bhm32::MixedParams&, State& R) {
-        bhd::ray_step<RADIO, TIME>(P, R);
+    static __device__ __forceinline__ void step(const TraceParams& P, const bhm32::MixedParams&, const TraceParams& F,
+                                                const bhm32::MixedParams&, State& R) {
+        bhd::ray_step<RADIO, TIME>(P, F, R);
     }
     static __device__ __forceinline__ int result(const TraceParams& P, const State& R, RayResult& out) {
         bhd::ray_result(P, R, out);
@@ -189,8 +190,9 @@ struct Tracer<BH_PREC_MIXED, RADIO, TIME> {
                                                 State& R) {
         bhm32::ray_init_m<RADIO>(P, M, x, y, R);
     }
-    static __device__ __forceinline__ void step(const TraceParams& P, const bhm32::MixedParams& M, State& R) {
-        bhm32::ray_step_m<RADIO, TIME>(P, M, R);
+    static __device__ __forceinline__ void step(const TraceParams& P, const bhm32::MixedParams& M, const TraceParams& F,
+                                                const bhm32::MixedParams& FM, State& R) {
+        bhm32::ray_step_m<RADIO, TIME>(P, M, F, FM, R);
     }
     static __device__ __forceinline__ int result(const TraceParams& P, const State& R, RayResult& out) {
         return bhm32::ray_result_m(P, R, out);
@@ -262,17 +264,24 @@ __device__ __forceinline__ void persist_body(const Work& Wk, unsigned int* __res
         // frame parameters through the constant address space: wave-uniform scalar loads
         using CFrame = const __attribute__((address_space(4))) BatchFrame;
         CFrame* cfr = (CFrame*)frames;
-        const TraceParams& P = *(const TraceParams*)&cfr[cf].P;
-        const bhm32::MixedParams& M = *(const bhm32::MixedParams*)&cfr[cf].M;
+        const TraceParams& P0 = *(const TraceParams*)&cfr[cf].P;
+        const bhm32::MixedParams& M0 = *(const bhm32::MixedParams*)&cfr[cf].M;
+        // What every attempt reads of them is loaded once per interval, into scalar registers: read
+        // through P0, each field is loaded again at its use and the wave waits for the scalar cache, 5
+        // times an attempt in the vacuum and some 25 times in the flow. The flow's tables stay behind P0
+        // and M0 (with them the registers spill). FP64 vacuum records of 256^2 3.2 -> 2.8 ms; mixed
+        // radio, 8 frames of 4.0 M rays, 11.0 -> 9.8; 1024^2 with the surrogate 2.9 -> 2.6 (kernel).
+        const TraceParams P = P0;
+        const bhm32::MixedParams M = M0;
         for (int k = 0; k < interval; ++k)
-            if (active && !R.done) T::step(P, M, R);
+            if (active && !R.done) T::step(P, M, P0, M0, R);
         // Finished rays are written here, all of the interval's together: inside the loop nearly every
         // step of a 64-ray wave would end some ray and hold the others up for its output (LDS sums, a
         // store, the escape direction). Mixed radio, 8 frames of 4.0 M rays: 11.6 -> 11.0 ms; 1024^2 with
         // the surrogate: 3.02 -> 2.94.
         if (active && R.done) {
             RayResult r;
-            const int f64 = T::result(P, R, r);
+            const int f64 = T::result(P0, R, r);
             Wk.finish(cf, ent, r);
             s_flux[tid] += r.I[0];
             s_stat[0][tid] += (unsigned long long)r.steps;

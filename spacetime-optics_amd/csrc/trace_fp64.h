@@ -518,8 +518,9 @@ __device__ __forceinline__ void ray_init(const TraceParams& P, double x, double 
 }
 
 // One iteration of trace.cuh:81-163 (one DP54 attempt); sets R.done when the ray stops.
+// P is what every attempt reads, F the same frame for what only a sample of the flow reads.
 template <int RADIO, bool TIME>
-__device__ __forceinline__ void ray_step(const TraceParams& P, RayState& R) {
+__device__ __forceinline__ void ray_step(const TraceParams& P, const TraceParams& F, RayState& R) {
     const bool flow = RADIO && P.flow_on;
     State n;
     double hc = R.h;
@@ -554,7 +555,7 @@ __device__ __forceinline__ void ray_step(const TraceParams& P, RayState& R) {
     if (flow && n.y0 < P.r_flow_max) {
         double dI, dtau;
         ++R.flow_steps;
-        flow_step<RADIO>(P, n.y0, n.y2, w, R.sn, n.y4, sv, cv, n.y5, R.c.lam, R.c.E, hc, &dI, &dtau);
+        flow_step<RADIO>(F, n.y0, n.y2, w, R.sn, n.y4, sv, cv, n.y5, R.c.lam, R.c.E, hc, &dI, &dtau);
         double cI = R.trans * dI;
         int ord = (int)(R.psi * (1.0 / PI));
         R.acc0 += cI;
@@ -654,7 +655,7 @@ template <int RADIO, bool TIME>
 __device__ __forceinline__ void trace_ray_fp64(const TraceParams& P, double x, double yv, RayResult& out) {
     RayState R;
     ray_init<RADIO>(P, x, yv, R);
-    while (!R.done) ray_step<RADIO, TIME>(P, R);
+    while (!R.done) ray_step<RADIO, TIME>(P, P, R);
     ray_result(P, R, out);
 }
 

@@ -746,11 +746,14 @@ __device__ __forceinline__ void ray_init_m(const TraceParams& P, const MixedPara
     R.done = P.max_steps <= 0;
 }
 
-// One attempt of trace.cuh:81-163 under the mixed policy. TCACHE keeps the ray's turbulence cell
+// One attempt of trace.cuh:81-163 under the mixed policy. P and M are what every attempt reads (the
+// persistent engine holds them in registers), F and FM the same frame for what only a sample of the
+// flow reads. TCACHE keeps the ray's turbulence cell
 // in its state across attempts (the persistent engine); without it every flow sample loads its
 // corners (the frame kernel, already at the register limit, would spill the cache in its loop).
 template <int RADIO, bool TIME, bool TCACHE = true>
-__device__ __forceinline__ void ray_step_m(const TraceParams& P, const MixedParams& M, RayStateM& R) {
+__device__ __forceinline__ void ray_step_m(const TraceParams& P, const MixedParams& M, const TraceParams& F,
+                                           const MixedParams& FM, RayStateM& R) {
     const bool flow = RADIO && P.flow_on;
     State n;
     double hc = R.h;
@@ -773,8 +776,10 @@ __device__ __forceinline__ void ray_step_m(const TraceParams& P, const MixedPara
         }
         // inside the emission region the scene tolerance, relaxed for a ray that has already taken
         // relax_after attempts (an orbit near the photon sphere)
-        const double inv_tol = R.s.y0 < M.r_tol ? (R.it >= M.relax_after ? M.inv_tol_relax : M.inv_tol)
-                                                : (R.s.y0 < M.r_far ? M.inv_tol_mid : M.inv_tol_far);
+        // values, not lvalues: a choice of addresses would put the parameters in memory
+        const double near = R.it >= M.relax_after ? +M.inv_tol_relax : +M.inv_tol;
+        const double far = R.s.y0 < M.r_far ? +M.inv_tol_mid : +M.inv_tol_far;
+        const double inv_tol = R.s.y0 < M.r_tol ? near : far;
         if constexpr (RADIO == bhd::RADIO_OFF) err = dp54_n<TIME>(make_nconst(P, R.c), R.s, hc, inv_tol, M.inv_tol_t, n);
         else err = dp54<double, TIME>(cd, R.s, hc, inv_tol, M.inv_tol_t, n);
         ++R.fp64_attempts;
@@ -798,7 +803,7 @@ __device__ __forceinline__ void ray_step_m(const TraceParams& P, const MixedPara
     TurbCache tl;
     TurbCache& tc = TCACHE ? R.tc : tl;
     bool emits = false;
-    if (in_flow) emits = flow_begin<RADIO, TCACHE>(P, M.E, n.y0, n.y2, n.y4, n.y5, R.c.lam, R.c.E, hc, f, q, tc);
+    if (in_flow) emits = flow_begin<RADIO, TCACHE>(F, M.E, n.y0, n.y2, n.y4, n.y5, R.c.lam, R.c.E, hc, f, q, tc);
     // sin theta of the new state (FP64 1 - u^2, then FP32): the ring angle and the next step cap
     const float s1 = sqrtf_(fmaxf((float)(1.0 - n.y2 * n.y2), 0.f));
     if (RADIO) {
@@ -815,20 +820,20 @@ __device__ __forceinline__ void ray_step_m(const TraceParams& P, const MixedPara
     if ((R.s.y2 > 0.0) != (n.y2 > 0.0)) ++R.ncross;
     if (in_flow) {
         ++R.flow_steps;
-        if (emits && flow_finish<RADIO>(P, M.E, n.y0, n.y4, n.y5, f, q, tc)) {
+        if (emits && flow_finish<RADIO>(F, M.E, n.y0, n.y4, n.y5, f, q, tc)) {
             float ln_j, ln_a, ln_bnu;
-            if (M.use_surrogate) {
+            if (FM.use_surrogate) {
                 // the table's loads first; the exact formula runs while they are in flight, and the
                 // table replaces its values wherever the cell is trusted
                 SurrogateFetch sf;
-                surrogate_fetch(M.S, f.ln_nu - f.ln_nuc - (float)bhmlp::LN_2_9 - 2.f * f.ln_th - f.ln_sinb, f.ln_th,
+                surrogate_fetch(FM.S, f.ln_nu - f.ln_nuc - (float)bhmlp::LN_2_9 - 2.f * f.ln_th - f.ln_sinb, f.ln_th,
                                 f.ln_sinb, sf);
                 synchrotron_exact(M.E, f.ln_ne, f.ln_th, f.ln_k2, f.ln_nu, f.ln_nuc, f.ln_sinb, &ln_j, &ln_a, &ln_bnu);
                 if (sf.use) {
                     float fj, fa;
                     surrogate_blend(sf, &fj, &fa);
-                    ln_j = f.ln_ne + M.ln_e2_over_c + f.ln_nuc + fj;
-                    ln_a = f.ln_ne + M.ln_e2_over_mec - f.ln_nuc + fa;
+                    ln_j = f.ln_ne + FM.ln_e2_over_c + f.ln_nuc + fj;
+                    ln_a = f.ln_ne + FM.ln_e2_over_mec - f.ln_nuc + fa;
                     ln_bnu = ln_j - ln_a;   // both within the table's floors: no cancellation
                 }
             } else {
@@ -908,7 +913,7 @@ __device__ __forceinline__ int trace_ray_mixed(const TraceParams& P, const Mixed
                                                RayResult& out) {
     RayStateM R;
     ray_init_m<RADIO>(P, M, x, yv, R);
-    while (!R.done) ray_step_m<RADIO, TIME, false>(P, M, R);
+    while (!R.done) ray_step_m<RADIO, TIME, false>(P, M, P, M, R);
     return ray_result_m(P, R, out);
 }
 
