@@ -8,10 +8,12 @@
    keep about 16 significant bits of every operand, so BF16 rounding does not bound the surrogate's
    accuracy. The 3 -> 64 input layer and the 64 -> 2 output layer run on the FP32 VALU.
 
-   Work layout: one wave64 per workgroup; a wave processes tiles of 16 samples. MFMA operand layout
-   (16x16x16, wave64): A[i][k] lane i + 16*(k/4), element k % 4; B[k][j] lane j + 16*(k/4), element
-   k % 4; D[i][j] lane j + 16*(i/4), element i % 4. Activations go through LDS between layers to
-   change from the D layout to the A layout. */
+   Work layout: tiles of 16 samples, four waves per tile, each wave owning 16 columns of every layer.
+   MFMA operand layout (16x16x16, wave64): A[i][k] lane i + 16*(k/4), element k % 4; B[k][j] lane
+   j + 16*(k/4), element k % 4; D[i][j] lane j + 16*(i/4), element i % 4. The products are taken
+   transposed (weights as A, activations as B): a wave's result then has the layout that the next
+   product's B operand needs, so a layer is handed on through LDS as whole 16-byte fragments. The
+   weights stay in registers, each wave its own columns' share, loaded and split once. */
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -32,7 +34,7 @@ typedef float f4 __attribute__((ext_vector_type(4)));
 
 constexpr int TM = 16;           // samples per tile
 constexpr int LDA = NH + 4;      // padded row of an activation tile (floats)
-constexpr int LDW = NH + 8;      // padded row of a BF16 weight matrix (halves)
+constexpr int PSTRIDE = (NPARAM + 3) / 4 * 4;   // row of a partial gradient (floats): 16-byte aligned rows
 
 typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
 typedef float fl2 __attribute__((ext_vector_type(2)));
@@ -66,138 +68,120 @@ __device__ __forceinline__ f4 mfma3(s4 ah, s4 al, s4 bh, s4 bl, f4 c) {
 __device__ __forceinline__ float sigm(float z) {
     return __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-1.4426950408889634f * z));
 }
-__device__ __forceinline__ float silu(float z) { return z * sigm(z); }
-__device__ __forceinline__ float dsilu(float z) {
-    const float s = sigm(z);
-    return s * (1.f + z * (1.f - s));
+
+constexpr int TILE_WAVES = 4;    // waves per tile: wave w owns columns 16 w .. 16 w + 15 of every layer
+typedef unsigned int u4 __attribute__((ext_vector_type(4)));
+typedef u4 Frag[TILE_WAVES][64];     // B operands of the transposed products: (head, tail) per wave and lane
+
+// a D-layout fragment of the transposed activations as the next product's B operand
+__device__ __forceinline__ u4 pack_frag(const float v[4]) {
+    s4 h, l;
+    split4(v, h, l);
+    const u2 hh = __builtin_bit_cast(u2, h), ll = __builtin_bit_cast(u2, l);
+    return u4{hh[0], hh[1], ll[0], ll[1]};
+}
+__device__ __forceinline__ void unpack_frag(u4 f, s4& h, s4& l) {
+    h = __builtin_bit_cast(s4, (u2){f[0], f[1]});
+    l = __builtin_bit_cast(s4, (u2){f[2], f[3]});
 }
 
-struct alignas(16) WeightsLDS {   // 16-byte aligned: load_weights stores BF16 pairs as 32-bit words
-    unsigned short w2h[NH * LDW], w2l[NH * LDW], w3h[NH * LDW], w3l[NH * LDW];
+// A wave's 16 columns of a 64 x 64 matrix as A operands, split into head and tail: four steps of the
+// contraction. Forward: A[j][k] = W[k][16 w + j]; backward: A[k][j] = W[16 w + k][j].
+struct WFrag {
+    s4 h[4], l[4];
 };
-struct TileLDS {
-    float x[TM][4];
-    float z1[TM * LDA], h1[TM * LDA], z2[TM * LDA], h2[TM * LDA], z3[TM * LDA], h3[TM * LDA];
-    float g0[TM * LDA], g1[TM * LDA];   // back-propagated gradients (ping-pong)
-    float y[TM][2], t[TM][2], w[TM];
-};
-
-// split the FP32 master W2, W3 (row-major [k][j]) into BF16 head/tail arrays in LDS, two adjacent
-// j at a time (LDW is even, so each pair is one aligned 32-bit store)
-__device__ void load_weights(const float* __restrict__ P, WeightsLDS& W) {
-    for (int e = 2 * threadIdx.x; e < NH * NH; e += 2 * blockDim.x) {
-        const int k = e / NH, j = e % NH;
-        const float a0 = P[OFF_W2 + e], a1 = P[OFF_W2 + e + 1], b0 = P[OFF_W3 + e], b1 = P[OFF_W3 + e + 1];
-        const unsigned int ah = bf16x2(a0, a1), bh = bf16x2(b0, b1);
-        *(unsigned int*)&W.w2h[k * LDW + j] = ah;
-        *(unsigned int*)&W.w2l[k * LDW + j] = bf16x2(a0 - bf16_lo(ah), a1 - bf16_hi(ah));
-        *(unsigned int*)&W.w3h[k * LDW + j] = bh;
-        *(unsigned int*)&W.w3l[k * LDW + j] = bf16x2(b0 - bf16_lo(bh), b1 - bf16_hi(bh));
-    }
+__device__ __forceinline__ void load_fwd(const float* __restrict__ M, int w, int r, int g, WFrag& F) {
+    float v[4][4];
+    for (int kb = 0; kb < 4; ++kb)
+        for (int e = 0; e < 4; ++e) v[kb][e] = M[(16 * kb + 4 * g + e) * NH + 16 * w + r];
+    for (int kb = 0; kb < 4; ++kb) split4(v[kb], F.h[kb], F.l[kb]);
 }
-
-// D(16 x 64) = A(16 x 64, LDS rows of LDA floats) * W (64 x 64 BF16 head/tail, [k][j])
-__device__ __forceinline__ void gemm_fwd(const float* A, const unsigned short* Wh, const unsigned short* Wl, f4 acc[4]) {
-    const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
-    for (int jb = 0; jb < 4; ++jb) acc[jb] = f4{0.f, 0.f, 0.f, 0.f};
-    for (int kb = 0; kb < 4; ++kb) {
-        const int k0 = 16 * kb + 4 * g;
-        float av[4] = {A[r * LDA + k0], A[r * LDA + k0 + 1], A[r * LDA + k0 + 2], A[r * LDA + k0 + 3]};
-        s4 ah, al;
-        split4(av, ah, al);
-        for (int jb = 0; jb < 4; ++jb) {
-            const int j = 16 * jb + r;
-            s4 bh, bl;
-            for (int e = 0; e < 4; ++e) {
-                bh[e] = (short)Wh[(k0 + e) * LDW + j];
-                bl[e] = (short)Wl[(k0 + e) * LDW + j];
-            }
-            acc[jb] = mfma3(ah, al, bh, bl, acc[jb]);
-        }
-    }
-}
-
-// D(16 x 64)[i][k] = sum_j G[i][j] W[k][j]  (G: LDS rows of LDA floats; W: BF16 head/tail [k][j])
-__device__ __forceinline__ void gemm_bwd(const float* G, const unsigned short* Wh, const unsigned short* Wl, f4 acc[4]) {
-    const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
-    for (int kb = 0; kb < 4; ++kb) acc[kb] = f4{0.f, 0.f, 0.f, 0.f};
+__device__ __forceinline__ void load_bwd(const float* __restrict__ M, int w, int r, int g, WFrag& F) {
+    f4 v[4];
+    for (int jb = 0; jb < 4; ++jb) v[jb] = *(const f4*)&M[(16 * w + r) * NH + 16 * jb + 4 * g];
     for (int jb = 0; jb < 4; ++jb) {
-        const int j0 = 16 * jb + 4 * g;
-        float av[4] = {G[r * LDA + j0], G[r * LDA + j0 + 1], G[r * LDA + j0 + 2], G[r * LDA + j0 + 3]};
-        s4 ah, al;
-        split4(av, ah, al);
-        for (int kb = 0; kb < 4; ++kb) {
-            const int k = 16 * kb + r;
-            s4 bh, bl;
-            for (int e = 0; e < 4; ++e) {
-                bh[e] = (short)Wh[k * LDW + j0 + e];
-                bl[e] = (short)Wl[k * LDW + j0 + e];
-            }
-            acc[kb] = mfma3(ah, al, bh, bl, acc[kb]);
-        }
+        const float q[4] = {v[jb][0], v[jb][1], v[jb][2], v[jb][3]};
+        split4(q, F.h[jb], F.l[jb]);
     }
 }
 
-// gW[m][j] += sum_i H[i][m] G[i][j] over the 16 samples of a tile; gW in D layout [mb][jb]
-__device__ __forceinline__ void gemm_wgrad(const float* H, const float* G, f4 gW[4][4]) {
-    const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
-    s4 bh[4], bl[4];
+// The wave's 16 rows of (W^T or W) X^T, X^T from the fragments that the tile's four waves left. The
+// products are taken activation tail first, then the weight's, then the heads.
+__device__ __forceinline__ f4 gemm_t(const WFrag& W, const Frag& X, int lane) {
+    f4 acc = {0.f, 0.f, 0.f, 0.f};
+    for (int kb = 0; kb < 4; ++kb) {
+        s4 xh, xl;
+        unpack_frag(X[kb][lane], xh, xl);
+        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(W.h[kb], xl, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(W.l[kb], xh, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(W.h[kb], xh, acc, 0, 0, 0);
+    }
+    return acc;
+}
+
+// gW[m][j] = sum_i H[i][m] G[i][j] over a tile's 16 samples, m of the wave's 16 columns; D layout [jb]
+__device__ __forceinline__ void gemm_wgrad(const float* H, const float* G, int w, int r, int g, f4 gW[4]) {
+    float av[4];
+    for (int e = 0; e < 4; ++e) av[e] = H[(4 * g + e) * LDA + 16 * w + r];
+    s4 ah, al;
+    split4(av, ah, al);
     for (int jb = 0; jb < 4; ++jb) {
         float bv[4];
         for (int e = 0; e < 4; ++e) bv[e] = G[(4 * g + e) * LDA + 16 * jb + r];
-        split4(bv, bh[jb], bl[jb]);
-    }
-    for (int mb = 0; mb < 4; ++mb) {
-        float av[4];
-        for (int e = 0; e < 4; ++e) av[e] = H[(4 * g + e) * LDA + 16 * mb + r];
-        s4 ah, al;
-        split4(av, ah, al);
-        for (int jb = 0; jb < 4; ++jb) gW[mb][jb] = mfma3(ah, al, bh[jb], bl[jb], gW[mb][jb]);
+        s4 bh, bl;
+        split4(bv, bh, bl);
+        gW[jb] = mfma3(ah, al, bh, bl, f4{0.f, 0.f, 0.f, 0.f});
     }
 }
 
-// store a D-layout 16 x 64 result (+ bias) to LDS as pre-activation Z and activation H
-__device__ __forceinline__ void store_act(const f4 acc[4], const float* __restrict__ bias, float* Z, float* Hh) {
-    const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
-    for (int jb = 0; jb < 4; ++jb)
-        for (int e = 0; e < 4; ++e) {
-            const int i = 4 * g + e, j = 16 * jb + r;
-            const float z = acc[jb][e] + bias[j];
-            Z[i * LDA + j] = z;
-            Hh[i * LDA + j] = silu(z);
-        }
+// silu and its derivative from one sigmoid
+__device__ __forceinline__ void act4(const f4 z, float h[4], float d[4]) {
+    for (int e = 0; e < 4; ++e) {
+        const float s = sigm(z[e]);
+        h[e] = z[e] * s;
+        d[e] = s * (1.f + z[e] * (1.f - s));
+    }
 }
 
-// forward pass of one tile whose normalised inputs are in T.x; leaves Z1..3, H1..3, y in LDS
-__device__ void forward_tile(const float* __restrict__ P, const WeightsLDS& W, TileLDS& T) {
-    const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
-    // layer 1 (FP32): lane owns (i = 4g + e, j = 16 jb + r)
-    for (int jb = 0; jb < 4; ++jb) {
-        const int j = 16 * jb + r;
-        const float w0 = P[OFF_W1 + j], w1 = P[OFF_W1 + NH + j], w2 = P[OFF_W1 + 2 * NH + j], b = P[OFF_B1 + j];
-        for (int e = 0; e < 4; ++e) {
-            const int i = 4 * g + e;
-            const float z = b + T.x[i][0] * w0 + T.x[i][1] * w1 + T.x[i][2] * w2;
-            T.z1[i * LDA + j] = z;
-            T.h1[i * LDA + j] = silu(z);
-        }
+// the lane's four columns of row i of an FP32 tile
+__device__ __forceinline__ void put_row(float* X, int i, int j, const float v[4]) {
+    *(f4*)&X[i * LDA + j] = f4{v[0], v[1], v[2], v[3]};
+}
+
+// A wave's share of the network in the forward direction, in registers
+struct FwdWeights {
+    f4 w1[3], b1, b2, b3;
+    WFrag W2, W3;
+};
+__device__ __forceinline__ void load_forward(const float* __restrict__ P, int w, int r, int g, FwdWeights& F) {
+    const int j = 16 * w + 4 * g;
+    for (int k = 0; k < 3; ++k) F.w1[k] = *(const f4*)&P[OFF_W1 + k * NH + j];
+    F.b1 = *(const f4*)&P[OFF_B1 + j];
+    F.b2 = *(const f4*)&P[OFF_B2 + j];
+    F.b3 = *(const f4*)&P[OFF_B3 + j];
+    load_fwd(P + OFF_W2, w, r, g, F.W2);
+    load_fwd(P + OFF_W3, w, r, g, F.W3);
+}
+__device__ __forceinline__ f4 layer1(const FwdWeights& F, const float x[3]) {
+    f4 z;
+    for (int e = 0; e < 4; ++e) z[e] = F.b1[e] + x[0] * F.w1[0][e] + x[1] * F.w1[1][e] + x[2] * F.w1[2][e];
+    return z;
+}
+
+// The output layer's 64 weights of each output, and its 32 sums (one per lane 0..31 of a tile's first wave)
+struct alignas(16) OutLayer {
+    float w[NOUT][NH];
+};
+__device__ __forceinline__ void load_out(const float* __restrict__ P, OutLayer& O) {
+    for (int q = threadIdx.x; q < NH * NOUT; q += blockDim.x) O.w[q % NOUT][q / NOUT] = P[OFF_W4 + q];
+}
+__device__ __forceinline__ float out_sum(float b4, const OutLayer& O, const float* X, int i, int o) {
+    float y = b4;
+    for (int k = 0; k < NH; k += 4) {
+        const f4 h = *(const f4*)&X[i * LDA + k], w = *(const f4*)&O.w[o][k];
+        for (int e = 0; e < 4; ++e) y += h[e] * w[e];
     }
-    __syncthreads();
-    f4 acc[4];
-    gemm_fwd(T.h1, W.w2h, W.w2l, acc);
-    store_act(acc, P + OFF_B2, T.z2, T.h2);
-    __syncthreads();
-    gemm_fwd(T.h2, W.w3h, W.w3l, acc);
-    store_act(acc, P + OFF_B3, T.z3, T.h3);
-    __syncthreads();
-    // layer 4 (FP32): lanes 0..31 own (i = lane / 2, o = lane % 2)
-    if (lane < 2 * TM) {
-        const int i = lane >> 1, o = lane & 1;
-        float y = P[OFF_B4 + o];
-        for (int k = 0; k < NH; ++k) y += T.h3[i * LDA + k] * P[OFF_W4 + k * NOUT + o];
-        T.y[i][o] = y;
-    }
-    __syncthreads();
+    return y;
 }
 
 __device__ __forceinline__ uint64_t splitmix(uint64_t x) {
@@ -260,143 +244,180 @@ __global__ __launch_bounds__(256) void k_mlp_sample(uint64_t seed, int n, const 
     ws[i] = 1.f + hot_weight / (1.f + expf(-(float)(fj + 12.0)));
 }
 
-// Gradient workgroups: GRAD_WAVES waves share one copy of the split weights in LDS, and each wave
-// takes GRAD_TILES 16-sample tiles with its own activation buffers (36 KB of weights + 35 KB per
-// wave). The default batch of 8192 samples is then 256 workgroups, one per CU with two busy SIMDs.
-// Measured per training step with one wave per workgroup: 4 tiles 104 us (half the CUs idle),
-// 2 tiles 83 us, 1 tile 92 us (twice the weight loads and partial gradients to reduce).
-constexpr int GRAD_WAVES = 2, GRAD_TILES = 1;
-static_assert(GRAD_WAVES == 2, "k_mlp_grad combines the partial gradients of exactly two waves");
+// One training step is a chain of small products, so its time is latency: the longest chain of one tile,
+// not the matrix rate (1.3 GFLOP). Four waves share a tile, so each runs a quarter of every product, and the
+// weight gradients, which nothing waits for, come after the chain. Two tiles per workgroup: the default
+// batch of 8192 samples is 256 workgroups, one per CU with two waves per SIMD. Per step of that batch:
+// one wave per tile with the split weights in LDS, read 2 bytes at a time: 26.7 us; this one 13.6. Beyond
+// the chain that is the first touch of weights and samples, and the 8.9 MB of partial gradients.
+constexpr int GRAD_TILES = 2, GRAD_BLOCK = 64 * TILE_WAVES * GRAD_TILES;
+static_assert(GRAD_TILES == 2, "the two tiles' halves add the partial gradient of one matrix each");
 
-/* One training step's gradient over `count` samples starting at `first` (indices mod n): each
-   workgroup (one wave) takes `tiles` consecutive 16-sample tiles and writes its partial gradient
-   (8706 floats) and partial loss. Loss = sum_i w_i |y_i - t_i|^2 / count on normalised outputs. */
-// The partial gradient held by one lane, visited in the parameter layout: f(index, value)
-template <typename F>
-__device__ __forceinline__ void for_partial(int lane, const float gW1[3], float gb1, float gb2, float gb3,
-                                            const float gW4[2], float gb4, const f4 gW2[4][4], const f4 gW3[4][4],
-                                            F f) {
-    const int r = lane & 15, g = lane >> 4;
-    for (int k = 0; k < 3; ++k) f(OFF_W1 + k * NH + lane, gW1[k]);
-    f(OFF_B1 + lane, gb1);
-    f(OFF_B2 + lane, gb2);
-    f(OFF_B3 + lane, gb3);
-    f(OFF_W4 + lane * NOUT, gW4[0]);
-    f(OFF_W4 + lane * NOUT + 1, gW4[1]);
-    if (lane < 2) f(OFF_B4 + lane, gb4);
-    for (int mb = 0; mb < 4; ++mb)
-        for (int jb = 0; jb < 4; ++jb)
-            for (int e = 0; e < 4; ++e) {
-                const int m = 16 * mb + 4 * g + e, j = 16 * jb + r;
-                f(OFF_W2 + m * NH + j, gW2[mb][jb][e]);
-                f(OFF_W3 + m * NH + j, gW3[mb][jb][e]);
-            }
+struct alignas(16) GradTile {
+    float h1[TM * LDA], h2[TM * LDA], h3[TM * LDA];    // activations
+    float g1[TM * LDA], g2[TM * LDA], g3[TM * LDA];    // gradients by the pre-activations
+    Frag f1, f2;                                       // fragments, by turns
+    float x[TM][4], dy[TM][2];
+};
+
+// Row index of a partial gradient: everything but W2 and W3 lies as in the parameters; each of W2 and W3
+// as a lane holds it (wave, jb, lane, e), so that the partials are stored and added 16 bytes at a time.
+__device__ __forceinline__ int partial_param(int q) {
+    const int off = q >= OFF_W3 && q < OFF_B3 ? OFF_W3 : OFF_W2;
+    if (q < OFF_W2 || q >= OFF_B3 || (q >= OFF_B2 && q < OFF_W3)) return q;
+    const int v = q - off, e = v & 3, lane = (v >> 2) & 63, jb = (v >> 8) & 3, w = v >> 10;
+    return off + (16 * w + 4 * (lane >> 4) + e) * NH + 16 * jb + (lane & 15);
 }
 
-__global__ __launch_bounds__(64 * GRAD_WAVES) void k_mlp_grad(const float* __restrict__ P, Norm N, const float* __restrict__ xs,
+/* One training step's gradient over `count` samples starting at `first` (indices mod n): each
+   workgroup takes two consecutive 16-sample tiles and writes the sum of their partial gradients
+   (8706 floats, rows as partial_param) and of their losses.
+   Loss = sum_i w_i |y_i - t_i|^2 / count on normalised outputs. */
+__global__ __launch_bounds__(GRAD_BLOCK) void k_mlp_grad(const float* __restrict__ P, Norm N, const float* __restrict__ xs,
                                                  const float* __restrict__ ts, const float* __restrict__ ws, int n,
-                                                 int first, int count, int tiles, float* __restrict__ partial,
+                                                 int first, int count, float* __restrict__ partial,
                                                  float* __restrict__ loss_partial) {
-    __shared__ WeightsLDS W;
-    __shared__ TileLDS TT[GRAD_WAVES];
-    __shared__ float wave_loss[GRAD_WAVES];
-    const int wave = threadIdx.x >> 6;
-    TileLDS& T = TT[wave];
+    __shared__ GradTile TT[GRAD_TILES];
+    __shared__ OutLayer O;
+    __shared__ f4 swap[GRAD_TILES][4 * 64 * TILE_WAVES];   // a tile's gradient of the other tile's matrix
+    __shared__ float small[2 * NH + 2 * NH + NIN * NH + NH * NOUT];
+    __shared__ float tile_loss[GRAD_TILES], small4[NOUT];
+    const int tile = threadIdx.x / (64 * TILE_WAVES), w = (threadIdx.x >> 6) & (TILE_WAVES - 1);
+    GradTile& T = TT[tile];
     const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
-    load_weights(P, W);
-    __syncthreads();
-    f4 gW2[4][4], gW3[4][4];
-    for (int a = 0; a < 4; ++a)
-        for (int b = 0; b < 4; ++b) gW2[a][b] = gW3[a][b] = f4{0.f, 0.f, 0.f, 0.f};
-    float gW1[3] = {0.f, 0.f, 0.f}, gb1 = 0.f, gb2 = 0.f, gb3 = 0.f, gW4[2] = {0.f, 0.f}, gb4 = 0.f, loss = 0.f;
+    const int col = 16 * w + 4 * g;        // the lane's four columns of sample r
     const float inv_count = 1.f / (float)count;
-    for (int tl = 0; tl < tiles; ++tl) {
-        const int base = ((blockIdx.x * GRAD_WAVES + wave) * tiles + tl) * TM;   // sample offset in the batch
-        if (lane < TM) {
-            const int s = lane;
-            const bool in = base + s < count;
-            const size_t idx = (size_t)((first + base + s) % n);
-            for (int k = 0; k < 3; ++k) T.x[s][k] = in ? xs[3 * idx + k] : 0.f;
-            T.t[s][0] = in ? (ts[2 * idx] - N.y_mu[0]) / N.y_sd[0] : 0.f;
-            T.t[s][1] = in ? (ts[2 * idx + 1] - N.y_mu[1]) / N.y_sd[1] : 0.f;
-            T.w[s] = in ? ws[idx] : 0.f;
-        }
-        __syncthreads();
-        forward_tile(P, W, T);
-        // loss gradient dY (normalised outputs), lanes 0..31
-        if (lane < 2 * TM) {
-            const int i = lane >> 1, o = lane & 1;
-            const float d = T.y[i][o] - T.t[i][o];
-            loss += T.w[i] * d * d * inv_count;
-            T.y[i][o] = 2.f * T.w[i] * d * inv_count;   // reuse y as dY
-        }
-        __syncthreads();
-        // layer 4: lane k owns W4[k][0..1]; dZ3[i][k] = (sum_o dY[i][o] W4[k][o]) silu'(Z3[i][k])
-        {
-            const int k = lane;
-            const float w40 = P[OFF_W4 + k * NOUT], w41 = P[OFF_W4 + k * NOUT + 1];
-            for (int i = 0; i < TM; ++i) {
-                const float dy0 = T.y[i][0], dy1 = T.y[i][1];
-                gW4[0] += T.h3[i * LDA + k] * dy0;
-                gW4[1] += T.h3[i * LDA + k] * dy1;
-                T.g0[i * LDA + k] = (dy0 * w40 + dy1 * w41) * dsilu(T.z3[i * LDA + k]);
-            }
-            if (lane < 2)
-                for (int i = 0; i < TM; ++i) gb4 += T.y[i][lane];
-        }
-        __syncthreads();
-        // layer 3
-        gemm_wgrad(T.h2, T.g0, gW3);
-        for (int i = 0; i < TM; ++i) gb3 += T.g0[i * LDA + lane];
-        f4 acc[4];
-        gemm_bwd(T.g0, W.w3h, W.w3l, acc);
-        for (int kb = 0; kb < 4; ++kb)
-            for (int e = 0; e < 4; ++e) {
-                const int i = 4 * g + e, k = 16 * kb + r;
-                T.g1[i * LDA + k] = acc[kb][e] * dsilu(T.z2[i * LDA + k]);
-            }
-        __syncthreads();
-        // layer 2
-        gemm_wgrad(T.h1, T.g1, gW2);
-        for (int i = 0; i < TM; ++i) gb2 += T.g1[i * LDA + lane];
-        gemm_bwd(T.g1, W.w2h, W.w2l, acc);
-        __syncthreads();   // every lane has read g0's predecessor data; g0 is reused below
-        for (int kb = 0; kb < 4; ++kb)
-            for (int e = 0; e < 4; ++e) {
-                const int i = 4 * g + e, k = 16 * kb + r;
-                T.g0[i * LDA + k] = acc[kb][e] * dsilu(T.z1[i * LDA + k]);
-            }
-        __syncthreads();
-        // layer 1: lane j owns W1[0..2][j], b1[j]
-        for (int i = 0; i < TM; ++i) {
-            const float d = T.g0[i * LDA + lane];
-            gW1[0] += T.x[i][0] * d;
-            gW1[1] += T.x[i][1] * d;
-            gW1[2] += T.x[i][2] * d;
-            gb1 += d;
-        }
-        __syncthreads();
+    const int base = (blockIdx.x * GRAD_TILES + tile) * TM;   // sample offset in the batch
+    // the lane's sample, and on the first wave the target and weight of its output sum
+    float x[3];
+    {
+        const bool in = base + r < count;
+        const size_t idx = (size_t)((first + base + r) % n);
+        for (int k = 0; k < 3; ++k) x[k] = in ? xs[3 * idx + k] : 0.f;
     }
-    // the workgroup's partial gradient: wave 1 leaves its sums in its own (no longer used) tile
-    // buffer, wave 0 adds them to its own and writes the result, always in that order
-    for (int off = 32; off > 0; off >>= 1) loss += __shfl_down(loss, off, 64);
-    if (lane == 0) wave_loss[wave] = loss;
+    const int oi = (lane >> 1) & 15, oo = lane & 1;
+    float tgt = 0.f, wgt = 0.f, b4 = 0.f;
+    if (w == 0) {
+        const bool in = base + oi < count;
+        const size_t idx = (size_t)((first + base + oi) % n);
+        tgt = in ? (ts[2 * idx + oo] - N.y_mu[oo]) / N.y_sd[oo] : 0.f;
+        wgt = in ? ws[idx] : 0.f;
+        b4 = P[OFF_B4 + oo];
+    }
+    FwdWeights F;
+    load_forward(P, w, r, g, F);
+    WFrag B2, B3;
+    load_bwd(P + OFF_W3, w, r, g, B3);
+    load_bwd(P + OFF_W2, w, r, g, B2);
+    float w4[4][2];
+    for (int e = 0; e < 4; ++e)
+        for (int o = 0; o < 2; ++o) w4[e][o] = P[OFF_W4 + (col + e) * NOUT + o];
+    load_out(P, O);
+    if (w == 0 && g == 0)
+        for (int k = 0; k < 3; ++k) T.x[r][k] = x[k];
+    // forward
+    float h[4], d1[4], d2[4], d3[4];
+    act4(layer1(F, x), h, d1);
+    T.f1[w][lane] = pack_frag(h);
+    put_row(T.h1, r, col, h);
     __syncthreads();
-    float* red = reinterpret_cast<float*>(&TT[1]);
-    static_assert(sizeof(TileLDS) >= sizeof(float) * NPARAM, "a tile buffer holds a partial gradient");
-    if (wave == 1) for_partial(lane, gW1, gb1, gb2, gb3, gW4, gb4, gW2, gW3, [&](int i, float v) { red[i] = v; });
+    act4(gemm_t(F.W2, T.f1, lane) + F.b2, h, d2);
+    T.f2[w][lane] = pack_frag(h);
+    put_row(T.h2, r, col, h);
     __syncthreads();
-    if (wave == 0) {
-        float* out = partial + (size_t)blockIdx.x * NPARAM;
-        for_partial(lane, gW1, gb1, gb2, gb3, gW4, gb4, gW2, gW3, [&](int i, float v) { out[i] = v + red[i]; });
-        if (lane == 0) loss_partial[blockIdx.x] = wave_loss[0] + wave_loss[1];
+    act4(gemm_t(F.W3, T.f2, lane) + F.b3, h, d3);
+    put_row(T.h3, r, col, h);
+    __syncthreads();
+    // outputs, loss and its gradient: lanes 0..31 of the tile's first wave
+    if (w == 0) {
+        float loss = 0.f;
+        if (lane < 2 * TM) {
+            const float d = out_sum(b4, O, T.h3, oi, oo) - tgt;
+            loss += wgt * d * d * inv_count;
+            T.dy[oi][oo] = 2.f * wgt * d * inv_count;
+        }
+        for (int off = 32; off > 0; off >>= 1) loss += __shfl_down(loss, off, 64);
+        if (lane == 0) tile_loss[tile] = loss;
+    }
+    __syncthreads();
+    // backward: the chain first
+    float q[4];
+    {
+        const float dy0 = T.dy[r][0], dy1 = T.dy[r][1];
+        for (int e = 0; e < 4; ++e) q[e] = (dy0 * w4[e][0] + dy1 * w4[e][1]) * d3[e];
+    }
+    T.f1[w][lane] = pack_frag(q);
+    put_row(T.g3, r, col, q);
+    __syncthreads();
+    {
+        const f4 a = gemm_t(B3, T.f1, lane);
+        for (int e = 0; e < 4; ++e) q[e] = a[e] * d2[e];
+    }
+    T.f2[w][lane] = pack_frag(q);
+    put_row(T.g2, r, col, q);
+    __syncthreads();
+    {
+        const f4 a = gemm_t(B2, T.f2, lane);
+        for (int e = 0; e < 4; ++e) q[e] = a[e] * d1[e];
+    }
+    put_row(T.g1, r, col, q);
+    // the weight gradients: this tile's of the other tile's matrix first
+    f4 gW2[4], gW3[4];
+    gemm_wgrad(T.h2, T.g3, w, r, g, gW3);
+    gemm_wgrad(T.h1, T.g2, w, r, g, gW2);
+    for (int jb = 0; jb < 4; ++jb) swap[tile][(w * 4 + jb) * 64 + lane] = tile == 0 ? gW3[jb] : gW2[jb];
+    __syncthreads();
+    // the vectors' gradients, a share per wave: lane = column, sums over the samples in order
+    float v0 = 0.f, v1 = 0.f, v2 = 0.f;
+    if (w < 2) {
+        for (int i = 0; i < TM; ++i) v0 += T.h3[i * LDA + lane] * T.dy[i][w];            // W4[lane][w]
+        const float* G = w == 0 ? T.g3 : T.g2;
+        for (int i = 0; i < TM; ++i) v1 += G[i * LDA + lane];                            // b3, b2
+        if (w == 0 && lane < 2)
+            for (int i = 0; i < TM; ++i) v2 += T.dy[i][lane];                            // b4
+    } else if (w == 2) {
+        for (int i = 0; i < TM; ++i) {
+            const float d = T.g1[i * LDA + lane];
+            v0 += T.x[i][0] * d;
+            v1 += T.x[i][1] * d;
+        }
+    } else {
+        for (int i = 0; i < TM; ++i) {
+            const float d = T.g1[i * LDA + lane];
+            v0 += T.x[i][2] * d;
+            v1 += d;
+        }
+    }
+    // tile 1 hands its vectors over; tile 0 adds and stores them. Each tile adds and stores one matrix.
+    constexpr int S_W4 = 0, S_B3 = 2 * NH, S_B2 = 3 * NH, S_W1 = 4 * NH, S_B1 = 7 * NH;
+    const int i0 = w < 2 ? S_W4 + w * NH : S_W1 + (w == 2 ? 0 : 2) * NH;
+    const int i1 = w == 0 ? S_B3 : w == 1 ? S_B2 : w == 2 ? S_W1 + NH : S_B1;
+    if (tile == 1) {
+        small[i0 + lane] = v0;
+        small[i1 + lane] = v1;
+        if (w == 0 && lane < 2) small4[lane] = v2;
+    }
+    float* out = partial + (size_t)blockIdx.x * PSTRIDE;
+    for (int jb = 0; jb < 4; ++jb) {
+        const int k = (w * 4 + jb) * 64 + lane;
+        const f4 own = tile == 0 ? gW2[jb] : gW3[jb], other = swap[1 - tile][k];
+        *(f4*)&out[(tile == 0 ? OFF_W2 : OFF_W3) + 4 * k] = own + other;
+    }
+    __syncthreads();
+    if (tile == 0) {
+        const int p0 = w < 2 ? OFF_W4 + lane * NOUT + w : OFF_W1 + (w == 2 ? 0 : 2) * NH + lane;
+        const int p1 = (w == 0 ? OFF_B3 : w == 1 ? OFF_B2 : w == 2 ? OFF_W1 + NH : OFF_B1) + lane;
+        out[p0] = v0 + small[i0 + lane];
+        out[p1] = v1 + small[i1 + lane];
+        if (w == 0 && lane < 2) out[OFF_B4 + lane] = v2 + small4[lane];
+        if (threadIdx.x == 0) loss_partial[blockIdx.x] = tile_loss[0] + tile_loss[1];
     }
 }
 
 // grad[p] = sum over workgroups of partial[w][p]; loss likewise. A workgroup takes 64 parameters; its
 // eight waves each sum an eighth of the workgroups' partials (w = q, q + 8, ...) in eight running
-// sums (eight independent loads in flight), and the eighths are added through LDS. Every sum is
-// taken in a fixed order, so the result does not depend on timing.
+// sums, and the eighths are added through LDS. Every sum is taken in a fixed order, so the result
+// does not depend on timing. 256 partials: four rounds of eight loads, all in flight at once: 6.6 -> 4.9 us.
 // With P set, the same lane then takes the Adam step of its parameter (bias-corrected moments).
 struct AdamStep {
     float* P;   // nullptr: gradient only
@@ -413,13 +434,14 @@ __global__ __launch_bounds__(RED_BLOCK) void k_mlp_reduce(const float* __restric
     __shared__ float part_sum[RED_SPLIT][RED_PARAMS];
     static_assert(RED_SPLIT == 8, "the final sum below adds eight parts");
     const int lp = threadIdx.x % RED_PARAMS, qt = threadIdx.x / RED_PARAMS;
-    const int p = blockIdx.x * RED_PARAMS + lp;
+    const int row = blockIdx.x * RED_PARAMS + lp, p = partial_param(row);
     float total = 0.f;
     if (p < NPARAM) {
-        constexpr size_t STEP = (size_t)RED_SPLIT * NPARAM;   // between this group's rows
+        constexpr size_t STEP = (size_t)RED_SPLIT * PSTRIDE;   // between this group's rows
         float s0 = 0.f, s1 = 0.f, s2 = 0.f, s3 = 0.f, s4 = 0.f, s5 = 0.f, s6 = 0.f, s7 = 0.f, sr = 0.f;
-        const float* q = partial + (size_t)qt * NPARAM + p;
+        const float* q = partial + (size_t)qt * PSTRIDE + row;
         int w = qt;
+#pragma unroll 4
         for (; w + 7 * RED_SPLIT < nw; w += 8 * RED_SPLIT, q += 8 * STEP) {
             s0 += q[0];
             s1 += q[STEP];
@@ -455,23 +477,33 @@ __global__ __launch_bounds__(RED_BLOCK) void k_mlp_reduce(const float* __restric
 }
 
 
+constexpr int INFER_GRID = 2048;   // persistent workgroups of the inference, eight per CU
+
 /* Inference: n samples of raw inputs (u0, Theta, theta_B) or, with lattice != 0, the nodes of the
    (n0 x n1 x n2) lattice over (u0, log10 Theta, theta_B in [lo2, hi2]); writes (ln f_j, ln f_a). */
 struct Lattice {
     int n0, n1, n2;
     float lo0, lo1, lo2, d0, d1, d2;
 };
-__global__ __launch_bounds__(64) void k_mlp_infer(const float* __restrict__ P, Norm N, const float* __restrict__ in,
-                                                  int n, int lattice, Lattice L, float2* __restrict__ out) {
-    __shared__ WeightsLDS W;
-    __shared__ TileLDS T;
-    const int lane = threadIdx.x & 63;
-    load_weights(P, W);
-    __syncthreads();
+// Four waves per tile as in the training step, the weights in registers over all of a workgroup's tiles.
+// 200 003 points: one wave per tile with the split weights in LDS 215 us, this one 39 us.
+__global__ __launch_bounds__(64 * TILE_WAVES) void k_mlp_infer(const float* __restrict__ P, Norm N,
+                                                  const float* __restrict__ in, int n, int lattice, Lattice L,
+                                                  float* __restrict__ out) {
+    __shared__ Frag f1, f2;
+    __shared__ alignas(16) float h3[TM * LDA];
+    __shared__ OutLayer O;
+    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+    FwdWeights F;
+    load_forward(P, w, r, g, F);
+    load_out(P, O);
+    const int oi = lane >> 1, oo = lane & 1;
+    const float b4 = P[OFF_B4 + oo];
     const int ntiles = (n + TM - 1) / TM;
     for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-        if (lane < TM) {
-            const int s = tile * TM + lane;
+        float x[3];
+        {
+            const int s = tile * TM + r;
             float sc[3] = {0.f, 0.f, 0.f};   // surrogate coordinates
             if (s < n) {
                 if (lattice) {
@@ -487,15 +519,25 @@ __global__ __launch_bounds__(64) void k_mlp_infer(const float* __restrict__ P, N
                     sc[2] = ls;
                 }
             }
-            for (int k = 0; k < 3; ++k) T.x[lane][k] = (sc[k] - N.x_c[k]) / N.x_h[k];
+            for (int k = 0; k < 3; ++k) x[k] = (sc[k] - N.x_c[k]) / N.x_h[k];
         }
+        // every buffer is written behind a barrier that its readers in the tile before have passed: f1
+        // behind that tile's second and third, f2 and h3 behind this tile's first and second
+        float h[4], d[4];
+        act4(layer1(F, x), h, d);
+        f1[w][lane] = pack_frag(h);
         __syncthreads();
-        forward_tile(P, W, T);
-        if (lane < TM) {
-            const int s = tile * TM + lane;
-            if (s < n) out[s] = make_float2(T.y[lane][0] * N.y_sd[0] + N.y_mu[0], T.y[lane][1] * N.y_sd[1] + N.y_mu[1]);
+        act4(gemm_t(F.W2, f1, lane) + F.b2, h, d);
+        f2[w][lane] = pack_frag(h);
+        __syncthreads();
+        act4(gemm_t(F.W3, f2, lane) + F.b3, h, d);
+        put_row(h3, r, 16 * w + 4 * g, h);
+        __syncthreads();
+        if (w == 0 && lane < 2 * TM) {
+            const int s = tile * TM + oi;
+            const float y = out_sum(b4, O, h3, oi, oo);
+            if (s < n) out[2 * (size_t)s + oo] = y * N.y_sd[oo] + N.y_mu[oo];
         }
-        __syncthreads();
     }
 }
 
@@ -659,8 +701,7 @@ int bh_mlp_train(bh_ctx* c, const bh_mlp_train_cfg* cfg_in, bh_mlp_report* rep) 
     const int n = cfg.n_samples;
     float *xs = nullptr, *ts = nullptr, *ws = nullptr, *partial = nullptr, *lpart = nullptr, *grad = nullptr,
           *loss = nullptr;
-    const int tiles = GRAD_TILES;
-    const int nwg = (cfg.batch / TM + tiles * GRAD_WAVES - 1) / (tiles * GRAD_WAVES);
+    const int nwg = (cfg.batch / TM + GRAD_TILES - 1) / GRAD_TILES;
     auto cleanup = [&]() {
         for (float* p : {xs, ts, ws, partial, lpart, grad, loss})
             if (p) (void)hipFree(p);
@@ -669,7 +710,7 @@ int bh_mlp_train(bh_ctx* c, const bh_mlp_train_cfg* cfg_in, bh_mlp_report* rep) 
     if (hipMalloc((void**)&xs, sizeof(float) * 3 * (size_t)n) != hipSuccess ||
         hipMalloc((void**)&ts, sizeof(float) * 2 * (size_t)n) != hipSuccess ||
         hipMalloc((void**)&ws, sizeof(float) * (size_t)n) != hipSuccess ||
-        hipMalloc((void**)&partial, sizeof(float) * NPARAM * (size_t)nwg) != hipSuccess ||
+        hipMalloc((void**)&partial, sizeof(float) * PSTRIDE * (size_t)nwg) != hipSuccess ||
         hipMalloc((void**)&lpart, sizeof(float) * nwg) != hipSuccess ||
         hipMalloc((void**)&grad, sizeof(float) * NPARAM) != hipSuccess ||
         hipMalloc((void**)&loss, sizeof(float)) != hipSuccess) {
@@ -714,9 +755,8 @@ int bh_mlp_train(bh_ctx* c, const bh_mlp_train_cfg* cfg_in, bh_mlp_report* rep) 
     float first_loss = -1.f, last_loss = -1.f;
     for (int step = 0; step < total; ++step) {
         const int first = (int)(((long long)step * cfg.batch) % n);
-        hipLaunchKernelGGL(k_mlp_grad, dim3(nwg), dim3(64 * GRAD_WAVES), 0, c->st, c->d_mlp, N, xs, ts, ws, n, first,
-                           cfg.batch,
-                           tiles, partial, lpart);
+        hipLaunchKernelGGL(k_mlp_grad, dim3(nwg), dim3(GRAD_BLOCK), 0, c->st, c->d_mlp, N, xs, ts, ws, n, first,
+                           cfg.batch, partial, lpart);
         const double prog = (double)step / std::max(total - 1, 1);
         const float lr = (float)(cfg.lr_min + 0.5 * (cfg.lr - cfg.lr_min) * (1.0 + std::cos(3.141592653589793 * prog)));
         const float bc1 = (float)(1.0 - std::pow(0.9, step + 1)), bc2 = (float)(1.0 - std::pow(0.999, step + 1));
@@ -799,8 +839,8 @@ int bh_mlp_infer(bh_ctx* c, const float* in, int n, float* out) {
     } else {
         const int ntiles = (n + TM - 1) / TM;
         Lattice L{};
-        hipLaunchKernelGGL(k_mlp_infer, dim3(std::min(ntiles, 4096)), dim3(64), 0, c->st, c->d_mlp, c->mlp_norm, din,
-                           n, 0, L, dout);
+        hipLaunchKernelGGL(k_mlp_infer, dim3(std::min(ntiles, INFER_GRID)), dim3(64 * TILE_WAVES), 0, c->st, c->d_mlp,
+                           c->mlp_norm, din, n, 0, L, (float*)dout);
         if (hipGetLastError() != hipSuccess ||
             hipMemcpyAsync(out, dout, sizeof(float2) * (size_t)n, hipMemcpyDeviceToHost, c->st) != hipSuccess ||
             hipStreamSynchronize(c->st) != hipSuccess)
@@ -846,7 +886,7 @@ int bh_mlp_grad(bh_ctx* c, const float* params, const float* norm, const float* 
     if (!c || !params || !norm || !xn || !tn || !w || !grad_out || n <= 0 || n % TM != 0) return BH_ERR_ARG;
     MCK(c, hipSetDevice(c->device));
     const Norm N = norm_from_floats(norm);
-    const int tiles = GRAD_TILES, nwg = (n / TM + tiles * GRAD_WAVES - 1) / (tiles * GRAD_WAVES);
+    const int nwg = (n / TM + GRAD_TILES - 1) / GRAD_TILES;
     float *dp = nullptr, *dx = nullptr, *dt = nullptr, *dw = nullptr, *part = nullptr, *lp = nullptr, *g = nullptr,
           *l = nullptr;
     int rc = BH_OK;
@@ -854,7 +894,7 @@ int bh_mlp_grad(bh_ctx* c, const float* params, const float* norm, const float* 
         hipMalloc((void**)&dx, sizeof(float) * 3 * (size_t)n) != hipSuccess ||
         hipMalloc((void**)&dt, sizeof(float) * 2 * (size_t)n) != hipSuccess ||
         hipMalloc((void**)&dw, sizeof(float) * (size_t)n) != hipSuccess ||
-        hipMalloc((void**)&part, sizeof(float) * NPARAM * (size_t)nwg) != hipSuccess ||
+        hipMalloc((void**)&part, sizeof(float) * PSTRIDE * (size_t)nwg) != hipSuccess ||
         hipMalloc((void**)&lp, sizeof(float) * nwg) != hipSuccess ||
         hipMalloc((void**)&g, sizeof(float) * NPARAM) != hipSuccess || hipMalloc((void**)&l, sizeof(float)) != hipSuccess ||
         hipMemcpy(dp, params, sizeof(float) * NPARAM, hipMemcpyHostToDevice) != hipSuccess ||
@@ -863,8 +903,7 @@ int bh_mlp_grad(bh_ctx* c, const float* params, const float* norm, const float* 
         hipMemcpy(dw, w, sizeof(float) * (size_t)n, hipMemcpyHostToDevice) != hipSuccess) {
         rc = BH_ERR_HIP;
     } else {
-        hipLaunchKernelGGL(k_mlp_grad, dim3(nwg), dim3(64 * GRAD_WAVES), 0, c->st, dp, N, dx, dt, dw, n, 0, n, tiles,
-                           part, lp);
+        hipLaunchKernelGGL(k_mlp_grad, dim3(nwg), dim3(GRAD_BLOCK), 0, c->st, dp, N, dx, dt, dw, n, 0, n, part, lp);
         hipLaunchKernelGGL(k_mlp_reduce, dim3((NPARAM + RED_PARAMS - 1) / RED_PARAMS), dim3(RED_BLOCK), 0, c->st, part,
                            nwg, lp, g, l, AdamStep{});
         if (hipGetLastError() != hipSuccess ||
@@ -917,8 +956,8 @@ int bh_mlp_bake(bh_ctx* c, int n0, int n1, int n2, float judge_tol, bh_mlp_bake_
     L.d2 = (float)((LS_HI - LS_LO) / (n2 - 1));
     double t0 = now_ms();
     const int ntiles = (int)((nodes + TM - 1) / TM);
-    hipLaunchKernelGGL(k_mlp_infer, dim3(std::min(ntiles, 8192)), dim3(64), 0, c->st, c->d_mlp, c->mlp_norm, nullptr,
-                       (int)nodes, 1, L, c->d_stab);
+    hipLaunchKernelGGL(k_mlp_infer, dim3(std::min(ntiles, INFER_GRID)), dim3(64 * TILE_WAVES), 0, c->st, c->d_mlp,
+                       c->mlp_norm, nullptr, (int)nodes, 1, L, (float*)c->d_stab);
     hipEvent_t e0, e1;
     (void)hipEventCreate(&e0);
     (void)hipEventCreate(&e1);
