@@ -188,13 +188,8 @@ namespace {
 // spills); 1 leaves the register budget to the compiler.
 static_assert(BLOCK == bhp::MAX_BLOCK && NCNT == bhp::NSTAT, "persistent kernel slots");
 
-template <int PREC, int RADIO, bool TIME, int WAVES, class Work>
-__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WAVES))) void k_persist(
-    const Work wk, unsigned int* __restrict__ queue, int interval, int refill_min, int prio_age,
-    BlockOut* __restrict__ blk) {
-    double flux;
-    unsigned long long c[NCNT];
-    bhp::persist_body<PREC, RADIO, TIME>(wk, queue, interval, refill_min, prio_age, &flux, c);
+// The workgroup's flux and counters from its lanes' sums
+__device__ __forceinline__ void block_out(double flux, unsigned long long c[NCNT], BlockOut* __restrict__ blk) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
     __shared__ double s_flux[BLOCK / 64];
     __shared__ unsigned long long s_cnt[BLOCK / 64][NCNT];
@@ -215,6 +210,26 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WAVES))) 
         }
         blk[blockIdx.x] = b;
     }
+}
+
+template <int PREC, int RADIO, bool TIME, int WAVES, class Work>
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WAVES))) void k_persist(
+    const Work wk, unsigned int* __restrict__ queue, int interval, int refill_min, int prio_age,
+    BlockOut* __restrict__ blk) {
+    double flux;
+    unsigned long long c[NCNT];
+    bhp::persist_body<PREC, RADIO, TIME>(wk, queue, interval, refill_min, prio_age, &flux, c);
+    block_out(flux, c, blk);
+}
+
+// Two waves per 64 rays (persist.h): an integrating and an evaluating wave per SIMD.
+template <int PREC, int RADIO, bool TIME, class Work>
+__global__ __launch_bounds__(bhp::PAIR_BLOCK) __attribute__((amdgpu_waves_per_eu(2))) void k_pair(
+    const Work wk, unsigned int* __restrict__ queue, int interval, int refill_min, int, BlockOut* __restrict__ blk) {
+    double flux;
+    unsigned long long c[NCNT];
+    bhp::pair_body<PREC, RADIO, TIME>(wk, queue, interval, refill_min, &flux, c);
+    block_out(flux, c, blk);
 }
 
 /* ---- adaptive sampling (render.cu:89-242, 677-721), deterministic form ----
@@ -1014,6 +1029,21 @@ WorkFn<Work> pick_persist_w(int prec, const Variant& v) {
                                 : pick_variant<BH_PREC_MIXED, Work::RECORDS>(v, PersistAt<BH_PREC_MIXED, W, Work>{});
 }
 
+template <int PREC, class Work>
+struct PairAt {
+    template <int RADIO, bool TIME>
+    WorkFn<Work> operator()() const {
+        if constexpr (RADIO == bhd::RADIO_OFF) return nullptr;
+        else return k_pair<PREC, RADIO, TIME, Work>;
+    }
+};
+
+template <class Work>
+WorkFn<Work> pick_pair(int prec, const Variant& v) {
+    return prec == BH_PREC_FP64 ? pick_variant<BH_PREC_FP64, Work::RECORDS>(v, PairAt<BH_PREC_FP64, Work>{})
+                                : pick_variant<BH_PREC_MIXED, Work::RECORDS>(v, PairAt<BH_PREC_MIXED, Work>{});
+}
+
 // adaptive passes and ray records: the kernel compiled for at least 3 waves per SIMD (waves 3 or 4) or
 // for the compiler's register budget (waves 0)
 template <class Work>
@@ -1041,6 +1071,12 @@ int persist_grid(const bh_ctx* c, const void* k, int block, int grid_per_cu) {
 
 constexpr size_t PLAIN_SPP_SAMPLE_BUDGET = size_t(1) << 30;   // bytes of per-sample storage of bh_render, spp > 1
 constexpr long long BATCH_MAX_PIXELS = 1ll << 30;   // per frame: keeps the 32-bit queue counters from wrapping
+
+/* Waves of rays per compute unit up to which a radio launch takes two waves per 64 rays (k_pair, 4 workgroups
+   per CU), from where the launch times cross (plain -> paired, ms). FP64: 64^2 3.5 -> 2.7, 256^2 4.5 -> 3.9,
+   384^2 (w = 9) 4.7 -> 4.4, 448^2 (12) 5.5 -> 5.7, 512^2 (16) 5.9 -> 7.1. Mixed: 64^2 1.19 -> 0.82, 256^2 1.74 ->
+   1.25, 512^2 (16) 2.04 -> 1.64, 640^2 (25) 1.94 -> 1.48, 768^2 (36) 2.28 -> 2.00, 896^2 (49) 2.41 -> 2.50. */
+constexpr double PAIR_W_MIXED = 40.0, PAIR_W_FP64 = 10.0;
 
 /* Defaults of a persistent launch of `entries` rays (all frames). w = waves of rays per compute unit; a
    CU holds 12 waves of these kernels (3 per SIMD). Measured on frames of 32^2 to 2048^2 (MI355X, ms of
@@ -1105,6 +1141,32 @@ int resolve_cfg(bh_ctx* c, const bh_batch_cfg& d, bh_batch_cfg* g) {
         return fail(c, BH_ERR_ARG, "order must be 0, 1, 2 or 3");
     if (g->prio_age > (1 << 24)) return fail(c, BH_ERR_ARG, "prio_age must be at most 2^24");
     return BH_OK;
+}
+
+// The kernel and grid of a persistent launch of `entries` rays: two waves per 64 rays up to PAIR_W_*, with the
+// default configuration; another one, given or tuned, keeps its kernel.
+template <class Work>
+struct PersistPlan {
+    WorkFn<Work> k;
+    int block, grid;
+};
+
+template <class Work>
+PersistPlan<Work> plan_persist(const bh_ctx* c, int prec, const Variant& v, long long entries, const bh_batch_cfg& dflt,
+                               const bh_batch_cfg& g, WorkFn<Work> plain) {
+    const double w = (double)entries / 64.0 / c->n_cu;
+    const bool as_default = g.block == dflt.block && g.grid_per_cu == dflt.grid_per_cu && g.interval == dflt.interval &&
+                            g.refill_min == dflt.refill_min && g.waves == dflt.waves && g.order == dflt.order &&
+                            g.prio_age == dflt.prio_age;
+    PersistPlan<Work> p{plain, g.block, 0};
+    int per_cu = g.grid_per_cu;
+    if (v.radio != bhd::RADIO_OFF && as_default && w <= (prec == BH_PREC_MIXED ? PAIR_W_MIXED : PAIR_W_FP64)) {
+        p.k = pick_pair<Work>(prec, v);
+        p.block = bhp::PAIR_BLOCK;
+        per_cu = 4;
+    }
+    p.grid = persist_grid(c, (const void*)p.k, p.block, per_cu);
+    return p;
 }
 
 // Enqueues the counting sort that fills each frame's tile order (frames already on the device;
@@ -1206,8 +1268,10 @@ int launch_batch(bh_ctx* c, const bh_batch_frame* frames, int n, const bh_trace_
         }
     }
     const int prio = cfg.prio_age > 0 ? cfg.prio_age : 0;
-    PersistFn k = pick_persist(o.precision, v, cfg.waves);
-    const int grid = persist_grid(c, (const void*)k, cfg.block, cfg.grid_per_cu);
+    const auto plan = plan_persist<bhp::BatchWork>(c, o.precision, v, batch_entries(frames, n), dflt, cfg,
+                                                   pick_persist(o.precision, v, cfg.waves));
+    const PersistFn k = plan.k;
+    const int grid = plan.grid;
     rc = ensure(c, &c->d_bframes, &c->bframes_cap, sizeof(bhp::BatchFrame) * (size_t)n);
     if (rc) return rc;
     rc = ensure(c, &c->d_queue, &c->queue_cap, (size_t)n);
@@ -1219,7 +1283,7 @@ int launch_batch(bh_ctx* c, const bh_batch_frame* frames, int n, const bh_trace_
     auto enqueue = [&]() -> hipError_t {
         hipLaunchKernelGGL(k_zero_u32, dim3((n + 255) / 256), dim3(256), 0, c->st, c->d_queue, n);
         if (ordered) enqueue_tile_order(c->st, dframes, n, max_tiles, c->d_ohist, cfg.order);
-        hipLaunchKernelGGL(k, dim3(grid), dim3(cfg.block), 0, c->st, bhp::BatchWork{dframes, n}, c->d_queue,
+        hipLaunchKernelGGL(k, dim3(grid), dim3(plan.block), 0, c->st, bhp::BatchWork{dframes, n}, c->d_queue,
                            cfg.interval, cfg.refill_min, prio, c->d_blk);
         hipLaunchKernelGGL(k_reduce, dim3(1), dim3(256), 0, c->st, c->d_blk, grid, c->d_tot);
         return hipGetLastError();
@@ -1232,7 +1296,7 @@ int launch_batch(bh_ctx* c, const bh_batch_frame* frames, int n, const bh_trace_
                                             (unsigned long long)(uintptr_t)c->d_queue,
                                             (unsigned long long)(uintptr_t)c->d_blk,
                                             (unsigned long long)(uintptr_t)c->d_tot, (unsigned long long)n,
-                                            (unsigned long long)grid, (unsigned long long)cfg.block,
+                                            (unsigned long long)grid, (unsigned long long)plan.block,
                                             (unsigned long long)cfg.interval, (unsigned long long)cfg.refill_min,
                                             (unsigned long long)ordered, (unsigned long long)max_tiles,
                                             (unsigned long long)(uintptr_t)c->d_ohist, (unsigned long long)prio,
@@ -1301,8 +1365,9 @@ int launch_records(bh_ctx* c, const bh_frame* f, const bh_trace_opts* opts, int 
     if (rc) return rc;
     rc = prepare_turbulence(c, c->S, f);
     if (rc) return rc;
-    const auto k = pick_adaptive<bhp::RecordWork>(o.precision, v, cfg.waves);
-    const int grid = persist_grid(c, (const void*)k, cfg.block, cfg.grid_per_cu);
+    const auto plan = plan_persist<bhp::RecordWork>(c, o.precision, v, (long long)tiles * 64, dflt, cfg,
+                                                    pick_adaptive<bhp::RecordWork>(o.precision, v, cfg.waves));
+    const int grid = plan.grid;
     bhp::BatchFrame B;
     std::memset(&B, 0, sizeof B);
     B.P = make_params(c, f);
@@ -1334,7 +1399,7 @@ int launch_records(bh_ctx* c, const bh_frame* f, const bh_trace_opts* opts, int 
     HIPCK(c, hipMemcpyAsync(c->d_bframes, &B, sizeof B, hipMemcpyHostToDevice, c->st));
     hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, c->st, c->d_queue, 1);
     if (ordered) enqueue_tile_order(c->st, dB, 1, (unsigned int)tiles, c->d_ohist, cfg.order);
-    hipLaunchKernelGGL(k, dim3(grid), dim3(cfg.block), 0, c->st, bhp::RecordWork{dB, 1, c->d_rays}, c->d_queue,
+    hipLaunchKernelGGL(plan.k, dim3(grid), dim3(plan.block), 0, c->st, bhp::RecordWork{dB, 1, c->d_rays}, c->d_queue,
                        cfg.interval, cfg.refill_min, cfg.prio_age > 0 ? cfg.prio_age : 0, c->d_blk);
     HIPCK(c, hipGetLastError());
     return BH_OK;
@@ -1354,8 +1419,9 @@ int launch_samples(bh_ctx* c, const bh_frame* f, const bh_trace_opts& o, int spp
     if (rc) return rc;
     rc = prepare_turbulence(c, c->S, f);
     if (rc) return rc;
-    const auto k = pick_adaptive<bhp::SampleWork>(o.precision, v, cfg.waves);
-    const int grid = persist_grid(c, (const void*)k, cfg.block, cfg.grid_per_cu);
+    const auto plan = plan_persist<bhp::SampleWork>(c, o.precision, v, (long long)tiles * 64 * spp, dflt, cfg,
+                                                    pick_adaptive<bhp::SampleWork>(o.precision, v, cfg.waves));
+    const int grid = plan.grid;
     const bool ordered = cfg.order != BH_ORDER_ROWS;
     std::memset(B, 0, 2 * sizeof B[0]);
     B[0].P = make_params(c, f);
@@ -1389,7 +1455,7 @@ int launch_samples(bh_ctx* c, const bh_frame* f, const bh_trace_opts& o, int spp
     HIPCK(c, hipMemcpyAsync(c->d_bframes, B, 2 * sizeof B[0], hipMemcpyHostToDevice, c->st));
     hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, c->st, c->d_queue, 1);
     if (ordered) enqueue_tile_order(c->st, dB + 1, 1, (unsigned int)tiles, c->d_ohist, cfg.order);
-    hipLaunchKernelGGL(k, dim3(grid), dim3(cfg.block), 0, c->st, bhp::SampleWork{dB, 1, spp, c->d_samp1}, c->d_queue,
+    hipLaunchKernelGGL(plan.k, dim3(grid), dim3(plan.block), 0, c->st, bhp::SampleWork{dB, 1, spp, c->d_samp1}, c->d_queue,
                        cfg.interval, cfg.refill_min, cfg.prio_age > 0 ? cfg.prio_age : 0, c->d_blk);
     HIPCK(c, hipGetLastError());
     *cfg_out = cfg;
@@ -1464,8 +1530,9 @@ int launch_adaptive(bh_ctx* c, const bh_frame* f, const bh_trace_opts* opts, lon
             if (!c->tuned_ok[o.precision]) cfg = dflt;
             rc = resolve_cfg(c, dflt, &cfg);
             if (rc) return rc;
-            const auto k2 = pick_adaptive<bhp::ChunkWork>(o.precision, v, cfg.waves);
-            grid = persist_grid(c, (const void*)k2, cfg.block, cfg.grid_per_cu);
+            const auto plan = plan_persist<bhp::ChunkWork>(c, o.precision, v, (long long)total * ADAPT_CHUNK, dflt, cfg,
+                                                           pick_adaptive<bhp::ChunkWork>(o.precision, v, cfg.waves));
+            grid = plan.grid;
             if ((rc = ensure(c, &c->d_samp2, &c->samp2_cap, (size_t)total * ADAPT_CHUNK)) ||
                 (rc = ensure(c, &c->d_blk, &c->blk_cap, (size_t)grid)))
                 return rc;
@@ -1475,7 +1542,7 @@ int launch_adaptive(bh_ctx* c, const bh_frame* f, const bh_trace_opts* opts, lon
             HIPCK(c, hipMemcpyAsync(c->d_bframes + sizeof(bhp::BatchFrame), &B[1], sizeof B[1], hipMemcpyHostToDevice,
                                     c->st));
             hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, c->st, c->d_queue, 1);
-            hipLaunchKernelGGL(k2, dim3(grid), dim3(cfg.block), 0, c->st,
+            hipLaunchKernelGGL(plan.k, dim3(grid), dim3(plan.block), 0, c->st,
                                bhp::ChunkWork{dB + 1, 1, spp, npix, c->d_offsets, c->d_samp2}, c->d_queue,
                                cfg.interval, cfg.refill_min, cfg.prio_age > 0 ? cfg.prio_age : 0, c->d_blk);
             hipLaunchKernelGGL(k_reduce, dim3(1), dim3(256), 0, c->st, c->d_blk, grid, c->d_tot);

@@ -517,14 +517,73 @@ __device__ __forceinline__ void ray_init(const TraceParams& P, double x, double 
     R.done = P.max_steps <= 0;
 }
 
+// One DP54 attempt from R (trace.cuh:81-97): n is the accepted state; false when the attempt is rejected.
+// ray_step spells the same out: through this function the persistent kernels take 11 more registers, and the
+// 1024^2 frame 21.2 ms for 20.0.
+template <int RADIO, bool TIME>
+__device__ __forceinline__ bool ray_attempt(const TraceParams& P, RayState& R, State& n, double& hc) {
+    hc = R.h;
+    if (RADIO && P.flow_on && R.s.y0 < P.r_flow_max) {
+        double cap = P.step_frac * fmin(bhm::quot_(R.s.y0, fabs(R.s.y1) + 1e-30),
+                                        bhm::quot_(fmax(R.sn, 0.05), fabs(R.s.y3) + 1e-30));
+        hc = fmin(hc, cap);
+    }
+    const double err = dp54_step<TIME>(P, R.c, R.s, hc, n);
+    ++R.it;
+    R.h = hc * step_factor(err);
+    if (!(err <= 1.0)) {
+        if (R.it >= P.max_steps) R.done = true;
+        return false;
+    }
+    ++R.accepted;
+    return true;
+}
+
+// The accepted state becomes the ray's; sets R.done when the ray stops there (trace.cuh:146-163).
+__device__ __forceinline__ void ray_settle(const TraceParams& P, RayState& R, const State& n) {
+    R.s = n;
+    project_radial(P, R.c, R.s);
+    if (R.s.y0 < P.r_stop) {
+        R.fate = -1;
+        R.done = true;
+        return;
+    }
+    if (R.s.y0 > P.r_escape && R.s.y1 > 0.0) {
+        R.fate = 1;   // escape angles are taken from the final state in ray_result
+        R.done = true;
+        return;
+    }
+    if (R.it >= P.max_steps) R.done = true;
+}
+
+// Angle between the directions p (of z component ppz) and q of two consecutive accepted states.
+__device__ __forceinline__ double ring_angle(double ppx, double ppy, double ppz, double pnx, double pny, double pnz) {
+    double cx = ppy * pnz - ppz * pny, cy = ppz * pnx - ppx * pnz, cz = ppx * pny - ppy * pnx;
+    double cl = bhm::sqrt_nn_(cx * cx + cy * cy + cz * cz);
+    double dt = ppx * pnx + ppy * pny + ppz * pnz;
+    return angle_pos(cl, dt);
+}
+
+// Adds a flow sample's emission dI and transmission e; true when the ray is opaque from here on.
+template <class RayS>
+__device__ __forceinline__ bool ray_absorb(RayS& R, int ord, double dI, double e) {
+    double cI = R.trans * dI;
+    R.acc0 += cI;
+    // value selects, not a branch chain: the chain becomes a dynamically indexed stack array
+    R.acc1 += ord == 1 ? cI : 0.0;
+    R.acc2 += ord == 2 ? cI : 0.0;
+    R.acc3 += ord >= 3 ? cI : 0.0;
+    R.trans *= e;
+    return R.trans < 1e-5;
+}
+
 // One iteration of trace.cuh:81-163 (one DP54 attempt); sets R.done when the ray stops.
 // P is what every attempt reads, F the same frame for what only a sample of the flow reads.
 template <int RADIO, bool TIME>
 __device__ __forceinline__ void ray_step(const TraceParams& P, const TraceParams& F, RayState& R) {
-    const bool flow = RADIO && P.flow_on;
     State n;
     double hc = R.h;
-    if (flow && R.s.y0 < P.r_flow_max) {
+    if (RADIO && P.flow_on && R.s.y0 < P.r_flow_max) {
         double cap = P.step_frac * fmin(bhm::quot_(R.s.y0, fabs(R.s.y1) + 1e-30),
                                         bhm::quot_(fmax(R.sn, 0.05), fabs(R.s.y3) + 1e-30));
         hc = fmin(hc, cap);
@@ -542,47 +601,80 @@ __device__ __forceinline__ void ray_step(const TraceParams& P, const TraceParams
         w = 1.0 - n.y2 * n.y2;
         const double sn = bhm::sqrt_nn_(fmax(w, 0.0));
         bhm::sincos(n.y4, &sv, &cv);
-        const double pnx = sn * cv, pny = sn * sv, pnz = n.y2, ppz = R.s.y2;
-        double cx = R.ppy * pnz - ppz * pny, cy = ppz * pnx - R.ppx * pnz, cz = R.ppx * pny - R.ppy * pnx;
-        double cl = bhm::sqrt_nn_(cx * cx + cy * cy + cz * cz);
-        double dt = R.ppx * pnx + R.ppy * pny + ppz * pnz;
-        R.psi += angle_pos(cl, dt);
+        const double pnx = sn * cv, pny = sn * sv;
+        R.psi += ring_angle(R.ppx, R.ppy, R.s.y2, pnx, pny, n.y2);
         R.ppx = pnx;
         R.ppy = pny;
         R.sn = sn;
     }
     if ((R.s.y2 > 0.0) != (n.y2 > 0.0)) ++R.ncross;
-    if (flow && n.y0 < P.r_flow_max) {
+    if (RADIO && P.flow_on && n.y0 < P.r_flow_max) {
         double dI, dtau;
         ++R.flow_steps;
         flow_step<RADIO>(F, n.y0, n.y2, w, R.sn, n.y4, sv, cv, n.y5, R.c.lam, R.c.E, hc, &dI, &dtau);
-        double cI = R.trans * dI;
-        int ord = (int)(R.psi * (1.0 / PI));
-        R.acc0 += cI;
-        // value selects, not a branch chain: the chain becomes a dynamically indexed stack array
-        R.acc1 += ord == 1 ? cI : 0.0;
-        R.acc2 += ord == 2 ? cI : 0.0;
-        R.acc3 += ord >= 3 ? cI : 0.0;
-        R.trans *= bhm::exp(-dtau);
-        if (R.trans < 1e-5) {
+        if (ray_absorb(R, (int)(R.psi * (1.0 / PI)), dI, bhm::exp(-dtau))) {
             R.fate = -1;
             R.done = true;
             return;
         }
     }
-    R.s = n;
-    project_radial(P, R.c, R.s);
-    if (R.s.y0 < P.r_stop) {
-        R.fate = -1;
-        R.done = true;
-        return;
-    }
-    if (R.s.y0 > P.r_escape && R.s.y1 > 0.0) {
-        R.fate = 1;   // escape angles are taken from the final state in ray_result
-        R.done = true;
-        return;
-    }
-    if (R.it >= P.max_steps) R.done = true;
+    ray_settle(P, R, n);
+}
+
+// What an accepted step leaves for another wave to evaluate: the new state and its step, the direction
+// before it, and whether the new state lies in the flow.
+struct StepSample {
+    double r, u, phi, t, h, u0, phi0;
+    bool flow;
+};
+
+// The attempt of ray_step without the ring angle and the flow: true when a step was accepted. SETTLE false
+// leaves the ray where it was, as ray_step does when the step's sample makes it opaque. R.ppx and R.ppy are
+// not kept up.
+template <int RADIO, bool TIME, bool SETTLE>
+__device__ __forceinline__ bool ray_move(const TraceParams& P, RayState& R, StepSample& q) {
+    State n;
+    if (!ray_attempt<RADIO, TIME>(P, R, n, q.h)) return false;
+    R.sn = bhm::sqrt_nn_(fmax(1.0 - n.y2 * n.y2, 0.0));
+    if ((R.s.y2 > 0.0) != (n.y2 > 0.0)) ++R.ncross;
+    q.r = n.y0;
+    q.u = n.y2;
+    q.phi = n.y4;
+    q.t = n.y5;
+    q.u0 = R.s.y2;
+    q.phi0 = R.s.y4;
+    q.flow = P.flow_on && n.y0 < P.r_flow_max;
+    if (q.flow) ++R.flow_steps;
+    if (SETTLE) ray_settle(P, R, n);
+    return true;
+}
+
+// The direction of a state as ray_step carries it
+struct Direction {
+    double x, y, z;
+};
+__device__ __forceinline__ Direction direction_of(double u, double phi) {
+    double sv, cv;
+    const double sn = bhm::sqrt_nn_(fmax(1.0 - u * u, 0.0));
+    bhm::sincos(phi, &sv, &cv);
+    return Direction{sn * cv, sn * sv, u};
+}
+
+// The ring angle, emission and transmission of a sample left by ray_move, as ray_step forms them; d is the
+// direction before the step, and after it on return.
+template <int RADIO>
+__device__ __forceinline__ void sample_eval(const TraceParams& F, double lam, double E, const StepSample& q, Direction& d,
+                                            double* ang, double* dI, double* e) {
+    double sv, cv;
+    const double w = 1.0 - q.u * q.u, sn = bhm::sqrt_nn_(fmax(w, 0.0));
+    bhm::sincos(q.phi, &sv, &cv);
+    const Direction n{sn * cv, sn * sv, q.u};
+    *ang = ring_angle(d.x, d.y, d.z, n.x, n.y, n.z);
+    d = n;
+    if (!q.flow) return;
+    double dtau;
+    flow_step<RADIO>(F, q.r, q.u, w, sn, q.phi, sv, cv, q.t, lam, E, q.h, dI, &dtau);
+    *e = bhm::exp(-dtau);
 }
 
 // blackholes/src/trace.cuh:25-33: galactic texture coordinates of the escape direction (th, ph),

@@ -746,17 +746,13 @@ __device__ __forceinline__ void ray_init_m(const TraceParams& P, const MixedPara
     R.done = P.max_steps <= 0;
 }
 
-// One attempt of trace.cuh:81-163 under the mixed policy. P and M are what every attempt reads (the
-// persistent engine holds them in registers), F and FM the same frame for what only a sample of the
-// flow reads. TCACHE keeps the ray's turbulence cell
-// in its state across attempts (the persistent engine); without it every flow sample loads its
-// corners (the frame kernel, already at the register limit, would spill the cache in its loop).
-template <int RADIO, bool TIME, bool TCACHE = true>
-__device__ __forceinline__ void ray_step_m(const TraceParams& P, const MixedParams& M, const TraceParams& F,
-                                           const MixedParams& FM, RayStateM& R) {
+// One attempt under the mixed policy: n is the accepted state and fac the controller's factor for the step
+// hc; false when the attempt is rejected.
+template <int RADIO, bool TIME>
+__device__ __forceinline__ bool ray_attempt_m(const TraceParams& P, const MixedParams& M, RayStateM& R, State& n,
+                                              double& hc, double& fac) {
     const bool flow = RADIO && P.flow_on;
-    State n;
-    double hc = R.h;
+    hc = R.h;
     if (flow && R.s.y0 < M.r_cut) {
         // the transfer step cap (trace.cuh:87-90) in FP32: a bound on the step, not part of its accuracy
         const float frac = (float)(R.it >= M.relax_after ? P.step_frac * M.relax_cap : P.step_frac);
@@ -787,76 +783,20 @@ __device__ __forceinline__ void ray_step_m(const TraceParams& P, const MixedPara
     R.k1_f32 = R.s.y0 >= M.r_f32;
     ++R.it;
     // one power for both outcomes (a rejected step's factor is below 0.9), so lanes that disagree share it
-    double fac = fmin(5.0, fmax(0.2, 0.9 * pow_m02_d(err)));
+    fac = fmin(5.0, fmax(0.2, 0.9 * pow_m02_d(err)));
     if (!(err <= 1.0)) {
         R.h = hc * fac;
         if (!(err == err)) R.h = hc * 0.1;
         if (R.it >= P.max_steps) R.done = true;
-        return;
+        return false;
     }
     ++R.accepted;
-    // the flow sample's density-free part first: its turbulence loads are in flight during the ring
-    // angle below
-    const bool in_flow = flow && n.y0 < M.r_cut;
-    FlowSample f;
-    FlowPending q;
-    TurbCache tl;
-    TurbCache& tc = TCACHE ? R.tc : tl;
-    bool emits = false;
-    if (in_flow) emits = flow_begin<RADIO, TCACHE>(F, M.E, n.y0, n.y2, n.y4, n.y5, R.c.lam, R.c.E, hc, f, q, tc);
-    // sin theta of the new state (FP64 1 - u^2, then FP32): the ring angle and the next step cap
-    const float s1 = sqrtf_(fmaxf((float)(1.0 - n.y2 * n.y2), 0.f));
-    if (RADIO) {
-        // angle between the radial directions p = (s0 cos phi0, s0 sin phi0, u0) of the previous and
-        // q of the new accepted state, from their chord without cancellation:
-        // |q - p|^2 = (u1 - u0)^2 + (s1 - s0)^2 + 4 s0 s1 sin^2(dphi / 2), angle = 2 asin(|q - p| / 2),
-        // with dphi taken in FP64 (no large-angle FP32 azimuth)
-        const float s0 = R.s_sin, du = (float)n.y2 - (float)R.s.y2, ds = s1 - s0;
-        const float hs = __sinf(0.5f * (float)(n.y4 - R.s.y4));
-        const float chord = sqrtf_(du * du + ds * ds + 4.f * s0 * s1 * hs * hs);
-        R.psi += 2.f * asin_pos(fminf(0.5f * chord, 1.f));
-    }
-    R.s_sin = s1;
-    if ((R.s.y2 > 0.0) != (n.y2 > 0.0)) ++R.ncross;
-    if (in_flow) {
-        ++R.flow_steps;
-        if (emits && flow_finish<RADIO>(F, M.E, n.y0, n.y4, n.y5, f, q, tc)) {
-            float ln_j, ln_a, ln_bnu;
-            if (FM.use_surrogate) {
-                // the table's loads first; the exact formula runs while they are in flight, and the
-                // table replaces its values wherever the cell is trusted
-                SurrogateFetch sf;
-                surrogate_fetch(FM.S, f.ln_nu - f.ln_nuc - (float)bhmlp::LN_2_9 - 2.f * f.ln_th - f.ln_sinb, f.ln_th,
-                                f.ln_sinb, sf);
-                synchrotron_exact(M.E, f.ln_ne, f.ln_th, f.ln_k2, f.ln_nu, f.ln_nuc, f.ln_sinb, &ln_j, &ln_a, &ln_bnu);
-                if (sf.use) {
-                    float fj, fa;
-                    surrogate_blend(sf, &fj, &fa);
-                    ln_j = f.ln_ne + FM.ln_e2_over_c + f.ln_nuc + fj;
-                    ln_a = f.ln_ne + FM.ln_e2_over_mec - f.ln_nuc + fa;
-                    ln_bnu = ln_j - ln_a;   // both within the table's floors: no cancellation
-                }
-            } else {
-                synchrotron_exact(M.E, f.ln_ne, f.ln_th, f.ln_k2, f.ln_nu, f.ln_nuc, f.ln_sinb, &ln_j, &ln_a, &ln_bnu);
-            }
-            double dI, dtau;
-            float etau;
-            transfer(M.E, f, ln_a, ln_bnu, &dI, &dtau, &etau);
-            double cI = R.trans * dI;
-            int ord = (int)(R.psi * 0.31830988618379067f);
-            R.acc0 += cI;
-            // value selects, not a branch chain: the chain becomes a dynamically indexed stack array
-            R.acc1 += ord == 1 ? cI : 0.0;
-            R.acc2 += ord == 2 ? cI : 0.0;
-            R.acc3 += ord >= 3 ? cI : 0.0;
-            R.trans *= (double)etau;
-            if (R.trans < 1e-5) {
-                R.fate = -1;
-                R.done = true;
-                return;
-            }
-        }
-    }
+    return true;
+}
+
+// The accepted state becomes the ray's; sets the next step, and R.done when the ray stops there.
+__device__ __forceinline__ void ray_settle_m(const TraceParams& P, const MixedParams& M, RayStateM& R, const State& n,
+                                             double hc, double fac) {
     const double r0 = R.s.y0;
     R.s = n;
     project_radial_m(P, R.c, R.s);
@@ -876,6 +816,121 @@ __device__ __forceinline__ void ray_step_m(const TraceParams& P, const MixedPara
         return;
     }
     if (R.it >= P.max_steps) R.done = true;
+}
+
+// Angle between the radial directions p = (s0 cos phi0, s0 sin phi0, u0) and q of two consecutive accepted
+// states, from their chord without cancellation: |q - p|^2 = (u1 - u0)^2 + (s1 - s0)^2 +
+// 4 s0 s1 sin^2(dphi / 2), angle = 2 asin(|q - p| / 2), with dphi taken in FP64 (no large-angle FP32 azimuth)
+__device__ __forceinline__ float ring_angle_m(double u0, double phi0, float s0, double u1, double phi1, float s1) {
+    const float du = (float)u1 - (float)u0, ds = s1 - s0;
+    const float hs = __sinf(0.5f * (float)(phi1 - phi0));
+    const float chord = sqrtf_(du * du + ds * ds + 4.f * s0 * s1 * hs * hs);
+    return 2.f * asin_pos(fminf(0.5f * chord, 1.f));
+}
+
+// sin theta of a state (FP64 1 - u^2, then FP32)
+__device__ __forceinline__ float sin_theta_m(double u) { return sqrtf_(fmaxf((float)(1.0 - u * u), 0.f)); }
+
+// Emission and absorption of a prepared flow sample.
+__device__ __forceinline__ void emission_m(const MixedParams& M, const MixedParams& FM, const FlowSample& f, double* dI,
+                                           double* dtau, float* etau) {
+    float ln_j, ln_a, ln_bnu;
+    if (FM.use_surrogate) {
+        // the table's loads first; the exact formula runs while they are in flight, and the
+        // table replaces its values wherever the cell is trusted
+        SurrogateFetch sf;
+        surrogate_fetch(FM.S, f.ln_nu - f.ln_nuc - (float)bhmlp::LN_2_9 - 2.f * f.ln_th - f.ln_sinb, f.ln_th,
+                        f.ln_sinb, sf);
+        synchrotron_exact(M.E, f.ln_ne, f.ln_th, f.ln_k2, f.ln_nu, f.ln_nuc, f.ln_sinb, &ln_j, &ln_a, &ln_bnu);
+        if (sf.use) {
+            float fj, fa;
+            surrogate_blend(sf, &fj, &fa);
+            ln_j = f.ln_ne + FM.ln_e2_over_c + f.ln_nuc + fj;
+            ln_a = f.ln_ne + FM.ln_e2_over_mec - f.ln_nuc + fa;
+            ln_bnu = ln_j - ln_a;   // both within the table's floors: no cancellation
+        }
+    } else {
+        synchrotron_exact(M.E, f.ln_ne, f.ln_th, f.ln_k2, f.ln_nu, f.ln_nuc, f.ln_sinb, &ln_j, &ln_a, &ln_bnu);
+    }
+    transfer(M.E, f, ln_a, ln_bnu, dI, dtau, etau);
+}
+
+// One attempt of trace.cuh:81-163 under the mixed policy. P and M are what every attempt reads (the
+// persistent engine holds them in registers), F and FM the same frame for what only a sample of the
+// flow reads. TCACHE keeps the ray's turbulence cell
+// in its state across attempts (the persistent engine); without it every flow sample loads its
+// corners (the frame kernel, already at the register limit, would spill the cache in its loop).
+template <int RADIO, bool TIME, bool TCACHE = true>
+__device__ __forceinline__ void ray_step_m(const TraceParams& P, const MixedParams& M, const TraceParams& F,
+                                           const MixedParams& FM, RayStateM& R) {
+    State n;
+    double hc, fac;
+    if (!ray_attempt_m<RADIO, TIME>(P, M, R, n, hc, fac)) return;
+    // the flow sample's density-free part first: its turbulence loads are in flight during the ring
+    // angle below
+    const bool in_flow = RADIO && P.flow_on && n.y0 < M.r_cut;
+    FlowSample f;
+    FlowPending q;
+    TurbCache tl;
+    TurbCache& tc = TCACHE ? R.tc : tl;
+    bool emits = false;
+    if (in_flow) emits = flow_begin<RADIO, TCACHE>(F, M.E, n.y0, n.y2, n.y4, n.y5, R.c.lam, R.c.E, hc, f, q, tc);
+    const float s1 = sin_theta_m(n.y2);   // for the ring angle and the next step cap
+    if (RADIO) R.psi += ring_angle_m(R.s.y2, R.s.y4, R.s_sin, n.y2, n.y4, s1);
+    R.s_sin = s1;
+    if ((R.s.y2 > 0.0) != (n.y2 > 0.0)) ++R.ncross;
+    if (in_flow) {
+        ++R.flow_steps;
+        if (emits && flow_finish<RADIO>(F, M.E, n.y0, n.y4, n.y5, f, q, tc)) {
+            double dI, dtau;
+            float etau;
+            emission_m(M, FM, f, &dI, &dtau, &etau);
+            if (bhd::ray_absorb(R, (int)(R.psi * 0.31830988618379067f), dI, (double)etau)) {
+                R.fate = -1;
+                R.done = true;
+                return;
+            }
+        }
+    }
+    ray_settle_m(P, M, R, n, hc, fac);
+}
+
+// bhd::ray_move and bhd::sample_eval under the mixed policy (the direction before the step is the sample's
+// own). emits: false for a sample that emits and absorbs nothing.
+template <int RADIO, bool TIME, bool SETTLE>
+__device__ __forceinline__ bool ray_move_m(const TraceParams& P, const MixedParams& M, RayStateM& R,
+                                           bhd::StepSample& q) {
+    State n;
+    double fac;
+    if (!ray_attempt_m<RADIO, TIME>(P, M, R, n, q.h, fac)) return false;
+    R.s_sin = sin_theta_m(n.y2);
+    if ((R.s.y2 > 0.0) != (n.y2 > 0.0)) ++R.ncross;
+    q.r = n.y0;
+    q.u = n.y2;
+    q.phi = n.y4;
+    q.t = n.y5;
+    q.u0 = R.s.y2;
+    q.phi0 = R.s.y4;
+    q.flow = P.flow_on && n.y0 < M.r_cut;
+    if (q.flow) ++R.flow_steps;
+    if (SETTLE) ray_settle_m(P, M, R, n, q.h, fac);
+    return true;
+}
+
+template <int RADIO>
+__device__ __forceinline__ void sample_eval_m(const TraceParams& F, const MixedParams& FM, double lam, double Ecam,
+                                              const bhd::StepSample& q, TurbCache& tc, float* ang, bool* emits,
+                                              double* dI, double* e) {
+    FlowSample f;
+    FlowPending p;
+    *emits = q.flow && flow_begin<RADIO, true>(F, FM.E, q.r, q.u, q.phi, q.t, lam, Ecam, q.h, f, p, tc);
+    *ang = ring_angle_m(q.u0, q.phi0, sin_theta_m(q.u0), q.u, q.phi, sin_theta_m(q.u));
+    if (*emits) *emits = flow_finish<RADIO>(F, FM.E, q.r, q.phi, q.t, f, p, tc);
+    if (!*emits) return;
+    double dtau;
+    float etau;
+    emission_m(FM, FM, f, dI, &dtau, &etau);
+    *e = (double)etau;
 }
 
 // Outputs of a finished ray; returns the number of FP64 step attempts.
