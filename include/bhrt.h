@@ -262,7 +262,8 @@ typedef struct bh_batch_cfg {
                            per SIMD, for launches that hold all their rays at once, to 256 threads and three
                            waves per SIMD; rows order for the largest FP64 launches and those without
                            generations, else critical; interval 64, refill_min 32 (mixed) / 48 (FP64), graph,
-                           waves 3, prio_age 256. */
+                           waves 3, prio_age 256. Radio launches of few rays (to 40 waves per CU mixed, 10
+                           FP64) integrate and evaluate in two waves side by side then; same results. */
 } bh_batch_cfg;
 
 /* Traces every frame of `frames`; px_out (nullable) receives the frames one after the other,
