@@ -163,6 +163,11 @@ struct ChunkWork {
     }
 };
 
+// A ray's counters after one of its attempts
+struct Marks {
+    int it, accepted, flow_steps, ncross, fp64;
+};
+
 template <int PREC, int RADIO, bool TIME>
 struct Tracer;
 
@@ -177,10 +182,18 @@ struct Tracer<BH_PREC_FP64, RADIO, TIME> {
                                                 const bhm32::MixedParams&, State& R) {
         bhd::ray_step<RADIO, TIME>(P, F, R);
     }
-    template <bool SETTLE>
     static __device__ __forceinline__ bool move(const TraceParams& P, const bhm32::MixedParams&, State& R,
                                                 bhd::StepSample& q) {
-        return bhd::ray_move<RADIO, TIME, SETTLE>(P, R, q);
+        return bhd::ray_move<RADIO, TIME>(P, R, q);
+    }
+    static __device__ __forceinline__ Marks marks(const State& R) {
+        return Marks{R.it, R.accepted, R.flow_steps, R.ncross, 0};
+    }
+    static __device__ __forceinline__ void set_marks(State& R, const Marks& m) {
+        R.it = m.it;
+        R.accepted = m.accepted;
+        R.flow_steps = m.flow_steps;
+        R.ncross = m.ncross;
     }
     // what a ray's samples add up to, in the wave that evaluates them
     struct Sums {
@@ -217,10 +230,19 @@ struct Tracer<BH_PREC_MIXED, RADIO, TIME> {
                                                 const bhm32::MixedParams& FM, State& R) {
         bhm32::ray_step_m<RADIO, TIME>(P, M, F, FM, R);
     }
-    template <bool SETTLE>
     static __device__ __forceinline__ bool move(const TraceParams& P, const bhm32::MixedParams& M, State& R,
                                                 bhd::StepSample& q) {
-        return bhm32::ray_move_m<RADIO, TIME, SETTLE>(P, M, R, q);
+        return bhm32::ray_move_m<RADIO, TIME>(P, M, R, q);
+    }
+    static __device__ __forceinline__ Marks marks(const State& R) {
+        return Marks{R.it, R.accepted, R.flow_steps, R.ncross, R.fp64_attempts};
+    }
+    static __device__ __forceinline__ void set_marks(State& R, const Marks& m) {
+        R.it = m.it;
+        R.accepted = m.accepted;
+        R.flow_steps = m.flow_steps;
+        R.ncross = m.ncross;
+        R.fp64_attempts = m.fp64;
     }
     struct Sums {
         double acc0, acc1, acc2, acc3, trans;
@@ -394,28 +416,49 @@ __device__ __forceinline__ void persist_body(const Work& Wk, unsigned int* __res
    long as its longest ray's chain of instructions. Of an attempt's chain only the integration is a chain: the
    flow sample and the ring angle (nearly half) feed nothing back but the end of an opaque ray. So the
    workgroup's first wave integrates and leaves each accepted step in LDS, and the second evaluates it during
-   the next attempt: one barrier per attempt, two slots by turns. A ray that turns out opaque has run on to the
-   end of the interval by then: it is taken back to the interval's start and repeats its attempts up to the
-   one that made it opaque, so what it leaves behind is the same. Every value is formed by the same operations
-   in the same order as in ray_step: same outputs. 37 x 29 FP64
-   records 1.59 -> 1.28 ms, 160^2 flux 4.7 -> 4.1, mixed 480 x 270 preview 2.2 -> 1.9.
+   the next attempt: one barrier per attempt, two slots by turns. Every value is formed by the same operations
+   in the same order as in ray_step: same outputs. One wave -> two, ms of the launch (frames 30 M wide at 17
+   degrees, the 0.6 Jy flow): mixed 64^2 1.32 -> 0.98, 256^2 2.04 -> 1.69; FP64 64^2 3.9 -> 2.9, 256^2 5.6 -> 4.4.
+   A ray that turned out opaque in attempt k is known to be so after the barrier of attempt k + 1, which it
+   has made too: it is taken back to what it was before the step of attempt k (its counters from registers;
+   its state, which only ray records hold, from attempt k's slot) and takes no further attempts. So an
+   opaque ray costs one attempt more than it has; learning of it only at the interval's end, and then repeating
+   the interval's attempts up to k, cost an optically thick flow (3000 times the density, 69 degrees) its gain
+   and more: mixed 256^2 0.73 ms, 448^2 1.25, 640^2 1.88; now 0.52, 0.84, 1.26; one wave 0.63, 0.81, 1.20.
    Both waves take every branch around a barrier on a value that both read from LDS. */
 constexpr int PAIR_BLOCK = 128;
 
-template <class T>
+template <bool RECORDS>
 struct PairLDS {
     double v[2][7][64];        // StepSample
+    double y[RECORDS ? 2 : 1][RECORDS ? 4 : 1][64];   // r, r', u', t before the step
     int tag[2][64];            // 0: no sample; 1: a step outside the flow; 3: inside
+    int opaque[2][64];         // the attempt's sample made the ray opaque
     int more[2];               // some ray runs on after this attempt
     int frame;                 // the rays' frame; -1: no rays are left
     int fresh[64];             // the lane has a new ray
-    int opaque[64];            // attempt of the interval that made the ray opaque, or -1
     double lam[64], E[64];
     double sums[6][64];        // acc0..3, trans, psi
-    typename T::State start[64];   // at the interval's start
     double flux[64];
     unsigned long long stat[NSTAT][64];
 };
+
+// Takes the lane's ray back to attempt m, in slot b, which made it opaque.
+template <class T, bool RECORDS>
+__device__ __forceinline__ void take_back(const PairLDS<RECORDS>& L, int b, int lane, const Marks& m,
+                                          typename T::State& R) {
+    T::set_marks(R, m);
+    if constexpr (RECORDS) {
+        R.s.y0 = L.y[b][0][lane];
+        R.s.y1 = L.y[b][1][lane];
+        R.s.y2 = L.v[b][5][lane];
+        R.s.y3 = L.y[b][2][lane];
+        R.s.y4 = L.v[b][6][lane];
+        R.s.y5 = L.y[b][3][lane];
+    }
+    R.fate = -1;
+    R.done = true;
+}
 
 template <int PREC, int RADIO, bool TIME, class Work>
 __device__ __forceinline__ void pair_body(const Work& Wk, unsigned int* __restrict__ queue, int interval,
@@ -423,7 +466,8 @@ __device__ __forceinline__ void pair_body(const Work& Wk, unsigned int* __restri
     using T = Tracer<PREC, RADIO, TIME>;
     using CFrame = const __attribute__((address_space(4))) BatchFrame;
     CFrame* cfr = (CFrame*)Wk.frames;
-    __shared__ PairLDS<T> L;
+    constexpr bool RECORDS = Work::RECORDS;
+    __shared__ PairLDS<RECORDS> L;
     const int lane = threadIdx.x & 63;
     const bool mover = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) == 0;
     *flux_out = 0.0;
@@ -444,17 +488,21 @@ __device__ __forceinline__ void pair_body(const Work& Wk, unsigned int* __restri
             if (active) {
                 L.lam[lane] = R.c.lam;
                 L.E[lane] = R.c.E;
-                L.start[lane] = R;
             }
             if (lane == 0) L.frame = !any && cur >= Wk.n ? -1 : cf;
             __syncthreads();   // A: the interval's rays
             if (!any && cur >= Wk.n) break;
             const TraceParams P = *(const TraceParams*)&cfr[cf].P;
             const bhm32::MixedParams M = *(const bhm32::MixedParams*)&cfr[cf].M;
-            for (int k = 0;; ++k) {
-                bhd::StepSample q;
-                const bool push = active && !R.done && T::template move<true>(P, M, R, q);
+            Marks m = T::marks(R);   // after the attempt before this one
+            int k = 0;
+            for (;; ++k) {
                 const int b = k & 1;
+                if (k >= 2 && L.opaque[b][lane]) take_back<T>(L, b, lane, m, R);   // by attempt k - 2
+                m = T::marks(R);
+                [[maybe_unused]] const double r0 = R.s.y0, dr0 = R.s.y1, du0 = R.s.y3, t0 = R.s.y5;
+                bhd::StepSample q;
+                const bool push = active && !R.done && T::move(P, M, R, q);
                 if (push) {
                     L.v[b][0][lane] = q.r;
                     L.v[b][1][lane] = q.u;
@@ -463,6 +511,12 @@ __device__ __forceinline__ void pair_body(const Work& Wk, unsigned int* __restri
                     L.v[b][4][lane] = q.h;
                     L.v[b][5][lane] = q.u0;
                     L.v[b][6][lane] = q.phi0;
+                    if constexpr (RECORDS) {
+                        L.y[b][0][lane] = r0;
+                        L.y[b][1][lane] = dr0;
+                        L.y[b][2][lane] = du0;
+                        L.y[b][3][lane] = t0;
+                    }
                 }
                 L.tag[b][lane] = push ? (q.flow ? 3 : 1) : 0;
                 const bool more = k + 1 < interval && __ballot(active && !R.done) != 0ull;
@@ -471,15 +525,9 @@ __device__ __forceinline__ void pair_body(const Work& Wk, unsigned int* __restri
                 if (!more) break;
             }
             __syncthreads();   // C: the interval's sums
-            const int last = active ? L.opaque[lane] : -1;
-            if (last >= 0) {
-                bhd::StepSample q;
-                R = L.start[lane];
-                for (int k = 0; k < last; ++k) T::template move<true>(P, M, R, q);
-                T::template move<false>(P, M, R, q);
-                R.fate = -1;
-                R.done = true;
-            }
+            // the last two attempts' samples
+            if (k > 0 && L.opaque[(k - 1) & 1][lane]) take_back<T>(L, (k - 1) & 1, lane, m, R);
+            else if (L.opaque[k & 1][lane]) take_back<T>(L, k & 1, lane, T::marks(R), R);
             if (active && R.done) {
                 R.acc0 = L.sums[0][lane];
                 R.acc1 = L.sums[1][lane];
@@ -516,19 +564,21 @@ __device__ __forceinline__ void pair_body(const Work& Wk, unsigned int* __restri
                 lam = L.lam[lane];
                 E = L.E[lane];
             }
-            int opaque = -1;
+            bool opaque = false;
             for (int k = 0;; ++k) {
                 __syncthreads();   // B
                 const int b = k & 1, tag = L.tag[b][lane];
                 const bool more = __builtin_amdgcn_readfirstlane(L.more[b]) != 0;
-                if (tag && opaque < 0) {
+                bool now = false;
+                if (tag && !opaque) {
                     const bhd::StepSample q{L.v[b][0][lane], L.v[b][1][lane], L.v[b][2][lane], L.v[b][3][lane],
                                             L.v[b][4][lane], L.v[b][5][lane], L.v[b][6][lane], tag == 3};
-                    if (T::add(F, FM, lam, E, q, S)) opaque = k;
+                    now = T::add(F, FM, lam, E, q, S);
                 }
+                L.opaque[b][lane] = now;
+                opaque = opaque || now;
                 if (!more) break;
             }
-            L.opaque[lane] = opaque;
             L.sums[0][lane] = S.acc0;
             L.sums[1][lane] = S.acc1;
             L.sums[2][lane] = S.acc2;
