@@ -24,6 +24,7 @@
 #include "trace_fp64.h"
 #include "trace_mixed.h"
 #include "ctx.h"
+#include "launch.h"
 #include "persist.h"
 
 using bhd::RayResult;
@@ -773,6 +774,49 @@ KernelFn pick_kernel(int prec, const Variant& v, bool rays) {
 constexpr double C_C = 2.99792458e10, C_H = 6.62607015e-27, C_ME = 9.1093837e-28, C_MP = 1.67262192e-24,
                  C_QE = 4.80320471e-10, C_PI = 3.14159265358979323846;
 
+// Emission weight j r^2 and absorption coefficient of the mid-plane flow at radius r
+void flow_cell(const bh_scene& S, const std::vector<float>& k2, float k2_l0, float k2_dl, double r, double* w,
+               double* alpha) {
+    const double ne = S.n0 * std::pow(r, -S.n_index) * (1.0 - std::exp(-(r - S.rh) * (r - S.rh) / 0.25));
+    const double th = S.theta0 * std::pow(r, -S.theta_index);
+    const double B = std::sqrt(8.0 * C_PI * ne * C_MP * C_C * C_C / (6.0 * r * S.beta_p));
+    const double nus = 2.0 / 9.0 * (C_QE * B / (2.0 * C_PI * C_ME * C_C)) * th * th;
+    const double X = S.nu_obs / nus, x3 = std::cbrt(X);
+    float f = ((float)std::log(th) - k2_l0) / k2_dl;
+    f = std::min(f > 0.f ? f : 0.f, (float)(k2.size() - 2) + 0.9999f);   // a NaN reads the first entry
+    const int k = (int)f;
+    const double lk2 = k2[k] + (k2[k + 1] - k2[k]) * (f - k);
+    const double brk = std::sqrt(X) + 1.887748625363387 * std::sqrt(x3);
+    // j_nu in cgs (emission.cuh:165-166) and alpha_nu = j_nu / B_nu(T_e) (Kirchhoff)
+    const double j = ne * std::sqrt(2.0) * C_PI * C_QE * C_QE * nus / (3.0 * C_C) * std::exp(-lk2) * brk * brk *
+                     std::exp(-x3);
+    const double bnu = 2.0 * C_H * S.nu_obs * S.nu_obs * S.nu_obs / (C_C * C_C) /
+                       std::expm1(C_H * S.nu_obs / (C_ME * C_C * C_C * th));
+    *w = std::isfinite(j) ? j * r * r : 0.0;
+    *alpha = std::isfinite(j) && bnu > 0.0 ? j / bnu : 0.0;
+}
+
+// Beyond it a vacuum ray does not circle the hole: the photon orbits and the horizon lie well inside
+double near_radius(const bh_scene& S) {
+    const double r_ph = 2.0 * (1.0 + std::cos(2.0 / 3.0 * std::acos(std::min(1.0, std::fabs(S.a)))));
+    return std::max(3.0 * S.rh, r_ph) + 1.0;
+}
+
+// Whether the mid-plane optical depth from the flow's edge down to near_radius exceeds 1, from 64 cells in ln r
+bool flow_opaque(const bh_ctx* c, const bh_scene& S) {
+    constexpr int N = 64;
+    const double r0 = near_radius(S), r1 = S.r_flow_max;
+    if (!S.flow_on || !(r1 > r0) || c->k2_host.size() < 2) return false;
+    const double dl = std::log(r1 / r0) / N;
+    double tau = 0.0, w, alpha;
+    for (int i = 0; i < N; ++i) {
+        const double r = r0 * std::exp(dl * (i + 0.5));
+        flow_cell(S, c->k2_host, c->k2_l0, c->k2_dl, r, &w, &alpha);
+        tau += alpha * r * dl * S.rg_cm;
+    }
+    return tau > 1.0;
+}
+
 /* Radius outside which the scene's flow model emits a fraction `frac` of its emission: the thermal
    synchrotron emissivity (emission.cuh:130-170 at nu_obs, in the mid-plane, sin theta_B = 1, no
    Doppler factor, no turbulence) weighted by r^2 (a face-on annulus of height ~ h_r r), integrated
@@ -783,28 +827,8 @@ double emission_radius(const bh_scene& S, const std::vector<float>& k2, float k2
     const double r0 = S.rh * 1.001, r1 = S.r_flow_max;
     if (!(r1 > r0) || k2.size() < 2) return r1;
     const double dr = (r1 - r0) / n;
-    // emission weight j r^2 and absorption coefficient of radial cell i (no storage: the bh_render_noalloc
-    // path must not allocate, so the two passes below evaluate each cell twice)
-    auto cell = [&](int i, double* w, double* alpha) {
-        const double r = r0 + dr * (i + 0.5);
-        const double ne = S.n0 * std::pow(r, -S.n_index) * (1.0 - std::exp(-(r - S.rh) * (r - S.rh) / 0.25));
-        const double th = S.theta0 * std::pow(r, -S.theta_index);
-        const double B = std::sqrt(8.0 * C_PI * ne * C_MP * C_C * C_C / (6.0 * r * S.beta_p));
-        const double nus = 2.0 / 9.0 * (C_QE * B / (2.0 * C_PI * C_ME * C_C)) * th * th;
-        const double X = S.nu_obs / nus, x3 = std::cbrt(X);
-        float f = ((float)std::log(th) - k2_l0) / k2_dl;
-        f = std::min(std::max(f, 0.f), (float)(k2.size() - 2) + 0.9999f);
-        const int k = (int)f;
-        const double lk2 = k2[k] + (k2[k + 1] - k2[k]) * (f - k);
-        const double brk = std::sqrt(X) + 1.887748625363387 * std::sqrt(x3);
-        // j_nu in cgs (emission.cuh:165-166) and alpha_nu = j_nu / B_nu(T_e) (Kirchhoff)
-        const double j = ne * std::sqrt(2.0) * C_PI * C_QE * C_QE * nus / (3.0 * C_C) * std::exp(-lk2) * brk * brk *
-                         std::exp(-x3);
-        const double bnu = 2.0 * C_H * S.nu_obs * S.nu_obs * S.nu_obs / (C_C * C_C) /
-                           std::expm1(C_H * S.nu_obs / (C_ME * C_C * C_C * th));
-        *w = std::isfinite(j) ? j * r * r : 0.0;
-        *alpha = std::isfinite(j) && bnu > 0.0 ? j / bnu : 0.0;
-    };
+    // no storage: the bh_render_noalloc path must not allocate, so the two passes below evaluate each cell twice
+    auto cell = [&](int i, double* w, double* alpha) { flow_cell(S, k2, k2_l0, k2_dl, r0 + dr * (i + 0.5), w, alpha); };
     double tot = 0.0, w, alpha;
     for (int i = 0; i < n; ++i) {
         cell(i, &w, &alpha);
@@ -855,8 +879,7 @@ bhm32::MixedParams make_mixed(bh_ctx* c, const bh_scene& S, const bh_frame* f, c
         const double axis = std::min(1.0, std::fabs(std::sin(f->th)) / std::sin(15.0 * PI / 180.0));
         M.tol_far = std::max(M.tol_mid, std::min(1e-4, 1e-4 * (f->pix * f->r) / 0.04) * axis);
     }
-    const double r_ph = 2.0 * (1.0 + std::cos(2.0 / 3.0 * std::acos(std::min(1.0, std::fabs(S.a)))));
-    const double r_near = o.r_near > 0 ? o.r_near : std::max(3.0 * S.rh, r_ph) + 1.0;
+    const double r_near = o.r_near > 0 ? o.r_near : near_radius(S);
     M.r_far = r_near;
     M.r_tol = r_near;
     if (S.mode == BH_MODE_RADIO && S.flow_on) {
@@ -1072,12 +1095,6 @@ int persist_grid(const bh_ctx* c, const void* k, int block, int grid_per_cu) {
 constexpr size_t PLAIN_SPP_SAMPLE_BUDGET = size_t(1) << 30;   // bytes of per-sample storage of bh_render, spp > 1
 constexpr long long BATCH_MAX_PIXELS = 1ll << 30;   // per frame: keeps the 32-bit queue counters from wrapping
 
-/* Waves of rays per compute unit up to which a radio launch takes two waves per 64 rays (k_pair, 4 workgroups
-   per CU), from where the launch times cross (plain -> paired, ms). FP64: 64^2 3.5 -> 2.7, 256^2 4.5 -> 3.9,
-   384^2 (w = 9) 4.7 -> 4.4, 448^2 (12) 5.5 -> 5.7, 512^2 (16) 5.9 -> 7.1. Mixed: 64^2 1.19 -> 0.82, 256^2 1.74 ->
-   1.25, 512^2 (16) 2.04 -> 1.64, 640^2 (25) 1.94 -> 1.48, 768^2 (36) 2.28 -> 2.00, 896^2 (49) 2.41 -> 2.50. */
-constexpr double PAIR_W_MIXED = 40.0, PAIR_W_FP64 = 10.0;
-
 /* Defaults of a persistent launch of `entries` rays (all frames). w = waves of rays per compute unit; a
    CU holds 12 waves of these kernels (3 per SIMD). Measured on frames of 32^2 to 2048^2 (MI355X, ms of
    the launch):
@@ -1102,7 +1119,7 @@ bh_batch_cfg batch_defaults(const bh_ctx* c, int prec, const Variant& v, long lo
     d.prio_age = prec == BH_PREC_MIXED ? 128 : 256;
     if (prec == BH_PREC_MIXED) {
         const bool vacuum = v.radio == bhd::RADIO_OFF;
-        const int per_cu = w <= (vacuum ? 8.0 : 20.0) ? 4 : (!vacuum && w <= 48.0 ? 8 : 12);
+        const int per_cu = w <= (vacuum ? 8.0 : launch::PAIR_REACH_OPAQUE) ? 4 : (!vacuum && w <= 48.0 ? 8 : 12);
         d.block = per_cu == 4 && !vacuum ? 64 : 256;
         d.grid_per_cu = per_cu * 64 / d.block;
         d.refill_min = 32;
@@ -1143,7 +1160,35 @@ int resolve_cfg(bh_ctx* c, const bh_batch_cfg& d, bh_batch_cfg* g) {
     return BH_OK;
 }
 
-// The kernel and grid of a persistent launch of `entries` rays: two waves per 64 rays up to PAIR_W_*, with the
+// What a launch over `n` frames' descriptors has to do; entries: its rays. With regions: the frames' P.x0 .. P.h
+// are the regions traced, each with nentries rays; else where its rays lie is not known, and all of them count
+// as reaching the flow.
+launch::Load load_of(bh_ctx* c, int prec, const Variant& v, const bhp::BatchFrame* B, const bh_scene* const* scenes,
+                     int n, long long entries, bool regions) {
+    launch::Load l;
+    l.precision = prec;
+    l.radio = v.radio;
+    l.w = (double)entries / 64.0 / c->n_cu;
+    l.reach = l.w;
+    // only where launch::pairs asks
+    if (v.radio == bhd::RADIO_OFF || prec != BH_PREC_MIXED || l.w <= launch::PAIR_REACH_OPAQUE || l.w > launch::PAIR_W_MIXED)
+        return l;
+    double rays = 0.0;
+    const bh_scene* last = nullptr;   // frames of a batch usually share their flow
+    for (int i = 0; i < n; ++i) {
+        const TraceParams& P = B[i].P;
+        if (regions)
+            rays += (double)B[i].nentries * launch::share_within(B[i].M.r_cut, P.kp[0], P.cx, P.cy, P.pix, P.W, P.H, P.x0,
+                                                                 P.y0, P.w, P.h);
+        if (l.opaque || (last && std::memcmp(last, scenes[i], sizeof *last) == 0)) continue;
+        last = scenes[i];
+        l.opaque = flow_opaque(c, *last);
+    }
+    if (regions) l.reach = rays / 64.0 / c->n_cu;
+    return l;
+}
+
+// The kernel and grid of a persistent launch: two waves per 64 rays where launch::pairs says so, with the
 // default configuration; another one, given or tuned, keeps its kernel.
 template <class Work>
 struct PersistPlan {
@@ -1152,16 +1197,15 @@ struct PersistPlan {
 };
 
 template <class Work>
-PersistPlan<Work> plan_persist(const bh_ctx* c, int prec, const Variant& v, long long entries, const bh_batch_cfg& dflt,
+PersistPlan<Work> plan_persist(const bh_ctx* c, const launch::Load& load, const Variant& v, const bh_batch_cfg& dflt,
                                const bh_batch_cfg& g, WorkFn<Work> plain) {
-    const double w = (double)entries / 64.0 / c->n_cu;
     const bool as_default = g.block == dflt.block && g.grid_per_cu == dflt.grid_per_cu && g.interval == dflt.interval &&
                             g.refill_min == dflt.refill_min && g.waves == dflt.waves && g.order == dflt.order &&
                             g.prio_age == dflt.prio_age;
     PersistPlan<Work> p{plain, g.block, 0};
     int per_cu = g.grid_per_cu;
-    if (v.radio != bhd::RADIO_OFF && as_default && w <= (prec == BH_PREC_MIXED ? PAIR_W_MIXED : PAIR_W_FP64)) {
-        p.k = pick_pair<Work>(prec, v);
+    if (as_default && launch::pairs(load)) {
+        p.k = pick_pair<Work>(load.precision, v);
         p.block = bhp::PAIR_BLOCK;
         per_cu = 4;
     }
@@ -1220,9 +1264,11 @@ int launch_batch(bh_ctx* c, const bh_batch_frame* frames, int n, const bh_trace_
     }
     long long total = 0;
     std::vector<bhp::BatchFrame> hb((size_t)n);
+    std::vector<const bh_scene*> scenes((size_t)n);
     for (int i = 0; i < n; ++i) {
         const bh_frame* f = &frames[i].frame;
         const bh_scene& S = frames[i].scene;
+        scenes[(size_t)i] = &S;
         if (f->W <= 0 || f->H <= 0 || (long long)f->W * f->H > BATCH_MAX_PIXELS)
             return fail(c, BH_ERR_ARG, "bad frame size in batch (at most 2^30 pixels per frame)");
         if (!(f->pix > 0.0)) return fail(c, BH_ERR_ARG, "frame pixel scale must be > 0");
@@ -1268,8 +1314,8 @@ int launch_batch(bh_ctx* c, const bh_batch_frame* frames, int n, const bh_trace_
         }
     }
     const int prio = cfg.prio_age > 0 ? cfg.prio_age : 0;
-    const auto plan = plan_persist<bhp::BatchWork>(c, o.precision, v, batch_entries(frames, n), dflt, cfg,
-                                                   pick_persist(o.precision, v, cfg.waves));
+    const launch::Load load = load_of(c, o.precision, v, hb.data(), scenes.data(), n, batch_entries(frames, n), true);
+    const auto plan = plan_persist<bhp::BatchWork>(c, load, v, dflt, cfg, pick_persist(o.precision, v, cfg.waves));
     const PersistFn k = plan.k;
     const int grid = plan.grid;
     rc = ensure(c, &c->d_bframes, &c->bframes_cap, sizeof(bhp::BatchFrame) * (size_t)n);
@@ -1365,9 +1411,6 @@ int launch_records(bh_ctx* c, const bh_frame* f, const bh_trace_opts* opts, int 
     if (rc) return rc;
     rc = prepare_turbulence(c, c->S, f);
     if (rc) return rc;
-    const auto plan = plan_persist<bhp::RecordWork>(c, o.precision, v, (long long)tiles * 64, dflt, cfg,
-                                                    pick_adaptive<bhp::RecordWork>(o.precision, v, cfg.waves));
-    const int grid = plan.grid;
     bhp::BatchFrame B;
     std::memset(&B, 0, sizeof B);
     B.P = make_params(c, f);
@@ -1384,6 +1427,11 @@ int launch_records(bh_ctx* c, const bh_frame* f, const bh_trace_opts* opts, int 
     }
     B.tiles_x = tiles_x;
     B.nentries = (unsigned int)tiles * 64u;
+    const bh_scene* scene = &c->S;
+    const launch::Load load = load_of(c, o.precision, v, &B, &scene, 1, (long long)tiles * 64, true);
+    const auto plan = plan_persist<bhp::RecordWork>(c, load, v, dflt, cfg,
+                                                    pick_adaptive<bhp::RecordWork>(o.precision, v, cfg.waves));
+    const int grid = plan.grid;
     const bool ordered = cfg.order != BH_ORDER_ROWS;
     if (ordered) {
         if ((rc = ensure(c, &c->d_order, &c->order_cap, (size_t)tiles)) ||
@@ -1419,9 +1467,6 @@ int launch_samples(bh_ctx* c, const bh_frame* f, const bh_trace_opts& o, int spp
     if (rc) return rc;
     rc = prepare_turbulence(c, c->S, f);
     if (rc) return rc;
-    const auto plan = plan_persist<bhp::SampleWork>(c, o.precision, v, (long long)tiles * 64 * spp, dflt, cfg,
-                                                    pick_adaptive<bhp::SampleWork>(o.precision, v, cfg.waves));
-    const int grid = plan.grid;
     const bool ordered = cfg.order != BH_ORDER_ROWS;
     std::memset(B, 0, 2 * sizeof B[0]);
     B[0].P = make_params(c, f);
@@ -1436,6 +1481,11 @@ int launch_samples(bh_ctx* c, const bh_frame* f, const bh_trace_opts& o, int spp
     }
     B[0].tiles_x = tiles_x;
     B[0].nentries = (unsigned int)(tiles * 64 * spp);
+    const bh_scene* scene = &c->S;
+    const launch::Load load = load_of(c, o.precision, v, B, &scene, 1, (long long)tiles * 64 * spp, true);
+    const auto plan = plan_persist<bhp::SampleWork>(c, load, v, dflt, cfg,
+                                                    pick_adaptive<bhp::SampleWork>(o.precision, v, cfg.waves));
+    const int grid = plan.grid;
     if (ordered) {
         if ((rc = ensure(c, &c->d_order, &c->order_cap, (size_t)tiles)) ||
             (rc = ensure(c, &c->d_ohist, &c->ohist_cap, (size_t)ORDER_BUCKETS)))
@@ -1530,7 +1580,9 @@ int launch_adaptive(bh_ctx* c, const bh_frame* f, const bh_trace_opts* opts, lon
             if (!c->tuned_ok[o.precision]) cfg = dflt;
             rc = resolve_cfg(c, dflt, &cfg);
             if (rc) return rc;
-            const auto plan = plan_persist<bhp::ChunkWork>(c, o.precision, v, (long long)total * ADAPT_CHUNK, dflt, cfg,
+            const bh_scene* scene = &c->S;
+            const launch::Load load = load_of(c, o.precision, v, B, &scene, 1, (long long)total * ADAPT_CHUNK, false);
+            const auto plan = plan_persist<bhp::ChunkWork>(c, load, v, dflt, cfg,
                                                            pick_adaptive<bhp::ChunkWork>(o.precision, v, cfg.waves));
             grid = plan.grid;
             if ((rc = ensure(c, &c->d_samp2, &c->samp2_cap, (size_t)total * ADAPT_CHUNK)) ||

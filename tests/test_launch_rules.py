@@ -1,0 +1,56 @@
+"""The rules that shape a persistent launch (csrc/launch.h), compiled with the host compiler: which radio launches
+integrate and evaluate in two waves, by the number of rays, how many of them reach the emitting region, and
+whether the flow is opaque; and the share of a region's rays that pass within a radius, against the area."""
+import math
+import os
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+FP64, MIXED = 0, 1
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    exe = str(tmp_path_factory.mktemp("rules") / "rules")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-Wall", "-Wextra", "-Werror", "-o", exe,
+                    os.path.join(HERE, "launch_rules", "rules.cpp")], check=True)
+
+    def ask(*lines):
+        out = subprocess.run([exe], input="\n".join(lines) + "\n", capture_output=True, text=True, check=True).stdout
+        return [float(x) for x in out.split()]
+    return ask
+
+
+@pytest.mark.parametrize("prec,w,reach,opaque,want", [
+    (FP64, 0.1, 0.1, 0, 1), (FP64, 10.0, 10.0, 0, 1), (FP64, 10.1, 10.1, 0, 0), (FP64, 9.0, 9.0, 1, 1),
+    (MIXED, 0.1, 0.1, 1, 1), (MIXED, 12.0, 12.0, 1, 1), (MIXED, 12.3, 12.3, 1, 0),   # an opaque flow, all rays in it
+    (MIXED, 25.0, 11.0, 1, 1), (MIXED, 25.0, 15.0, 1, 0),                            # few of them in it
+    (MIXED, 22.6, 22.6, 0, 1), (MIXED, 25.0, 25.0, 0, 0),                            # a thin one, all rays in it
+    (MIXED, 39.8, 17.0, 0, 1), (MIXED, 40.1, 1.0, 0, 0),
+])
+def test_pairs(rules, prec, w, reach, opaque, want):
+    assert rules(f"{prec} 1 {w} {reach} {opaque}") == [want]
+    assert rules(f"{prec} 0 {w} {reach} {opaque}") == [0]   # vacuum: nothing to evaluate
+
+
+@pytest.mark.parametrize("r,fov,w,h,want", [
+    (10.0, 40.0, 1024, 1024, math.pi / 16), (100.0, 40.0, 640, 480, 1.0), (0.0, 40.0, 64, 64, 0.0),
+    (15.0, 40.0, 512, 256, None),
+])
+def test_share(rules, r, fov, w, h, want):
+    pix = fov / w / 1000.0
+    got, = rules(f"share {r} 1000 0 0 {pix!r} {w} {h} 0 0 {w} {h}")
+    if want is None:   # a frame twice as wide as high: the disc is cut at |y| = 10
+        y = fov * h / w / 2
+        want = (2 * (y * math.sqrt(r * r - y * y) + r * r * math.asin(y / r))) / (fov * fov * h / w)
+    assert abs(got - want) <= 0.05   # 256 sample points: the edge passes through some 40 of them
+
+
+def test_share_off_centre(rules):
+    pix = 40.0 / 1000 / 1000.0
+    # a frame beside the disc, one inside it, a region of a frame that holds the disc, one that misses it
+    assert rules(f"share 10 1000 0.05 0 {pix!r} 1000 1000 0 0 1000 1000", f"share 30 1000 0 0 {pix!r} 1000 1000 0 0 1000 1000",
+                 f"share 10 1000 0 0 {pix!r} 1000 1000 400 400 200 200",
+                 f"share 10 1000 0 0 {pix!r} 1000 1000 0 0 200 200") == [0.0, 1.0, 1.0, 0.0]
