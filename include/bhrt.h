@@ -123,8 +123,8 @@ typedef struct bh_trace_opts {
                          absorption and the step cap over the whole flow as the FP64 tracer, with
                          tol_mid = max(1e-6, tol) */
     int engine;       /* bh_render / bh_render_resident / bh_trace_tile: BH_ENGINE_AUTO (0) -> the
-                         persistent engine (bh_autotune's last result for this precision, or the
-                         defaults): one sample per pixel as bh_trace_batch of one frame, more as the
+                         persistent engine (bh_autotune's last result for this precision, where it
+                         holds, or the defaults): one sample per pixel as bh_trace_batch of one frame, more as the
                          first pass of bh_render_adaptive alone; frames beyond 2^31 samples, or whose
                          samples would take more than 1 GiB (32 bytes each), on the frame kernel.
                          BH_ENGINE_FRAME -> always the frame kernel. Both give the same pixels,
@@ -206,7 +206,7 @@ int bh_render_noalloc(bh_ctx* ctx, const bh_frame* frame, const bh_trace_opts* o
 /* Tile interface (k_pass1's per-pixel launch, render.cu:89-128, with every per-ray output): rays of
    pixels x0 <= px < x0+w, y0 <= py < y0+h, one sample each (centre or jittered sample 0), written
    row-major to out[w*h]. opts->engine BH_ENGINE_AUTO (0): the persistent engine with bh_autotune's
-   last launch for the precision (or the defaults); BH_ENGINE_FRAME: the frame kernel. Both give the
+   last launch for the precision, where it holds (or the defaults); BH_ENGINE_FRAME: the frame kernel. Both give the
    same records. */
 int bh_trace_tile(bh_ctx* ctx, const bh_frame* frame, int x0, int y0, int w, int h, const bh_trace_opts* opts,
                   bh_ray_out* out);
@@ -257,13 +257,14 @@ typedef struct bh_batch_cfg {
                            which grows with the number of orbits near the critical curve); 0 -> the
                            default */
     int prio_age;       /* > 0: a wave holding a ray that has taken prio_age steps raises its issue
-                           priority; < 0: off; 0 -> the default. The defaults (a NULL cfg, no autotuned one)
-                           follow the launch's number of rays: from workgroups of one wave, one wave or fewer
-                           per SIMD, for launches that hold all their rays at once, to 256 threads and three
-                           waves per SIMD; rows order for the largest FP64 launches and those without
-                           generations, else critical; interval 64, refill_min 32 (mixed) / 48 (FP64), graph,
-                           waves 3, prio_age 256. Radio launches of few rays (to 40 waves per CU mixed, 10
-                           FP64) integrate and evaluate in two waves side by side then; same results. */
+                           priority; < 0: off; 0 -> the default (mixed 128, FP64 256).
+                           The defaults (a NULL cfg and no autotuned one that holds) follow the launch's
+                           number of rays, from workgroups of one wave, one or fewer per SIMD, to 256
+                           threads and three waves per SIMD; the other fields: interval 64, refill_min 32
+                           (mixed) / 48 (FP64), graph, waves 3, critical order (FP64: row order for the
+                           fewest and the most rays). Radio launches of few rays have the shape 64 / 4 /
+                           waves 3, and with this shape, given or not, integrate and evaluate 64 rays in two
+                           waves side by side; same results. */
 } bh_batch_cfg;
 
 /* Traces every frame of `frames`; px_out (nullable) receives the frames one after the other,
@@ -272,7 +273,9 @@ int bh_trace_batch(bh_ctx* ctx, const bh_batch_frame* frames, int n, const bh_tr
                    const bh_batch_cfg* cfg, float* px_out, bh_stats* stats);
 
 /* Times bh_trace_batch over a grid of configurations on the given workload and returns the fastest
-   (best) with its kernel time (best_ms): the median of three timed launches after a warm-up one. tried
+   (best) with its kernel time (best_ms): the median of three timed launches after a warm-up one. Later
+   calls without a cfg use it for launches whose defaults are those of this workload (the same precision,
+   with or without a flow, the same class of sizes); other launches keep their own defaults. tried
    (nullable, 8 doubles per configuration: block, grid_per_cu, interval, refill_min, ms, waves, order,
    prio_age) receives up to max_tried rows;
    *n_tried their number. */

@@ -1095,52 +1095,6 @@ int persist_grid(const bh_ctx* c, const void* k, int block, int grid_per_cu) {
 constexpr size_t PLAIN_SPP_SAMPLE_BUDGET = size_t(1) << 30;   // bytes of per-sample storage of bh_render, spp > 1
 constexpr long long BATCH_MAX_PIXELS = 1ll << 30;   // per frame: keeps the 32-bit queue counters from wrapping
 
-/* Defaults of a persistent launch of `entries` rays (all frames). w = waves of rays per compute unit; a
-   CU holds 12 waves of these kernels (3 per SIMD). Measured on frames of 32^2 to 2048^2 (MI355X, ms of
-   the launch):
-   - A SIMD issues one wave's instructions at half its rate, so 2 waves fill it and a third covers the
-     stalls; but the longest rays set the end of a launch, and each of their instructions waits for the
-     SIMD's other waves. Few rays are therefore spread thinly - and evenly: the waves that find no ray
-     exit, and with 3 resident waves per SIMD which SIMD they leave idle is chance. 256^2 vacuum, FP64:
-     4.2 with 12 waves per CU, 2.8 with 3; 512^2 radio, FP64: 8.7 with 12, 6.0 with 8; 1024^2: 18.3 with
-     12. Mixed radio, 256^2: 2.16 with 8, 2.01 with 4; 1400^2: 4.82 with 8, 4.17 with 12; zoom 768^2:
-     13.5 with 8, 11.9 with 12 (every ray is long: throughput, from 8 waves of rays per CU on).
-   - Longest rays first (critical order) where several generations of rays share the launch, but not so
-     many that its tail no longer counts: FP64 radio 384^2 6.0 -> 4.8, 768^2 11.3 -> 11.1, 1024^2 18.3
-     -> 18.9, 1500^2 37.6 -> 39.9. A launch that holds all its rays at once needs no sort. The mixed
-     tracer's rays differ by over 10x in length: always.
-   - Workgroups of one wave where they are few, so that the dispatcher can place each on its own. */
-bh_batch_cfg batch_defaults(const bh_ctx* c, int prec, const Variant& v, long long entries) {
-    bh_batch_cfg d{};
-    const double w = (double)entries / 64.0 / c->n_cu;
-    d.use_graph = 1;
-    d.waves = 3;
-    d.interval = 64;
-    d.prio_age = prec == BH_PREC_MIXED ? 128 : 256;
-    if (prec == BH_PREC_MIXED) {
-        const bool vacuum = v.radio == bhd::RADIO_OFF;
-        const int per_cu = w <= (vacuum ? 8.0 : launch::PAIR_REACH_OPAQUE) ? 4 : (!vacuum && w <= 48.0 ? 8 : 12);
-        d.block = per_cu == 4 && !vacuum ? 64 : 256;
-        d.grid_per_cu = per_cu * 64 / d.block;
-        d.refill_min = 32;
-        d.order = BH_ORDER_CRITICAL;
-    } else {
-        d.block = w <= 20.0 ? 64 : 256;
-        d.grid_per_cu = w <= 5.0 ? 3 : (w <= 7.0 ? 4 : (w <= 20.0 ? 8 : 3));
-        d.refill_min = 48;
-        d.order = w > 5.0 && w <= 48.0 ? BH_ORDER_CRITICAL : BH_ORDER_ROWS;
-    }
-    return d;
-}
-
-// Queue entries of a batch: the pixels of whole 8 x 8 tiles (frame sizes are checked later)
-long long batch_entries(const bh_batch_frame* frames, int n) {
-    long long e = 0;
-    for (int i = 0; i < n; ++i)
-        e += (long long)((std::max(frames[i].frame.W, 0) + 7ll) / 8) * ((std::max(frames[i].frame.H, 0) + 7ll) / 8) * 64;
-    return e;
-}
-
 // Replaces the 0 ("default") fields of a launch configuration and checks the ranges.
 int resolve_cfg(bh_ctx* c, const bh_batch_cfg& d, bh_batch_cfg* g) {
     if (g->block == 0) g->block = d.block;
@@ -1188,8 +1142,8 @@ launch::Load load_of(bh_ctx* c, int prec, const Variant& v, const bhp::BatchFram
     return l;
 }
 
-// The kernel and grid of a persistent launch: two waves per 64 rays where launch::pairs says so, with the
-// default configuration; another one, given or tuned, keeps its kernel.
+// The kernel and grid of a persistent launch: two waves per 64 rays where launch::pairs and the
+// configuration's shape say so, else the kernel `plain`.
 template <class Work>
 struct PersistPlan {
     WorkFn<Work> k;
@@ -1197,19 +1151,14 @@ struct PersistPlan {
 };
 
 template <class Work>
-PersistPlan<Work> plan_persist(const bh_ctx* c, const launch::Load& load, const Variant& v, const bh_batch_cfg& dflt,
-                               const bh_batch_cfg& g, WorkFn<Work> plain) {
-    const bool as_default = g.block == dflt.block && g.grid_per_cu == dflt.grid_per_cu && g.interval == dflt.interval &&
-                            g.refill_min == dflt.refill_min && g.waves == dflt.waves && g.order == dflt.order &&
-                            g.prio_age == dflt.prio_age;
+PersistPlan<Work> plan_persist(const bh_ctx* c, const launch::Load& load, const Variant& v, const bh_batch_cfg& g,
+                               WorkFn<Work> plain) {
     PersistPlan<Work> p{plain, g.block, 0};
-    int per_cu = g.grid_per_cu;
-    if (as_default && launch::pairs(load)) {
+    if (launch::pairs(load) && launch::pair_shape(g)) {
         p.k = pick_pair<Work>(load.precision, v);
         p.block = bhp::PAIR_BLOCK;
-        per_cu = 4;
     }
-    p.grid = persist_grid(c, (const void*)p.k, p.block, per_cu);
+    p.grid = persist_grid(c, (const void*)p.k, p.block, g.grid_per_cu);
     return p;
 }
 
@@ -1231,8 +1180,9 @@ void enqueue_tile_order(hipStream_t st, const bhp::BatchFrame* dframes, int n, u
 
 // Traces a batch with one persistent launch: [queue reset, k_persist, k_reduce], captured into a
 // hipGraph (rebuilt when a buffer, the kernel or the launch shape changes) or launched directly.
+// cfg_out (nullable): the configuration with its defaults filled in.
 int launch_batch(bh_ctx* c, const bh_batch_frame* frames, int n, const bh_trace_opts* opts, const bh_batch_cfg* cfg_in,
-                 long long* npix_out, bh_stats* st) {
+                 long long* npix_out, bh_stats* st, bh_batch_cfg* cfg_out = nullptr) {
     if (!frames || n <= 0) return fail(c, BH_ERR_ARG, "empty batch");
     bh_trace_opts o{};
     if (opts) o = *opts;
@@ -1241,10 +1191,6 @@ int launch_batch(bh_ctx* c, const bh_batch_frame* frames, int n, const bh_trace_
     // one kernel for all frames: it integrates the coordinate time if any of them reads it
     Variant v = variant_of(c, frames[0].scene, o);
     for (int i = 1; i < n; ++i) v.time = v.time || variant_of(c, frames[i].scene, o).time;
-    const bh_batch_cfg dflt = batch_defaults(c, o.precision, v, batch_entries(frames, n));
-    bh_batch_cfg cfg = cfg_in ? *cfg_in : (c->tuned_ok[o.precision] ? c->tuned[o.precision] : dflt);
-    rc = resolve_cfg(c, dflt, &cfg);
-    if (rc) return rc;
     const int mode = frames[0].scene.mode;
     if (c->turb_model == BH_TURB_SHEARED) {
         // one set of slices per launch: every frame must see the same turbulence bake
@@ -1262,7 +1208,7 @@ int launch_batch(bh_ctx* c, const bh_batch_frame* frames, int n, const bh_trace_
         rc = prepare_turbulence(c, frames[0].scene, &frames[0].frame);
         if (rc) return rc;
     }
-    long long total = 0;
+    long long total = 0, entries = 0;
     std::vector<bhp::BatchFrame> hb((size_t)n);
     std::vector<const bh_scene*> scenes((size_t)n);
     for (int i = 0; i < n; ++i) {
@@ -1288,8 +1234,15 @@ int launch_batch(bh_ctx* c, const bh_batch_frame* frames, int n, const bh_trace_
         }
         B.tiles_x = (f->W + 7) / 8;
         B.nentries = (unsigned int)((long long)B.tiles_x * ((f->H + 7) / 8) * 64);
+        entries += B.nentries;
         total += (long long)f->W * f->H;
     }
+    const launch::Load load = load_of(c, o.precision, v, hb.data(), scenes.data(), n, entries, true);
+    const bh_batch_cfg dflt = launch::defaults(load);
+    bh_batch_cfg cfg = cfg_in ? *cfg_in : launch::choose(c->tuned[o.precision], load, dflt);
+    rc = resolve_cfg(c, dflt, &cfg);
+    if (rc) return rc;
+    if (cfg_out) *cfg_out = cfg;
     rc = ensure(c, &c->d_bout, &c->bout_cap, (size_t)total);
     if (rc) return rc;
     long long off = 0;
@@ -1314,8 +1267,7 @@ int launch_batch(bh_ctx* c, const bh_batch_frame* frames, int n, const bh_trace_
         }
     }
     const int prio = cfg.prio_age > 0 ? cfg.prio_age : 0;
-    const launch::Load load = load_of(c, o.precision, v, hb.data(), scenes.data(), n, batch_entries(frames, n), true);
-    const auto plan = plan_persist<bhp::BatchWork>(c, load, v, dflt, cfg, pick_persist(o.precision, v, cfg.waves));
+    const auto plan = plan_persist<bhp::BatchWork>(c, load, v, cfg, pick_persist(o.precision, v, cfg.waves));
     const PersistFn k = plan.k;
     const int grid = plan.grid;
     rc = ensure(c, &c->d_bframes, &c->bframes_cap, sizeof(bhp::BatchFrame) * (size_t)n);
@@ -1405,10 +1357,6 @@ int launch_records(bh_ctx* c, const bh_frame* f, const bh_trace_opts* opts, int 
     if (rc) return rc;
     const int tiles_x = (w + 7) / 8, tiles = tiles_x * ((h + 7) / 8);
     const Variant v = variant_of(c, c->S, o);
-    const bh_batch_cfg dflt = batch_defaults(c, o.precision, v, (long long)tiles * 64);
-    bh_batch_cfg cfg = c->tuned_ok[o.precision] ? c->tuned[o.precision] : dflt;
-    rc = resolve_cfg(c, dflt, &cfg);
-    if (rc) return rc;
     rc = prepare_turbulence(c, c->S, f);
     if (rc) return rc;
     bhp::BatchFrame B;
@@ -1429,7 +1377,8 @@ int launch_records(bh_ctx* c, const bh_frame* f, const bh_trace_opts* opts, int 
     B.nentries = (unsigned int)tiles * 64u;
     const bh_scene* scene = &c->S;
     const launch::Load load = load_of(c, o.precision, v, &B, &scene, 1, (long long)tiles * 64, true);
-    const auto plan = plan_persist<bhp::RecordWork>(c, load, v, dflt, cfg,
+    const bh_batch_cfg cfg = launch::choose(c->tuned[o.precision], load, launch::defaults(load));
+    const auto plan = plan_persist<bhp::RecordWork>(c, load, v, cfg,
                                                     pick_adaptive<bhp::RecordWork>(o.precision, v, cfg.waves));
     const int grid = plan.grid;
     const bool ordered = cfg.order != BH_ORDER_ROWS;
@@ -1461,13 +1410,8 @@ int launch_samples(bh_ctx* c, const bh_frame* f, const bh_trace_opts& o, int spp
     const int W = f->W, H = f->H;
     const int tiles_x = (W + 7) / 8, tiles = tiles_x * ((H + 7) / 8);
     const Variant v = variant_of(c, c->S, o);
-    const bh_batch_cfg dflt = batch_defaults(c, o.precision, v, (long long)tiles * 64 * spp);
-    bh_batch_cfg cfg = c->tuned_ok[o.precision] ? c->tuned[o.precision] : dflt;
-    int rc = resolve_cfg(c, dflt, &cfg);
+    int rc = prepare_turbulence(c, c->S, f);
     if (rc) return rc;
-    rc = prepare_turbulence(c, c->S, f);
-    if (rc) return rc;
-    const bool ordered = cfg.order != BH_ORDER_ROWS;
     std::memset(B, 0, 2 * sizeof B[0]);
     B[0].P = make_params(c, f);
     B[0].P.w = W;
@@ -1483,9 +1427,11 @@ int launch_samples(bh_ctx* c, const bh_frame* f, const bh_trace_opts& o, int spp
     B[0].nentries = (unsigned int)(tiles * 64 * spp);
     const bh_scene* scene = &c->S;
     const launch::Load load = load_of(c, o.precision, v, B, &scene, 1, (long long)tiles * 64 * spp, true);
-    const auto plan = plan_persist<bhp::SampleWork>(c, load, v, dflt, cfg,
+    const bh_batch_cfg cfg = launch::choose(c->tuned[o.precision], load, launch::defaults(load));
+    const auto plan = plan_persist<bhp::SampleWork>(c, load, v, cfg,
                                                     pick_adaptive<bhp::SampleWork>(o.precision, v, cfg.waves));
     const int grid = plan.grid;
+    const bool ordered = cfg.order != BH_ORDER_ROWS;
     if (ordered) {
         if ((rc = ensure(c, &c->d_order, &c->order_cap, (size_t)tiles)) ||
             (rc = ensure(c, &c->d_ohist, &c->ohist_cap, (size_t)ORDER_BUCKETS)))
@@ -1576,13 +1522,10 @@ int launch_adaptive(bh_ctx* c, const bh_frame* f, const bh_trace_opts* opts, lon
         if (total > 0) {
             // pass 2's launch by its own number of rays
             const Variant v = variant_of(c, c->S, o);
-            const bh_batch_cfg dflt = batch_defaults(c, o.precision, v, (long long)total * ADAPT_CHUNK);
-            if (!c->tuned_ok[o.precision]) cfg = dflt;
-            rc = resolve_cfg(c, dflt, &cfg);
-            if (rc) return rc;
             const bh_scene* scene = &c->S;
             const launch::Load load = load_of(c, o.precision, v, B, &scene, 1, (long long)total * ADAPT_CHUNK, false);
-            const auto plan = plan_persist<bhp::ChunkWork>(c, load, v, dflt, cfg,
+            cfg = launch::choose(c->tuned[o.precision], load, launch::defaults(load));
+            const auto plan = plan_persist<bhp::ChunkWork>(c, load, v, cfg,
                                                            pick_adaptive<bhp::ChunkWork>(o.precision, v, cfg.waves));
             grid = plan.grid;
             if ((rc = ensure(c, &c->d_samp2, &c->samp2_cap, (size_t)total * ADAPT_CHUNK)) ||
@@ -1969,13 +1912,15 @@ int bh_autotune(bh_ctx* c, const bh_batch_frame* frames, int n, const bh_trace_o
     // coordinate descent from the defaults: one parameter at a time over its candidate list, two passes
     const int prec = opts ? opts->precision : BH_PREC_FP64;
     if (!frames || n <= 0) return fail(c, BH_ERR_ARG, "empty batch");
-    const Variant v = variant_of(c, frames[0].scene, opts ? *opts : bh_trace_opts{});
-    bh_batch_cfg cur = batch_defaults(c, prec, v, batch_entries(frames, n));
+    bh_batch_cfg cur{};   // the defaults, filled in by the first timed launches
+    cur.use_graph = 1;
+    cur.waves = 3;
     int count = 0;
     double cur_ms = 0.0;
-    auto time_cfg = [&](const bh_batch_cfg& g, double* ms) -> int {
+    auto time_cfg = [&](const bh_batch_cfg& asked, double* ms, bh_batch_cfg* filled) -> int {
         bh_stats s{};
-        int rc = launch_batch(c, frames, n, opts, &g, nullptr, &s);   // first run: warm caches and graph
+        bh_batch_cfg g;
+        int rc = launch_batch(c, frames, n, opts, &asked, nullptr, &s, &g);   // first run: warm caches and graph
         if (rc) return rc;
         double t[3];   // the median of three timed runs (launch-to-launch spread is up to 10 %)
         for (int rep = 0; rep < 3; ++rep) {
@@ -1997,10 +1942,12 @@ int bh_autotune(bh_ctx* c, const bh_batch_frame* frames, int n, const bh_trace_o
             row[7] = g.prio_age;
         }
         ++count;
+        if (filled) *filled = g;
         return BH_OK;
     };
-    int rc = time_cfg(cur, &cur_ms);
+    int rc = time_cfg(cur, &cur_ms, &cur);
     if (rc) return rc;
+    const bh_batch_cfg from = cur;
     const int blocks[] = {64, 128, 256}, grids[] = {1, 2, 3, 4, 8}, intervals[] = {2, 4, 8, 16, 32, 64},
               refills[] = {1, 8, 16, 32, 48}, waves[] = {0, 3, 4},
               orders[] = {BH_ORDER_ROWS, BH_ORDER_IMPACT, BH_ORDER_CRITICAL}, ages[] = {-1, 64, 128, 256, 512};
@@ -2016,7 +1963,7 @@ int bh_autotune(bh_ctx* c, const bh_batch_frame* frames, int n, const bh_trace_o
                 if (*field == vals[i]) continue;
                 *field = vals[i];
                 double ms;
-                rc = time_cfg(g, &ms);
+                rc = time_cfg(g, &ms, nullptr);
                 if (rc) return rc;
                 if (ms < cur_ms) {
                     cur = g;
@@ -2028,8 +1975,7 @@ int bh_autotune(bh_ctx* c, const bh_batch_frame* frames, int n, const bh_trace_o
     *best = cur;
     if (best_ms) *best_ms = cur_ms;
     if (n_tried) *n_tried = count;
-    c->tuned[prec] = cur;   // the precision was checked by the timed launches
-    c->tuned_ok[prec] = true;
+    c->tuned[prec] = launch::Tuned{true, frames[0].scene.mode == BH_MODE_RADIO, from, cur};   // the launches checked prec
     return BH_OK;
 }
 

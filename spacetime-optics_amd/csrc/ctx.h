@@ -8,6 +8,7 @@
 #include <vector>
 
 #include "../../include/bhrt.h"
+#include "launch.h"
 #include "mlp.h"
 #include "trace_fp64.h"
 #include "transfer.h"
@@ -104,7 +105,6 @@ struct bh_ctx {
     double4* d_samp2 = nullptr;
     size_t samp2_cap = 0;
     int n_cu = 0;
-    bh_batch_cfg tuned[2]{};   // last bh_autotune result per precision (used when no cfg is given)
-    bool tuned_ok[2]{};
+    launch::Tuned tuned[2]{};   // last bh_autotune result per precision (for launches like it when no cfg is given)
     std::string err;
 };

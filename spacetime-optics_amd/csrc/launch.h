@@ -49,4 +49,61 @@ inline bool pairs(const Load& l) {
     return l.w <= PAIR_W_MIXED && l.reach <= (l.opaque ? PAIR_REACH_OPAQUE : PAIR_REACH);
 }
 
+constexpr int PAIR_RAYS = 64, PAIR_PER_CU = 4;   // the shape of such a launch: rays of a workgroup, workgroups of a CU
+
+// Whether a resolved configuration asks for it where the load does: by its shape (interval, refill_min and order
+// hold for both kernels, prio_age for the other one only)
+inline bool pair_shape(const bh_batch_cfg& g) { return g.block == PAIR_RAYS && g.grid_per_cu == PAIR_PER_CU && g.waves == 3; }
+
+/* Defaults. Measured on frames of 32^2 to 2048^2:
+   - A SIMD issues one wave's instructions at half its rate, so 2 waves fill it and a third covers the
+     stalls; but the longest rays set the end of a launch, and each of their instructions waits for the
+     SIMD's other waves. Few rays are therefore spread thinly - and evenly: the waves that find no ray
+     exit, and with 3 resident waves per SIMD which SIMD they leave idle is chance. 256^2 vacuum, FP64:
+     4.2 with 12 waves per CU, 2.8 with 3; 512^2 radio, FP64: 8.7 with 12, 6.0 with 8; 1024^2: 18.3 with
+     12. Mixed radio: 1400^2 4.82 with 8, 4.17 with 12; zoom 768^2: 13.5 with 8, 11.9 with 12 (every ray is
+     long: throughput, from 8 waves of rays per CU on).
+   - Longest rays first (critical order) where several generations of rays share the launch, but not so
+     many that its tail no longer counts: FP64 radio 384^2 6.0 -> 4.8, 768^2 11.3 -> 11.1, 1024^2 18.3
+     -> 18.9, 1500^2 37.6 -> 39.9. The mixed tracer's rays differ by over 10x in length: always.
+   - Workgroups of one wave where they are few, so that the dispatcher can place each on its own. */
+inline bh_batch_cfg defaults(const Load& l) {
+    bh_batch_cfg d{};
+    const bool mixed = l.precision == BH_PREC_MIXED;
+    d.use_graph = 1;
+    d.waves = 3;
+    d.interval = 64;
+    d.refill_min = mixed ? 32 : 48;
+    d.prio_age = mixed ? 128 : 256;
+    d.order = mixed || (l.w > 5.0 && l.w <= 48.0) ? BH_ORDER_CRITICAL : BH_ORDER_ROWS;
+    if (pairs(l)) {
+        d.block = PAIR_RAYS;
+        d.grid_per_cu = PAIR_PER_CU;
+    } else if (mixed) {
+        d.block = 256;
+        d.grid_per_cu = l.radio == 0 ? (l.w <= 8.0 ? 1 : 3) : (l.w <= 48.0 ? 2 : 3);
+    } else {
+        d.block = l.w <= 20.0 ? 64 : 256;
+        d.grid_per_cu = l.w <= 5.0 ? 3 : (l.w <= 7.0 ? 4 : (l.w <= 20.0 ? 8 : 3));
+    }
+    return d;
+}
+
+/* A tuned configuration stands in for the defaults it was tuned from, and for no others: what is best for 1024^2
+   rays is not for 64^2 (FP64, tuned at 64^2, then 1024^2: 36.1 for 19.7; mixed, the other way round: 1.35 for
+   1.02). */
+struct Tuned {
+    bool ok = false;
+    int radio = 0;
+    bh_batch_cfg from{}, cfg{};
+};
+
+inline const bh_batch_cfg& choose(const Tuned& t, const Load& l, const bh_batch_cfg& dflt) {
+    const bh_batch_cfg &a = t.from, &b = dflt;
+    const bool same = t.ok && (t.radio != 0) == (l.radio != 0) && a.block == b.block && a.grid_per_cu == b.grid_per_cu &&
+                      a.interval == b.interval && a.refill_min == b.refill_min && a.waves == b.waves &&
+                      a.order == b.order && a.prio_age == b.prio_age;
+    return same ? t.cfg : dflt;
+}
+
 }  // namespace launch

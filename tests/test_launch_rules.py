@@ -1,6 +1,7 @@
 """The rules that shape a persistent launch (csrc/launch.h), compiled with the host compiler: which radio launches
 integrate and evaluate in two waves, by the number of rays, how many of them reach the emitting region, and
-whether the flow is opaque; and the share of a region's rays that pass within a radius, against the area."""
+whether the flow is opaque; the share of a region's rays that pass within a radius, against the area; the
+defaults at either side of their lines; and which launches a tuned configuration holds for."""
 import math
 import os
 import subprocess
@@ -54,3 +55,32 @@ def test_share_off_centre(rules):
     assert rules(f"share 10 1000 0.05 0 {pix!r} 1000 1000 0 0 1000 1000", f"share 30 1000 0 0 {pix!r} 1000 1000 0 0 1000 1000",
                  f"share 10 1000 0 0 {pix!r} 1000 1000 400 400 200 200",
                  f"share 10 1000 0 0 {pix!r} 1000 1000 0 0 200 200") == [0.0, 1.0, 1.0, 0.0]
+
+
+@pytest.mark.parametrize("load,want", [
+    ("0 1 0.1 0.1 0", [64, 4, 1, 1]), ("0 1 10 10 0", [64, 4, 3, 1]), ("0 1 10.1 10.1 0", [64, 8, 3, 0]),
+    ("0 1 20.1 20.1 0", [256, 3, 3, 0]), ("0 2 64 64 0", [256, 3, 1, 0]),
+    ("0 0 2.9 2.9 0", [64, 3, 1, 0]), ("0 0 6.9 6.9 0", [64, 4, 3, 0]), ("0 0 7.1 7.1 0", [64, 8, 3, 0]),
+    ("1 1 0.1 0.1 0", [64, 4, 3, 1]), ("1 2 39.9 17 0", [64, 4, 3, 1]), ("1 1 20 20 1", [256, 2, 3, 0]),
+    ("1 1 48.1 9 0", [256, 3, 3, 0]), ("1 0 8 8 0", [256, 1, 3, 0]), ("1 0 8.1 8.1 0", [256, 3, 3, 0]),
+])
+def test_defaults(rules, load, want):
+    assert rules(f"defaults {load}") == want
+
+
+SMALL, LARGE, VACUUM = "{p} 1 1 1 0", "{p} 1 64 30 0", "{p} 0 64 64 0"
+
+
+@pytest.mark.parametrize("p", [FP64, MIXED])
+def test_tuned_holds_for_launches_like_it(rules, p):
+    small, large, vacuum = (x.format(p=p) for x in (SMALL, LARGE, VACUUM))
+    # tuned on many rays: holds for as many and more, not for few, which keep the two waves
+    assert rules(f"tuned {large} {large} 128 8 32") == [128, 8, 32, 0]
+    assert rules(f"tuned {large} {p} 1 300 200 0 128 8 32") == [128, 8, 32, 0]
+    assert rules(f"tuned {large} {small} 128 8 32") == [64, 4, 64, 1]
+    # tuned on few rays: the shape of a launch that waits for its longest ray is not forced on many
+    assert rules(f"tuned {small} {small} 64 4 16") == [64, 4, 16, 1]
+    assert rules(f"tuned {small} {small} 64 1 64") == [64, 1, 64, 0]
+    assert rules(f"tuned {small} {large} 64 1 64")[:2] != [64, 1]
+    # tuned with a flow, used without one
+    assert rules(f"tuned {large} {vacuum} 128 8 32")[0] == 256
