@@ -7,6 +7,9 @@
    filled slot to the caller's pages while the next is on its way. Copies below MIN_BYTES, and into memory
    that is already pinned, go straight to the runtime; so do copies to the device, which it moves at 30
    GB/s (the same threads measured no faster).
+   The threads are woken when the first slot is filled: whatever the stream has to do before the copy, they
+   sleep. From then on the slots fill at the link's rate and they wait by yielding. There are at most as many as
+   the process has cores (affinity, and the control group's quota); with one or two the runtime's path is taken.
    One Transfer per device serves all of its contexts (16 MiB of pinned memory take milliseconds to get)
    and ends with the last of them; it runs one copy at a time, and a copy that finds it busy takes the
    runtime's path. Measured (MI355X, 16 host cores), runtime -> threads: 3 MiB into
@@ -14,11 +17,13 @@
    0.14, 64 MiB 3.8 -> 1.5. */
 #pragma once
 #include <hip/hip_runtime.h>
+#include <sched.h>
 
 #include <algorithm>
 #include <atomic>
 #include <condition_variable>
 #include <cstddef>
+#include <cstdio>
 #include <cstring>
 #include <map>
 #include <memory>
@@ -71,14 +76,7 @@ class Transfer {
         bytes_ = bytes;
         piece_ = piece;
         pieces_ = (bytes + piece - 1) / piece;
-        filled_.store(0, std::memory_order_relaxed);
         for (Slot& s : slots_) s.moved.store(0, std::memory_order_relaxed);
-        {
-            std::lock_guard<std::mutex> lock(mu_);
-            left_ = THREADS - 1;
-            ++turn_;
-        }
-        wake_.notify_all();
         hipError_t err = hipSuccess;
         auto fill = [&](size_t i) {
             Slot& s = slots_[i % SLOTS];
@@ -87,13 +85,27 @@ class Transfer {
             if (err == hipSuccess) err = hipEventRecord(s.filled, st);
         };
         for (size_t i = 0; i < std::min<size_t>(pieces_, SLOTS); ++i) fill(i);
+        if (err == hipSuccess) err = hipEventSynchronize(slots_[0].filled);
+        if (err != hipSuccess) {   // the threads have not been woken
+            (void)hipStreamSynchronize(st);
+            return err;
+        }
+        filled_.store(1, std::memory_order_relaxed);
+        {
+            std::lock_guard<std::mutex> lock(mu_);
+            left_ = count_ - 1;
+            ++turn_;
+        }
+        wake_.notify_all();
         for (size_t i = 0; i < pieces_; ++i) {
-            if (err == hipSuccess) err = hipEventSynchronize(slots_[i % SLOTS].filled);
-            if (err != hipSuccess) failed_.store(true, std::memory_order_relaxed);   // then nothing more is moved
-            filled_.store(i + 1, std::memory_order_release);
+            if (i > 0) {
+                if (err == hipSuccess) err = hipEventSynchronize(slots_[i % SLOTS].filled);
+                if (err != hipSuccess) failed_.store(true, std::memory_order_relaxed);   // then nothing more is moved
+                filled_.store(i + 1, std::memory_order_release);
+            }
             move_share(0, i);
             if (i + SLOTS < pieces_) {   // the slot is free again when every thread has taken its share
-                while (slots_[i % SLOTS].moved.load(std::memory_order_acquire) < THREADS) std::this_thread::yield();
+                while (slots_[i % SLOTS].moved.load(std::memory_order_acquire) < count_) std::this_thread::yield();
                 slots_[i % SLOTS].moved.store(0, std::memory_order_relaxed);
                 fill(i + SLOTS);
             }
@@ -128,16 +140,31 @@ class Transfer {
     // thread t's share of piece i: whole pages of it
     void move_share(int t, size_t i) {
         Slot& s = slots_[i % SLOTS];
-        const size_t n = length(i), share = ((n / THREADS) | 0xfff) + 1;
+        const size_t n = length(i), share = ((n / (size_t)count_) | 0xfff) + 1;
         const size_t a = std::min(n, share * (size_t)t), b = std::min(n, a + share);
         if (a < b && !failed_.load(std::memory_order_relaxed)) std::memcpy(dst_ + i * piece_ + a, s.mem + a, b - a);
         s.moved.fetch_add(1, std::memory_order_release);
+    }
+
+    // cores this process may use: its affinity, and the quota of its control group where there is one
+    static int cores() {
+        cpu_set_t set;
+        int n = sched_getaffinity(0, sizeof set, &set) == 0 ? CPU_COUNT(&set) : (int)std::thread::hardware_concurrency();
+        if (std::FILE* f = std::fopen("/sys/fs/cgroup/cpu.max", "r")) {
+            double quota, period;
+            if (std::fscanf(f, "%lf %lf", &quota, &period) == 2 && period > 0.0)
+                n = std::min(n, std::max(1, (int)(quota / period + 0.5)));
+            std::fclose(f);
+        }
+        return n;
     }
 
     // slots and threads, made at the first large copy; false (and the plain path) if they cannot be had
     bool ready() {
         if (state_ != 0) return state_ > 0;
         state_ = -1;
+        count_ = std::min(THREADS, cores());
+        if (count_ <= 2) return false;
         for (Slot& s : slots_)
             if (hipHostMalloc((void**)&s.mem, SLOT, hipHostMallocDefault) != hipSuccess ||
                 hipEventCreateWithFlags(&s.filled, hipEventDisableTiming) != hipSuccess) {
@@ -145,7 +172,7 @@ class Transfer {
                 return false;
             }
         try {
-            for (int t = 1; t < THREADS; ++t) threads_.emplace_back([this, t] { loop(t); });
+            for (int t = 1; t < count_; ++t) threads_.emplace_back([this, t] { loop(t); });
         } catch (...) {
             return false;   // the threads that did start wait for a copy that never comes, until the end
         }
@@ -173,6 +200,7 @@ class Transfer {
     }
 
     std::mutex busy_;   // one copy at a time
+    int count_ = 0;     // threads, the caller among them
     int state_ = 0;     // 0: not tried, 1: slots and threads are there, -1: the plain path
     Slot slots_[SLOTS];
     std::vector<std::thread> threads_;
