@@ -567,6 +567,16 @@ int ensure(bh_ctx* c, T** p, size_t* cap, size_t n) {
     return BH_OK;
 }
 
+// Whether a buffer can be had; if not, the caller takes a path without it.
+template <typename T>
+bool try_ensure(bh_ctx* c, T** p, size_t* cap, size_t n) {
+    const std::string err = c->err;
+    if (ensure(c, p, cap, n) == BH_OK) return true;
+    (void)hipGetLastError();   // it would be taken for a later launch's
+    c->err = err;
+    return false;
+}
+
 TraceParams make_params_scene(const bh_ctx* c, const bh_scene& S, const bh_frame* f) {
     TraceParams P;
     std::memset(&P, 0, sizeof P);
@@ -1093,6 +1103,7 @@ int persist_grid(const bh_ctx* c, const void* k, int block, int grid_per_cu) {
 }
 
 constexpr size_t PLAIN_SPP_SAMPLE_BUDGET = size_t(1) << 30;   // bytes of per-sample storage of bh_render, spp > 1
+constexpr size_t FLUX_SAMPLES_KEPT = size_t(64) << 20;   // bytes of bh_radio_flux's samples that outlive the call (n = 1024)
 constexpr long long BATCH_MAX_PIXELS = 1ll << 30;   // per frame: keeps the 32-bit queue counters from wrapping
 
 // Replaces the 0 ("default") fields of a launch configuration and checks the ranges.
@@ -1856,14 +1867,16 @@ int bh_radio_flux(bh_ctx* c, const bh_frame* f, int n, double pix_sr, double* jy
     o.jitter = 1;
     o.spp = 2;
     bh_stats st{};
+    int rc = check_frame(c, &g);
+    if (rc) return rc;
     const long long entries = (long long)((n + 7) / 8) * ((n + 7) / 8) * 64 * o.spp;
-    if ((double)entries * sizeof(double4) <= (double)PLAIN_SPP_SAMPLE_BUDGET) {
+    const size_t samples = (size_t)n * n * o.spp, had = c->samp1_cap;
+    if ((double)entries * sizeof(double4) <= (double)PLAIN_SPP_SAMPLE_BUDGET &&
+        try_ensure(c, &c->d_samp1, &c->samp1_cap, samples)) {
         // Each sample a ray of its own on the persistent engine. The frame kernel traces a pixel's two
         // samples one after the other and n = 160 is 100 workgroups for 256 CUs: it ends with the longest
-        // pair of rays on a lane, this with the longest ray (the 230 GHz flow at 17 degrees, three
-        // cameras in turn: 13.7 ms there, 10.6 here).
-        int rc = check_frame(c, &g);
-        if (rc) return rc;
+        // pair of rays on a lane, this with the longest ray (the 0.6 Jy flow at 17 degrees, n = 160, 512,
+        // 1024, 2048: 8.1, 28, 73, 178 ms there, 3.7, 24, 51, 140 here).
         bhp::BatchFrame B[2];
         bh_batch_cfg cfg;
         int grid, per_xcd;
@@ -1879,8 +1892,13 @@ int bh_radio_flux(bh_ctx* c, const bh_frame* f, int n, double pix_sr, double* jy
         HIPCK(c, hipMemcpyAsync(&tot, c->d_tot, sizeof tot, hipMemcpyDeviceToHost, c->st));
         HIPCK(c, hipStreamSynchronize(c->st));
         st.flux_sum = tot.flux;
-    } else {
-        int rc = launch_trace(c, &g, &o, 0, 0, n, n, false, &st);
+        if (samples > had && samples * sizeof(double4) > FLUX_SAMPLES_KEPT) {
+            HIPCK(c, hipFree(c->d_samp1));
+            c->d_samp1 = nullptr;
+            c->samp1_cap = 0;
+        }
+    } else {   // the frame kernel, which needs no memory for them
+        rc = launch_trace(c, &g, &o, 0, 0, n, n, false, &st);
         if (rc) return rc;
     }
     // render.cu:803-808: sum of the per-pixel means times the pixel solid angle, in Jy
