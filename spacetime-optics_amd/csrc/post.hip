@@ -295,6 +295,18 @@ int grow(bh_ctx* c, void** p, size_t* cap, size_t bytes) {
     return BH_OK;
 }
 
+// The buffers of the display statistics: the frame (already there after a blur), Y and the counters
+bool room_for_stats(bh_ctx* c, size_t npix) {
+    const std::string err = c->err;
+    if (grow(c, (void**)&c->d_post_lev, &c->post_lev_cap, sizeof(float4) * npix) == BH_OK &&
+        grow(c, (void**)&c->d_post_tmp, &c->post_tmp_cap, sizeof(float) * npix) == BH_OK &&
+        grow(c, (void**)&c->d_post_wt, &c->post_wt_cap, sizeof(LumState)) == BH_OK)
+        return true;
+    (void)hipGetLastError();   // it would be taken for a later launch's
+    c->err = err;
+    return false;
+}
+
 inline dim3 grid1(long long n) { return dim3((unsigned int)((n + POST_BLOCK - 1) / POST_BLOCK)); }
 
 // Appends to the workgroup's list, in order, the elements i < n that `hit` accepts. Every thread calls it.
@@ -463,16 +475,11 @@ int bh_post_radio(bh_ctx* c, float* px, int W, int H, const bh_post_params* para
     if (lum_percentile || lum_max) {
         const double q = std::min(std::max(percentile, 0.0), 1.0);
         // On the device for all but small frames: its launches take about as long as the host's pass over
-        // 16384 pixels, with the frame's copy to the device as long as that over 65536.
-        if (npix >= (blurred ? (size_t)1 << 14 : (size_t)1 << 16) && q == q) {
-            int rc;
-            if (!blurred) {
-                if ((rc = grow(c, (void**)&c->d_post_lev, &c->post_lev_cap, sizeof(float4) * npix))) return rc;
+        // 16384 pixels, with the frame's copy to the device as long as that over 65536. Where the device has no
+        // room for the frame, on the host too.
+        if (npix >= (blurred ? (size_t)1 << 14 : (size_t)1 << 16) && q == q && room_for_stats(c, npix)) {
+            if (!blurred)
                 PCK(c, hipMemcpyAsync(c->d_post_lev, px, sizeof(float4) * npix, hipMemcpyHostToDevice, c->st));
-            }
-            if ((rc = grow(c, (void**)&c->d_post_tmp, &c->post_tmp_cap, sizeof(float) * npix)) ||
-                (rc = grow(c, (void**)&c->d_post_wt, &c->post_wt_cap, sizeof(LumState))))
-                return rc;
             float* lum = (float*)c->d_post_tmp;
             LumState* S = (LumState*)c->d_post_wt;
             const dim3 one(1), blk(POST_BLOCK), g((unsigned)std::min<size_t>((npix + POST_BLOCK - 1) / POST_BLOCK, 1024));

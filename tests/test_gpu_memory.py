@@ -1,5 +1,6 @@
-"""Calls on a device that is nearly full: the normalising flux keeps working where its faster path's buffer cannot
-be had, with that path's result, and gives a large buffer back."""
+"""Calls on a device that is nearly full: the normalising flux and the display statistics keep working where their
+faster paths' buffers cannot be had, with the results of those paths, and the flux gives a large buffer back."""
+import numpy as np
 import pytest
 import torch
 
@@ -42,5 +43,31 @@ def test_flux_without_room_for_its_samples():
             torch.cuda.empty_cache()
         assert got == want and small > 0.0   # the same blocks and order of additions
         assert t.radio_flux(r["F"], n, 1e-20) == want
+    finally:
+        t.close()
+
+
+def test_statistics_without_room_for_the_frame():
+    r = setup(shot("c2_radio_1024.ini"), W=64, H=64)
+    t = tracer_for(r)
+    W, H = 8192, 6144   # 768 MiB
+    rng = np.random.default_rng(1)
+    img = np.zeros((H, W, 4), dtype=np.float32)
+    img[..., 0] = rng.random((H, W), dtype=np.float32) ** 8
+    img[:, ::5, 0] = 0.0
+    try:
+        want = t.post_radio(img)[1:]
+    finally:
+        t.close()
+    t = tracer_for(r)   # holds none of the buffers
+    try:
+        hogs = fill(600 * MIB, img.nbytes)
+        try:
+            got = t.post_radio(img)[1:]
+        finally:
+            del hogs
+            torch.cuda.empty_cache()
+        assert got == want and want[1] == img[..., 0].max()
+        assert t.post_radio(img)[1:] == want
     finally:
         t.close()
