@@ -406,7 +406,8 @@ int bh_tonemap_hud(bh_ctx* ctx, const float* px, int W, int H, const bh_tone_par
 
 /* Diagnostic: evaluates one elementary function of the device math library on n inputs (no context
    needed; device 0). fn: 0 exp, 1 log, 2 expm1, 3 cbrt, 4 x^-0.2, 5 sin, 6 cos, 7 atan2(x, y),
-   8 acos, 9 sqrt, 10 x / y, 11 asin. Used by the tests that pin the device functions bit for bit. */
+   8 acos, 9 sqrt, 10 x / y, 11 asin; the tracer's own forms: 12 x / y (y > 0), 13 sqrt, 14 the step controller's
+   factor for an error x, 15 the angle atan2(x, y) of a vector of length 1 with x >= 0. Used by the tests that pin the device functions bit for bit. */
 int bh_math_eval(int fn, const double* x, const double* y, double* out, int n);
 
 /* Renderer::~Renderer                                           render.cu:526-529 */

@@ -388,7 +388,7 @@ def k2_from_scene(ini, sets=""):
 
 
 MATH_FN = {"exp": 0, "log": 1, "expm1": 2, "cbrt": 3, "pow_m02": 4, "sin": 5, "cos": 6, "atan2": 7, "acos": 8,
-           "sqrt": 9, "div": 10, "asin": 11}
+           "sqrt": 9, "div": 10, "asin": 11, "quot": 12, "root": 13, "step_factor": 14, "angle": 15}
 
 
 def math_eval(fn, x, y=None):

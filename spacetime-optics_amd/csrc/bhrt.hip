@@ -519,6 +519,10 @@ __global__ void k_math_eval(int fn, const double* __restrict__ x, const double* 
         case 8: r = bhm::acos(a); break;
         case 11: r = bhm::asin(a); break;
         case 9: r = sqrt(a); break;
+        case 12: r = bhm::quot_ieee_(a, b); break;
+        case 13: r = bhm::sqrt_nn_(a); break;
+        case 14: r = bhd::step_factor(a); break;
+        case 15: r = bhd::angle_pos(a, b); break;
         default: r = a / b; break;
     }
     out[i] = r;
@@ -2026,7 +2030,7 @@ int bh_vacuum_fates(bh_ctx* c, const double* photons, int n, double tol, double 
 }
 
 int bh_math_eval(int fn, const double* x, const double* y, double* out, int n) {
-    if (!x || !y || !out || n < 0 || fn < 0 || fn > 11) return BH_ERR_ARG;
+    if (!x || !y || !out || n < 0 || fn < 0 || fn > 15) return BH_ERR_ARG;
     if (n == 0) return BH_OK;
     if (bh_device_count() <= 0) return BH_ERR_NODEVICE;
     double *dx = nullptr, *dy = nullptr, *dout = nullptr;
