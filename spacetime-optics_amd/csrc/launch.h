@@ -59,16 +59,19 @@ inline bool pair_shape(const bh_batch_cfg& g) { return g.block == PAIR_RAYS && g
    - A SIMD issues one wave's instructions at half its rate, so 2 waves fill it and a third covers the
      stalls; but the longest rays set the end of a launch, and each of their instructions waits for the
      SIMD's other waves. Few rays are therefore spread thinly - and evenly: the waves that find no ray
-     exit, and with 3 resident waves per SIMD which SIMD they leave idle is chance. FP64 vacuum, one wave
-     per SIMD to w = 7 (16 M wide, 8 -> 4 waves per CU: 272^2 (w = 4.5) 2.4 -> 1.9, 336^2 (6.9) 2.6 -> 2.4; 360^2
-     (7.9) and 448^2 (12) within 5 % either way); 512^2 radio, FP64: 8.7 with 12, 6.0 with 8; 1024^2: 18.3 with 12.
-     Mixed radio: 1400^2 4.82 with 8, 4.17 with 12; zoom 768^2: 13.5 with 8, 11.9 with 12 (every ray is
-     long: throughput, from 8 waves of rays per CU on).
+     exit, and with 3 resident waves per SIMD which SIMD they leave idle is chance. FP64 vacuum, at most one
+     wave per SIMD to w = 7 (16 M wide, 8 -> 4 waves per CU: 272^2 (w = 4.5) 2.4 -> 1.9, 336^2 (6.9) 2.6 -> 2.4;
+     360^2 (7.9) and 448^2 (12) within 5 % either way); 512^2 radio, FP64: 8.7 with 12, 6.0 with 8; 1024^2: 18.3
+     with 12. Mixed radio: 1400^2 4.82 with 8, 4.17 with 12; zoom 768^2: 13.5 with 8, 11.9 with 12 (every ray
+     is long: throughput, from 8 waves of rays per CU on).
    - Longest rays first (critical order) where several generations of rays share the launch, but not so
-     many that its tail no longer counts: FP64 vacuum 288^2 (w = 5) 2.7 -> 2.1, radio 280^2 (4.8, two waves per 64
-     rays) 4.7 -> 4.3, 384^2 6.0 -> 4.8, 768^2 11.3 -> 11.1, 1024^2 18.3 -> 18.9, 1500^2 37.6 -> 39.9. A launch that
-     holds all its rays at once (4 waves per CU to w = 4) needs no sort. The mixed tracer's rays differ by over
-     10x in length: always.
+     many that its tail no longer counts: FP64 vacuum 280^2 (w = 4.8, 3 waves per CU in rows -> 4, sorted) 2.8 ->
+     2.1 at 16 M wide, 2.7 -> 2.0 at 30 M, 2.1 -> 1.8 at 40 M; radio 280^2 (two waves per 64 rays) 4.7 -> 4.3, 384^2
+     6.0 -> 4.8, 768^2 11.3 -> 11.1, 1024^2 18.3 -> 18.9, 1500^2 37.6 -> 39.9. Up to w = 4 at most a quarter of the
+     rays waits for a place, short ones finish soon enough for them in most fields, and rows with 3 waves per CU
+     are ahead: 256^2 records 40 M wide, 3 rows / 3 sorted / 4 rows / 4 sorted: 3.20 / 3.28 / 3.40 / 3.41, 240^2 2.53 /
+     2.39 / 2.49 / 2.49, 224 x 288 2.69 / 2.73 / 2.79 / 2.88 (16 M wide, where most rays are long, 256^2 2.6 / 2.0 /
+     2.0 / 2.0). The mixed tracer's rays differ by over 10x in length: always.
    - Workgroups of one wave where they are few, so that the dispatcher can place each on its own. */
 inline bh_batch_cfg defaults(const Load& l) {
     bh_batch_cfg d{};
@@ -87,7 +90,7 @@ inline bh_batch_cfg defaults(const Load& l) {
         d.grid_per_cu = l.radio == 0 ? (l.w <= 8.0 ? 1 : 3) : (l.w <= 48.0 ? 2 : 3);
     } else {
         d.block = l.w <= 20.0 ? 64 : 256;
-        d.grid_per_cu = l.w <= 3.0 ? 3 : (l.w <= 7.0 ? 4 : (l.w <= 20.0 ? 8 : 3));
+        d.grid_per_cu = l.w <= 4.0 ? 3 : (l.w <= 7.0 ? 4 : (l.w <= 20.0 ? 8 : 3));
     }
     return d;
 }

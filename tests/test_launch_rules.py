@@ -86,8 +86,8 @@ def test_tuned_holds_for_launches_like_it(rules, p):
     assert rules(f"tuned {large} {vacuum} 128 8 32")[0] == 256
 
 
-@pytest.mark.parametrize("w,per_cu,order", [(2.9, 3, 1), (3.1, 4, 1), (4.0, 4, 1), (4.1, 4, 3), (5.0, 4, 3)])
-def test_fp64_holds_its_rays_or_sorts_them(rules, w, per_cu, order):
-    """As many waves as there are of rays, up to one per SIMD; beyond, the longest rays first."""
+@pytest.mark.parametrize("w,per_cu,order", [(2.9, 3, 1), (4.0, 3, 1), (4.1, 4, 3), (5.0, 4, 3)])
+def test_fp64_sorts_what_it_does_not_hold(rules, w, per_cu, order):
+    """Beyond one wave of rays per SIMD the longest rays go first."""
     assert rules(f"defaults 0 0 {w} {w} 0") == [64, per_cu, order, 0]
     assert rules(f"defaults 0 1 {w} {w} 0") == [64, 4, order, 1]
