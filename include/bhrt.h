@@ -216,7 +216,8 @@ int bh_trace_tile(bh_ctx* ctx, const bh_frame* frame, int x0, int y0, int w, int
 int bh_radio_flux(bh_ctx* ctx, const bh_frame* frame, int n, double pix_sr, double* jy);
 
 /* vacuum_fate (kerr.hpp:184-203) for n photons; photons[9*i..] = (lam, eta, E, y[6]) as
-   camera_photon returns them. fates[i] in {+1, -1, 0}. Used by the critical-curve search
+   camera_photon returns them. fates[i] in {+1, -1, 0}. tol is not read: the steps are held to the
+   scene's tol. Used by the critical-curve search
    (shot.cpp:148-164) and the self-test. */
 int bh_vacuum_fates(bh_ctx* ctx, const double* photons, int n, double tol, double r_escape, int max_steps,
                     int* fates);

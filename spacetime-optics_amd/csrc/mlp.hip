@@ -261,7 +261,8 @@ struct alignas(16) GradTile {
 };
 
 // Row index of a partial gradient: everything but W2 and W3 lies as in the parameters; each of W2 and W3
-// as a lane holds it (wave, jb, lane, e), so that the partials are stored and added 16 bytes at a time.
+// as a lane holds it (wave, jb, lane, e), so that the partials are stored 16 bytes at a time (the reduction
+// reads whole rows, 4 bytes a lane).
 __device__ __forceinline__ int partial_param(int q) {
     const int off = q >= OFF_W3 && q < OFF_B3 ? OFF_W3 : OFF_W2;
     if (q < OFF_W2 || q >= OFF_B3 || (q >= OFF_B2 && q < OFF_W3)) return q;
