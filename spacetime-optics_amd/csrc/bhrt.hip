@@ -816,9 +816,9 @@ double near_radius(const bh_scene& S) {
     return std::max(3.0 * S.rh, r_ph) + 1.0;
 }
 
-// Whether the mid-plane optical depth from the flow's edge down to near_radius exceeds 1, from 64 cells in ln r
+// Whether the mid-plane optical depth from the flow's edge down to near_radius exceeds 1, from 16 cells in ln r
 bool flow_opaque(const bh_ctx* c, const bh_scene& S) {
-    constexpr int N = 64;
+    constexpr int N = 16;
     const double r0 = near_radius(S), r1 = S.r_flow_max;
     if (!S.flow_on || !(r1 > r0) || c->k2_host.size() < 2) return false;
     const double dl = std::log(r1 / r0) / N;

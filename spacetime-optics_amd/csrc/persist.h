@@ -163,11 +163,6 @@ struct ChunkWork {
     }
 };
 
-// A ray's counters after one of its attempts
-struct Marks {
-    int it, accepted, flow_steps, ncross, fp64;
-};
-
 template <int PREC, int RADIO, bool TIME>
 struct Tracer;
 
@@ -182,19 +177,15 @@ struct Tracer<BH_PREC_FP64, RADIO, TIME> {
                                                 const bhm32::MixedParams&, State& R) {
         bhd::ray_step<RADIO, TIME>(P, F, R);
     }
+    template <bool SETTLE>
     static __device__ __forceinline__ bool move(const TraceParams& P, const bhm32::MixedParams&, State& R,
                                                 bhd::StepSample& q) {
-        return bhd::ray_move<RADIO, TIME>(P, R, q);
+        return bhd::ray_move<RADIO, TIME, SETTLE>(P, R, q);
     }
-    static __device__ __forceinline__ Marks marks(const State& R) {
-        return Marks{R.it, R.accepted, R.flow_steps, R.ncross, 0};
-    }
-    static __device__ __forceinline__ void set_marks(State& R, const Marks& m) {
-        R.it = m.it;
-        R.accepted = m.accepted;
-        R.flow_steps = m.flow_steps;
-        R.ncross = m.ncross;
-    }
+    // whether the ray's last attempt counted as an FP64 one, and taking some back (here every attempt does, and
+    // they are not counted apart)
+    static __device__ __forceinline__ bool last_fp64(const State&) { return false; }
+    static __device__ __forceinline__ void undo_fp64(State&, int) {}
     // what a ray's samples add up to, in the wave that evaluates them
     struct Sums {
         double acc0, acc1, acc2, acc3, trans, psi;
@@ -230,20 +221,13 @@ struct Tracer<BH_PREC_MIXED, RADIO, TIME> {
                                                 const bhm32::MixedParams& FM, State& R) {
         bhm32::ray_step_m<RADIO, TIME>(P, M, F, FM, R);
     }
+    template <bool SETTLE>
     static __device__ __forceinline__ bool move(const TraceParams& P, const bhm32::MixedParams& M, State& R,
                                                 bhd::StepSample& q) {
-        return bhm32::ray_move_m<RADIO, TIME>(P, M, R, q);
+        return bhm32::ray_move_m<RADIO, TIME, SETTLE>(P, M, R, q);
     }
-    static __device__ __forceinline__ Marks marks(const State& R) {
-        return Marks{R.it, R.accepted, R.flow_steps, R.ncross, R.fp64_attempts};
-    }
-    static __device__ __forceinline__ void set_marks(State& R, const Marks& m) {
-        R.it = m.it;
-        R.accepted = m.accepted;
-        R.flow_steps = m.flow_steps;
-        R.ncross = m.ncross;
-        R.fp64_attempts = m.fp64;
-    }
+    static __device__ __forceinline__ bool last_fp64(const State& R) { return !R.k1_f32; }
+    static __device__ __forceinline__ void undo_fp64(State& R, int n) { R.fp64_attempts -= n; }
     struct Sums {
         double acc0, acc1, acc2, acc3, trans;
         float psi;
@@ -419,20 +403,24 @@ __device__ __forceinline__ void persist_body(const Work& Wk, unsigned int* __res
    the next attempt: one barrier per attempt, two slots by turns. Every value is formed by the same operations
    in the same order as in ray_step: same outputs. One wave -> two, ms of the launch (frames 30 M wide at 17
    degrees, the 0.6 Jy flow): mixed 64^2 1.32 -> 0.98, 256^2 2.04 -> 1.69; FP64 64^2 3.9 -> 2.9, 256^2 5.6 -> 4.4.
-   A ray that turned out opaque in attempt k is known to be so after the barrier of attempt k + 1, which it
-   has made too: it is taken back to what it was before the step of attempt k (its counters from registers;
-   its state, which only ray records hold, from attempt k's slot) and takes no further attempts. So an
-   opaque ray costs one attempt more than it has; learning of it only at the interval's end, and then repeating
-   the interval's attempts up to k, cost an optically thick flow (3000 times the density, 69 degrees) its gain
-   and more: mixed 256^2 0.73 ms, 448^2 1.25, 640^2 1.88; now 0.52, 0.84, 1.26; one wave 0.63, 0.81, 1.20.
+   A ray that turned out opaque in attempt k is known to be so after the barrier of attempt k + 1. Its flag is
+   read then, and used after attempt k + 2 so that nothing waits for the read; the ray takes no further attempts,
+   and at the interval's end its counters are taken back by the tags of the attempts since. So it costs two
+   attempts more than it has. Ray records hold its state before attempt k too: they save the rays' state at the
+   interval's start, from which its attempts up to k are repeated (keeping every attempt's state for that cost all
+   records 2 %). Learning of the flag at the interval's end only, with every opaque ray's attempts repeated, cost a
+   thick flow (3000 times the density, 69 degrees) the gain and more: mixed 256^2 0.73 ms, 448^2 1.25, 640^2 1.88;
+   now 0.51, 0.84, 1.26; one wave 0.63, 0.81, 1.20.
    Both waves take every branch around a barrier on a value that both read from LDS. */
 constexpr int PAIR_BLOCK = 128;
 
-template <bool RECORDS>
+// What an attempt of a lane left (PairLDS::tag)
+constexpr int TAG_SAMPLE = 1, TAG_FLOW = 2, TAG_TRIED = 4, TAG_FP64 = 8;   // an accepted step; inside the flow; an attempt
+
+template <class T, bool RECORDS>
 struct PairLDS {
     double v[2][7][64];        // StepSample
-    double y[RECORDS ? 2 : 1][RECORDS ? 4 : 1][64];   // r, r', u', t before the step
-    int tag[2][64];            // 0: no sample; 1: a step outside the flow; 3: inside
+    int tag[2][64];
     int opaque[2][64];         // the attempt's sample made the ray opaque
     int more[2];               // some ray runs on after this attempt
     int frame;                 // the rays' frame; -1: no rays are left
@@ -441,23 +429,22 @@ struct PairLDS {
     double sums[6][64];        // acc0..3, trans, psi
     double flux[64];
     unsigned long long stat[NSTAT][64];
+    typename T::State start[RECORDS ? 64 : 1];   // ray records: at the interval's start
 };
 
-// Takes the lane's ray back to attempt m, in slot b, which made it opaque.
-template <class T, bool RECORDS>
-__device__ __forceinline__ void take_back(const PairLDS<RECORDS>& L, int b, int lane, const Marks& m,
-                                          typename T::State& R) {
-    T::set_marks(R, m);
-    if constexpr (RECORDS) {
-        R.s.y0 = L.y[b][0][lane];
-        R.s.y1 = L.y[b][1][lane];
-        R.s.y2 = L.v[b][5][lane];
-        R.s.y3 = L.y[b][2][lane];
-        R.s.y4 = L.v[b][6][lane];
-        R.s.y5 = L.y[b][3][lane];
-    }
-    R.fate = -1;
-    R.done = true;
+// What the ray's statistics hold of an attempt, three bits each (it, fp64_attempts, accepted, flow_steps)
+__device__ __forceinline__ int counts_of(int tag) {
+    return (tag & TAG_TRIED ? 1 : 0) | (tag & TAG_FP64 ? 1 << 3 : 0) | (tag & TAG_SAMPLE ? 1 << 6 : 0) |
+           (tag & TAG_FLOW ? 1 << 9 : 0);
+}
+constexpr int ENDED = 1 << 12;   // beside the counts to take back: a sample made the ray opaque
+
+template <class T>
+__device__ __forceinline__ void take_back(int back, typename T::State& R) {
+    R.it -= back & 7;
+    T::undo_fp64(R, back >> 3 & 7);
+    R.accepted -= back >> 6 & 7;
+    R.flow_steps -= back >> 9 & 7;
 }
 
 template <int PREC, int RADIO, bool TIME, class Work>
@@ -467,7 +454,7 @@ __device__ __forceinline__ void pair_body(const Work& Wk, unsigned int* __restri
     using CFrame = const __attribute__((address_space(4))) BatchFrame;
     CFrame* cfr = (CFrame*)Wk.frames;
     constexpr bool RECORDS = Work::RECORDS;
-    __shared__ PairLDS<RECORDS> L;
+    __shared__ PairLDS<T, RECORDS> L;
     const int lane = threadIdx.x & 63;
     const bool mover = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) == 0;
     *flux_out = 0.0;
@@ -488,21 +475,31 @@ __device__ __forceinline__ void pair_body(const Work& Wk, unsigned int* __restri
             if (active) {
                 L.lam[lane] = R.c.lam;
                 L.E[lane] = R.c.E;
+                if constexpr (RECORDS) L.start[lane] = R;
             }
             if (lane == 0) L.frame = !any && cur >= Wk.n ? -1 : cf;
             __syncthreads();   // A: the interval's rays
             if (!any && cur >= Wk.n) break;
             const TraceParams P = *(const TraceParams*)&cfr[cf].P;
             const bhm32::MixedParams M = *(const bhm32::MixedParams*)&cfr[cf].M;
-            Marks m = T::marks(R);   // after the attempt before this one
-            int k = 0;
+            // of a ray that a sample made opaque: its counts to take back (ray records: that sample's attempt + 1)
+            int k = 0, back = 0;
             for (;; ++k) {
                 const int b = k & 1;
-                if (k >= 2 && L.opaque[b][lane]) take_back<T>(L, b, lane, m, R);   // by attempt k - 2
-                m = T::marks(R);
-                [[maybe_unused]] const double r0 = R.s.y0, dr0 = R.s.y1, du0 = R.s.y3, t0 = R.s.y5;
+                const int opaque = L.opaque[b][lane];   // by attempt k - 2; an older interval's before that
+                const bool run = active && !R.done;
                 bhd::StepSample q;
-                const bool push = active && !R.done && T::move(P, M, R, q);
+                bool push = run && T::template move<true>(P, M, R, q);
+                int tag = (run ? TAG_TRIED | (T::last_fp64(R) ? TAG_FP64 : 0) : 0) |
+                          (push ? TAG_SAMPLE | (q.flow ? TAG_FLOW : 0) : 0);
+                if (opaque && k >= 2) {
+                    if constexpr (RECORDS) back = k - 1;
+                    else
+                        back = ENDED + counts_of(tag) + counts_of(L.tag[b ^ 1][lane]);
+                    R.done = true;
+                    push = false;
+                    tag = 0;
+                }
                 if (push) {
                     L.v[b][0][lane] = q.r;
                     L.v[b][1][lane] = q.u;
@@ -511,23 +508,33 @@ __device__ __forceinline__ void pair_body(const Work& Wk, unsigned int* __restri
                     L.v[b][4][lane] = q.h;
                     L.v[b][5][lane] = q.u0;
                     L.v[b][6][lane] = q.phi0;
-                    if constexpr (RECORDS) {
-                        L.y[b][0][lane] = r0;
-                        L.y[b][1][lane] = dr0;
-                        L.y[b][2][lane] = du0;
-                        L.y[b][3][lane] = t0;
-                    }
                 }
-                L.tag[b][lane] = push ? (q.flow ? 3 : 1) : 0;
+                L.tag[b][lane] = tag;
                 const bool more = k + 1 < interval && __ballot(active && !R.done) != 0ull;
                 if (lane == 0) L.more[b] = more;
                 __syncthreads();   // B: attempt k's samples
                 if (!more) break;
             }
             __syncthreads();   // C: the interval's sums
-            // the last two attempts' samples
-            if (k > 0 && L.opaque[(k - 1) & 1][lane]) take_back<T>(L, (k - 1) & 1, lane, m, R);
-            else if (L.opaque[k & 1][lane]) take_back<T>(L, k & 1, lane, T::marks(R), R);
+            {   // the last two attempts' samples
+                const int b = k & 1;
+                if (k > 0 && L.opaque[b ^ 1][lane])
+                    back = RECORDS ? k : ENDED + counts_of(L.tag[b][lane]);
+                else if (L.opaque[b][lane])
+                    back = RECORDS ? k + 1 : ENDED;
+            }
+            if (back) {
+                if constexpr (RECORDS) {
+                    bhd::StepSample q;
+                    R = L.start[lane];
+                    for (int i = 1; i < back; ++i) T::template move<true>(P, M, R, q);
+                    T::template move<false>(P, M, R, q);
+                } else {
+                    take_back<T>(back, R);
+                }
+                R.fate = -1;
+                R.done = true;
+            }
             if (active && R.done) {
                 R.acc0 = L.sums[0][lane];
                 R.acc1 = L.sums[1][lane];
@@ -570,9 +577,9 @@ __device__ __forceinline__ void pair_body(const Work& Wk, unsigned int* __restri
                 const int b = k & 1, tag = L.tag[b][lane];
                 const bool more = __builtin_amdgcn_readfirstlane(L.more[b]) != 0;
                 bool now = false;
-                if (tag && !opaque) {
+                if ((tag & TAG_SAMPLE) && !opaque) {
                     const bhd::StepSample q{L.v[b][0][lane], L.v[b][1][lane], L.v[b][2][lane], L.v[b][3][lane],
-                                            L.v[b][4][lane], L.v[b][5][lane], L.v[b][6][lane], tag == 3};
+                                            L.v[b][4][lane], L.v[b][5][lane], L.v[b][6][lane], (tag & TAG_FLOW) != 0};
                     now = T::add(F, FM, lam, E, q, S);
                 }
                 L.opaque[b][lane] = now;

@@ -628,9 +628,10 @@ struct StepSample {
     bool flow;
 };
 
-// The attempt of ray_step without the ring angle and the flow: true when a step was accepted. R.ppx and R.ppy
-// are not kept up.
-template <int RADIO, bool TIME>
+// The attempt of ray_step without the ring angle and the flow: true when a step was accepted. SETTLE false
+// leaves the ray where it was, as ray_step does when the step's sample makes it opaque. R.ppx and R.ppy are
+// not kept up.
+template <int RADIO, bool TIME, bool SETTLE>
 __device__ __forceinline__ bool ray_move(const TraceParams& P, RayState& R, StepSample& q) {
     State n;
     if (!ray_attempt<RADIO, TIME>(P, R, n, q.h)) return false;
@@ -644,7 +645,7 @@ __device__ __forceinline__ bool ray_move(const TraceParams& P, RayState& R, Step
     q.phi0 = R.s.y4;
     q.flow = P.flow_on && n.y0 < P.r_flow_max;
     if (q.flow) ++R.flow_steps;
-    ray_settle(P, R, n);
+    if (SETTLE) ray_settle(P, R, n);
     return true;
 }
 

@@ -897,7 +897,7 @@ __device__ __forceinline__ void ray_step_m(const TraceParams& P, const MixedPara
 
 // bhd::ray_move and bhd::sample_eval under the mixed policy (the direction before the step is the sample's
 // own). emits: false for a sample that emits and absorbs nothing.
-template <int RADIO, bool TIME>
+template <int RADIO, bool TIME, bool SETTLE>
 __device__ __forceinline__ bool ray_move_m(const TraceParams& P, const MixedParams& M, RayStateM& R,
                                            bhd::StepSample& q) {
     State n;
@@ -913,7 +913,7 @@ __device__ __forceinline__ bool ray_move_m(const TraceParams& P, const MixedPara
     q.phi0 = R.s.y4;
     q.flow = P.flow_on && n.y0 < M.r_cut;
     if (q.flow) ++R.flow_steps;
-    ray_settle_m(P, M, R, n, q.h, fac);
+    if (SETTLE) ray_settle_m(P, M, R, n, q.h, fac);
     return true;
 }
 
