@@ -7,8 +7,9 @@
    filled slot to the caller's pages while the next is on its way. Copies below MIN_BYTES, and into memory
    that is already pinned, go straight to the runtime; so do copies to the device, which it moves at 30
    GB/s (the same threads measured no faster).
-   The threads are woken when the first slot is filled: whatever the stream has to do before the copy, they
-   sleep. From then on the slots fill at the link's rate and they wait by yielding. There are at most as many as
+   The threads are woken when the stream reaches the copy: whatever it has to do before, they sleep. They
+   are awake when the first slot is filled, and from then on the slots fill at the link's rate and they wait by
+   yielding. There are at most as many as
    the process has cores (affinity, and the control group's quota); with one or two the runtime's path is taken.
    One Transfer per device serves all of its contexts (16 MiB of pinned memory take milliseconds to get)
    and ends with the last of them; it runs one copy at a time, and a copy that finds it busy takes the
@@ -61,6 +62,7 @@ class Transfer {
             if (s.filled) (void)hipEventDestroy(s.filled);
             if (s.mem) (void)hipHostFree(s.mem);
         }
+        if (reached_) (void)hipEventDestroy(reached_);
     }
 
     // device -> host after the work on the stream, complete on return
@@ -84,13 +86,14 @@ class Transfer {
                 err = hipMemcpyAsync(s.mem, (const char*)src + i * piece, length(i), hipMemcpyDeviceToHost, st);
             if (err == hipSuccess) err = hipEventRecord(s.filled, st);
         };
+        err = hipEventRecord(reached_, st);
         for (size_t i = 0; i < std::min<size_t>(pieces_, SLOTS); ++i) fill(i);
-        if (err == hipSuccess) err = hipEventSynchronize(slots_[0].filled);
+        if (err == hipSuccess) err = hipEventSynchronize(reached_);
         if (err != hipSuccess) {   // the threads have not been woken
             (void)hipStreamSynchronize(st);
             return err;
         }
-        filled_.store(1, std::memory_order_relaxed);
+        filled_.store(0, std::memory_order_relaxed);
         {
             std::lock_guard<std::mutex> lock(mu_);
             left_ = count_ - 1;
@@ -98,11 +101,9 @@ class Transfer {
         }
         wake_.notify_all();
         for (size_t i = 0; i < pieces_; ++i) {
-            if (i > 0) {
-                if (err == hipSuccess) err = hipEventSynchronize(slots_[i % SLOTS].filled);
-                if (err != hipSuccess) failed_.store(true, std::memory_order_relaxed);   // then nothing more is moved
-                filled_.store(i + 1, std::memory_order_release);
-            }
+            if (err == hipSuccess) err = hipEventSynchronize(slots_[i % SLOTS].filled);
+            if (err != hipSuccess) failed_.store(true, std::memory_order_relaxed);   // then nothing more is moved
+            filled_.store(i + 1, std::memory_order_release);
             move_share(0, i);
             if (i + SLOTS < pieces_) {   // the slot is free again when every thread has taken its share
                 while (slots_[i % SLOTS].moved.load(std::memory_order_acquire) < count_) std::this_thread::yield();
@@ -165,6 +166,10 @@ class Transfer {
         state_ = -1;
         count_ = std::min(THREADS, cores());
         if (count_ <= 2) return false;
+        if (hipEventCreateWithFlags(&reached_, hipEventDisableTiming) != hipSuccess) {
+            (void)hipGetLastError();
+            return false;
+        }
         for (Slot& s : slots_)
             if (hipHostMalloc((void**)&s.mem, SLOT, hipHostMallocDefault) != hipSuccess ||
                 hipEventCreateWithFlags(&s.filled, hipEventDisableTiming) != hipSuccess) {
@@ -202,6 +207,7 @@ class Transfer {
     std::mutex busy_;   // one copy at a time
     int count_ = 0;     // threads, the caller among them
     int state_ = 0;     // 0: not tried, 1: slots and threads are there, -1: the plain path
+    hipEvent_t reached_ = nullptr;   // the stream's work before the copy
     Slot slots_[SLOTS];
     std::vector<std::thread> threads_;
     std::mutex mu_;
